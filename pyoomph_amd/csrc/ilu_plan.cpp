@@ -12,6 +12,7 @@
 #include "ilu_plan.h"
 
 #include <algorithm>
+#include <climits>
 #include <utility>
 
 namespace pyhip {
@@ -141,6 +142,154 @@ int ilu_plan_host(int64_t n, const int32_t *rs, const int32_t *col, const std::v
     out.pdiag = std::move(pdiag);
     out.multicolor = mc_any;
     return 0;
+}
+
+// One side (lower or upper) of the sliced plan for the handled sub-problems: level lists
+// from the merged level lists `rows` / `ptr` of the whole batch.
+static int sliced_side(const IluHostPlan &H, const std::vector<int32_t> &rows, const std::vector<int64_t> &ptr,
+                       bool lower, const std::vector<int32_t> &slot_of, const IluSlicedPlan &P, const std::vector<int32_t> &row_sub, IluSlicedSide &S,
+                       std::vector<int32_t> &big, std::vector<int64_t> &big_ptr, std::string &err) {
+    const int nh = (int)P.subs.size(), nl = (int)ptr.size() - 1;
+    // per handled sub-problem: (level, rows) lists in level order
+    std::vector<std::vector<std::pair<int32_t, std::vector<int32_t>>>> lists(nh);
+    big_ptr.assign(1, 0);
+    for (int l = 0; l < nl; l++) {
+        for (int64_t w = ptr[l]; w < ptr[l + 1]; w++) {
+            const int32_t r = rows[w], t = slot_of[row_sub[r]];
+            if (t < 0) {
+                big.push_back(r);
+                continue;
+            }
+            if (lists[t].empty() || lists[t].back().first != l) lists[t].push_back({l, {}});
+            lists[t].back().second.push_back(r);
+        }
+        if ((int64_t)big.size() > big_ptr.back()) big_ptr.push_back((int64_t)big.size());
+    }
+    auto len = [&](int32_t r) { return lower ? H.pdiag[r] - H.prs[r] : H.prs[r + 1] - H.pdiag[r] - 1; };
+    S.chunk0.assign(1, 0);
+    struct Slice {
+        int level, lanes;
+        size_t b, n;
+        const std::vector<int32_t> *rows;
+    };
+    for (int t = 0; t < nh; t++) {
+        const int32_t r0 = P.row0[t], dummy = P.rows[t];
+        std::vector<std::vector<Slice>> waves(kIluSliceWaves);
+        for (size_t l = 0; l < lists[t].size(); l++) {
+            auto &R = lists[t][l].second;
+            std::stable_sort(R.begin(), R.end(), [&](int32_t a, int32_t b) { return len(a) > len(b); });
+            // lanes that still leave the level at most one slice per wave
+            int fill = 1;
+            while (fill < 16 && 2 * fill * (int64_t)R.size() <= kIluSliceLanes * kIluSliceWaves && fill < len(R[0]))
+                fill *= 2;
+            int k = 0;
+            for (size_t b = 0; b < R.size(); k++) {
+                int lanes = fill;
+                while (lanes < 16 && (len(R[b]) + lanes - 1) / lanes > kIluChunk) lanes *= 2;
+                const size_t m = std::min<size_t>(kIluSliceLanes / lanes, R.size() - b);
+                waves[k % kIluSliceWaves].push_back({(int)l, lanes, b, m, &R});
+                b += m;
+            }
+        }
+        S.nlev.push_back((int32_t)lists[t].size());
+        for (const auto &tasks : waves) {
+            const size_t first = S.chunk0.back();
+            uint16_t mark = 0;
+            // appends an empty chunk
+            auto chunk = [&]() -> size_t {
+                const size_t c = S.idx.size() / kIluChunkIdx;
+                S.idx.resize((c + 1) * kIluChunkIdx, (uint16_t)dummy);
+                S.src.resize((c + 1) * kIluChunkVal, -1);
+                for (int lane = 0; lane < kIluSliceLanes; lane++) {
+                    S.idx[c * kIluChunkIdx + lane * 8 + kIluChunk] = kIluNoRow;
+                    S.idx[c * kIluChunkIdx + lane * 8 + kIluChunk + 1] = mark;
+                }
+                return c;
+            };
+            for (const Slice &sl : tasks) {
+                const std::vector<int32_t> &R = *sl.rows;
+                const int lanes = sl.lanes, w = (len(R[sl.b]) + lanes - 1) / lanes;
+                const int nch = std::max(1, (w + kIluChunk - 1) / kIluChunk);
+                const uint16_t base = (uint16_t)(sl.level | __builtin_ctz(lanes) << 12);
+                size_t c0 = 0;
+                for (int c = 0; c < nch; c++) {
+                    mark = (uint16_t)(base | (c + 1 < nch ? 1 << 15 : 0));
+                    const size_t at = chunk();
+                    if (c == 0) c0 = at;
+                    for (int lane = 0; lane < kIluSliceLanes; lane++)
+                        if ((size_t)(lane / lanes) < sl.n)
+                            S.idx[at * kIluChunkIdx + lane * 8 + kIluChunk] =
+                                (uint16_t)(R[sl.b + lane / lanes] - r0);
+                }
+                for (size_t q = 0; q < sl.n; q++) {
+                    const int32_t r = R[sl.b + q], k0 = lower ? H.prs[r] : H.pdiag[r] + 1;
+                    for (int e = 0; e < len(r); e++) {
+                        const int step = e / lanes, j = step % kIluChunk;
+                        const size_t lane = q * lanes + e % lanes, c = c0 + step / kIluChunk;
+                        S.idx[c * kIluChunkIdx + lane * 8 + j] = (uint16_t)(H.pcol[k0 + e] - r0);
+                        S.src[c * kIluChunkVal + (j / 2) * 2 * kIluSliceLanes + 2 * lane + j % 2] = k0 + e;
+                    }
+                }
+            }
+            mark &= 0xfff;   // padding stays on the wave's last level
+            while ((S.idx.size() / kIluChunkIdx - first) % kIluDepth) chunk();
+            if (S.src.size() >= (size_t)INT32_MAX) {
+                err = "ILU(0) sliced plan: too many entries";
+                return -1;
+            }
+            S.chunk0.push_back((int32_t)(S.idx.size() / kIluChunkIdx));
+        }
+    }
+    return 0;
+}
+
+int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, int cap, IluSlicedPlan &out,
+                    std::string &err) {
+    out = IluSlicedPlan();
+    const int nsub = (int)sub_off.size() - 1;
+    const int64_t n = (int64_t)H.perm.size();
+    if (cap >= (int)kIluNoRow) {
+        err = "ILU(0) sliced plan: more rows than 16-bit indices";
+        return -1;
+    }
+    // levels of each sub-problem on each side: the merged lists' levels that hold its rows
+    std::vector<int32_t> row_sub(n), levels[2];
+    for (int s = 0; s < nsub; s++)
+        for (int64_t r = sub_off[s]; r < sub_off[s + 1]; r++) row_sub[r] = s;
+    for (int u = 0; u < 2; u++) {
+        const auto &rows = u ? H.up_rows : H.lo_rows;
+        const auto &ptr = u ? H.up_ptr : H.lo_ptr;
+        levels[u].assign(nsub, 0);
+        for (size_t l = 0; l + 1 < ptr.size(); l++)
+            for (int64_t w = ptr[l]; w < ptr[l + 1]; w++) levels[u][row_sub[rows[w]]] = (int32_t)l + 1;
+    }
+    std::vector<int32_t> order;
+    for (int s = 0; s < nsub; s++) {
+        const int64_t m = sub_off[s + 1] - sub_off[s];
+        const int64_t entries = (int64_t)H.prs[sub_off[s + 1]] - H.prs[sub_off[s]] - m;
+        if (m > 0 && m <= cap && levels[0][s] <= kIluMaxLevels && levels[1][s] <= kIluMaxLevels &&
+            entries <= kIluEntriesPerLevel * (levels[0][s] + levels[1][s]))
+            order.push_back(s);
+    }
+    // longest first: the last workgroups to start are the shortest
+    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+        return sub_off[a + 1] - sub_off[a] > sub_off[b + 1] - sub_off[b];
+    });
+    std::vector<int32_t> slot_of(nsub, -1);
+    for (size_t t = 0; t < order.size(); t++) {
+        const int s = order[t];
+        slot_of[s] = (int32_t)t;
+        out.subs.push_back(s);
+        out.row0.push_back((int32_t)sub_off[s]);
+        out.rows.push_back((int32_t)(sub_off[s + 1] - sub_off[s]));
+        out.max_rows = std::max(out.max_rows, out.rows.back());
+    }
+    int rc = sliced_side(H, H.lo_rows, H.lo_ptr, true, slot_of, out, row_sub, out.lo, out.big_lo,
+                         out.big_lo_ptr, err);
+    if (!rc)
+        rc = sliced_side(H, H.up_rows, H.up_ptr, false, slot_of, out, row_sub, out.up, out.big_up,
+                         out.big_up_ptr, err);
+    return rc;
 }
 
 }  // namespace pyhip

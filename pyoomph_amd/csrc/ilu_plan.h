@@ -23,4 +23,52 @@ struct IluHostPlan {
 int ilu_plan_host(int64_t n, const int32_t *rs, const int32_t *col, const std::vector<int64_t> &sub_off,
                   const std::vector<char> &is_p, int order, int auto_levels, IluHostPlan &out, std::string &err);
 
+// Sliced copy of the triangular factors for the sub-problems of at most `cap` rows, whose
+// solves run in one workgroup of kIluSliceWaves waves each (ilu_sliced.h). Every level of a
+// sub-problem's lower and upper solve is cut into slices of 64 lanes, `lanes` lanes per row (a
+// power of two): rows sorted by decreasing length within the level, wide enough that a
+// narrow level spreads over all waves and a row takes at most kIluChunk steps where 16 lanes
+// allow it. Lane = row-in-slice * lanes + u takes the row's entries u, u + lanes, ...: one
+// step each. A slice is stored in chunks of kIluChunk steps (one, unless a row has more than
+// 16 * kIluChunk entries), every lane's part of a chunk contiguous for 16-byte loads:
+//   idx [chunk][lane][8]      local columns of the steps, the lane's local row (kIluNoRow:
+//                             none), the chunk's mark
+//   val [chunk][3][lane][2]   factor entries, two steps at a time
+// Mark: level | log2(lanes) << 12 | 1 << 15 where the slice goes on in the next chunk.
+// Slice k of a level belongs to wave k mod kIluSliceWaves; a wave's chunks follow each other
+// in level order, padded with empty ones to a multiple of kIluDepth, so that a wave reads one
+// stream. Columns and rows are local to the sub-problem (16 bits); steps past a row's end
+// point at the local row `rows` (one past the last), where the solve keeps a zero.
+constexpr int kIluSliceLanes = 64;
+constexpr int kIluSliceWaves = 16;
+constexpr int kIluChunk = 6;
+constexpr int kIluDepth = 3;                // chunks a wave loads ahead
+constexpr int kIluChunkIdx = kIluSliceLanes * 8, kIluChunkVal = kIluSliceLanes * kIluChunk;
+constexpr uint16_t kIluNoRow = 0xffff;
+constexpr int kIluMaxLevels = 4096;
+struct IluSlicedSide {
+    std::vector<int32_t> nlev;               // [handled] levels of each sub-problem
+    std::vector<int32_t> chunk0;             // [handled * waves + 1] first chunk of each wave
+    std::vector<uint16_t> idx;               // [chunks * kIluChunkIdx]
+    std::vector<int32_t> src;                // [chunks * kIluChunkVal] index in the permuted pattern (-1: none)
+};
+struct IluSlicedPlan {
+    std::vector<int32_t> subs, row0, rows;   // handled sub-problems (longest first), first permuted row, row count
+    IluSlicedSide lo, up;
+    std::vector<int32_t> big_lo, big_up;     // rows of the other sub-problems by level (as lo_rows / up_rows)
+    std::vector<int64_t> big_lo_ptr, big_up_ptr;
+    int max_rows = 0;                        // largest handled sub-problem
+};
+
+// The sliced plan of H (ilu_plan_host); cap < 65535. A sub-problem is handled if it has at
+// most cap rows and kIluMaxLevels levels on each side, and at most kIluEntriesPerLevel
+// triangle entries per level (both sides): one CU takes about 0.28 us per 1000 entries
+// (P2 Poisson 41^2, 67 k entries in 7 + 7 levels: 22 us; 64^2, 166 k in 7 + 7: 47 us;
+// Taylor-Hood 26^2, 223 k in 23 + 23: 58 us), a launch per level about 3 us (42, 42 and
+// 150 us). Decided per sub-problem, so that its solve is the same alone and in any batch.
+// Returns 0 or -1 (err).
+constexpr int64_t kIluEntriesPerLevel = 10000;
+int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, int cap, IluSlicedPlan &out,
+                    std::string &err);
+
 }  // namespace pyhip

@@ -65,6 +65,36 @@ int pyhip_ilu_plan_copy(const void *h, int32_t *perm, int32_t *prs, int32_t *pco
     return 0;
 }
 
+// The sliced plan of a plan (ilu_sliced_host with `cap`), side 0 lower / 1 upper. sizes:
+// [0] handled sub-problems, [1] chunks, [2] rows of the other sub-problems, [3] their
+// levels. Null arrays are not written.
+int pyhip_ilu_sliced_copy(const void *h, int nsub, const int64_t *sub_off, int cap, int side, int64_t *sizes,
+                          int32_t *subs, int32_t *nlev, int32_t *chunk0, uint16_t *idx, int32_t *src, int32_t *big,
+                          int64_t *big_ptr) {
+    const IluHostPlan *P = (const IluHostPlan *)h;
+    if (!P || !sizes || !sub_off || nsub < 1) return -1;
+    IluSlicedPlan Q;
+    if (ilu_sliced_host(*P, std::vector<int64_t>(sub_off, sub_off + nsub + 1), cap, Q, g_ilu_err)) return -1;
+    const IluSlicedSide &S = side ? Q.up : Q.lo;
+    const auto &bg = side ? Q.big_up : Q.big_lo;
+    const auto &bp = side ? Q.big_up_ptr : Q.big_lo_ptr;
+    sizes[0] = (int64_t)Q.subs.size();
+    sizes[1] = (int64_t)S.idx.size() / kIluChunkIdx;
+    sizes[2] = (int64_t)bg.size();
+    sizes[3] = (int64_t)bp.size() - 1;
+    auto cp = [](auto *dst, const auto &v) {
+        if (dst && !v.empty()) std::memcpy(dst, v.data(), v.size() * sizeof(v[0]));
+    };
+    cp(subs, Q.subs);
+    cp(nlev, S.nlev);
+    cp(chunk0, S.chunk0);
+    cp(idx, S.idx);
+    cp(src, S.src);
+    cp(big, bg);
+    cp(big_ptr, bp);
+    return 0;
+}
+
 void pyhip_ilu_plan_free(void *h) { delete (IluHostPlan *)h; }
 
 }  // extern "C"

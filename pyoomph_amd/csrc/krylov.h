@@ -22,15 +22,29 @@ struct IluPlan {
     int32_t *col = nullptr;       // [nnz]
     int32_t *src = nullptr;       // [nnz] index of the entry in the problem's CSR values
     int32_t *diag = nullptr;      // [n]
-    int32_t *lo_rows = nullptr;   // rows grouped by lower-solve / factorisation level
-    int32_t *up_rows = nullptr;   // rows grouped by upper-solve level
-    std::vector<int64_t> lo_ptr, up_ptr;   // level boundaries (host)
+    int32_t *lo_rows = nullptr;   // rows grouped by factorisation level
+    std::vector<int64_t> lo_ptr;  // factorisation level boundaries (host)
     void *lu = nullptr;           // [nnz] factor values (T)
     int lu_prec = -1;
-    double *tmp64 = nullptr;      // [n] permuted work vectors
+    double *tmp64 = nullptr;      // [n] permuted work vectors (allocated with big rows)
     double *tmp64b = nullptr;
     float *tmp32 = nullptr;
     float *tmp32b = nullptr;
+    // sub-problems solved in one workgroup each (ilu_sliced.h); big_lo / big_up with
+    // the level boundaries lo_solve / up_solve hold the rows of the others
+    struct Side {
+        int32_t *nlev = nullptr, *chunk0 = nullptr, *src = nullptr;
+        uint16_t *idx = nullptr;
+        void *val = nullptr;      // [nval] (T)
+        int64_t nval = 0;
+    } slo, sup;
+    int nsliced = 0, max_rows = 0;
+    int32_t *ssubs = nullptr, *srow0 = nullptr, *srows = nullptr;   // [nsliced]
+    int32_t *sdsrc = nullptr;     // [chunks * 64] pivot of each lane's row in lu (upper side)
+    void *sdiag = nullptr;        // [chunks * 64] reciprocal pivots (T)
+    int64_t ndiag = 0;
+    int32_t *big_lo = nullptr, *big_up = nullptr;
+    std::vector<int64_t> lo_solve, up_solve;
 };
 
 // Block-triangular preconditioner of Taylor-Hood Jacobians [A G; D 0] (block_precond.hip):

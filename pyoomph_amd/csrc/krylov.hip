@@ -24,7 +24,7 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "ilu_plan.h"
+#include "ilu_sliced.h"
 #include "krylov.h"
 #include "spmv.h"
 
@@ -366,14 +366,21 @@ __global__ __launch_bounds__(256) void trsv_level_kernel(int64_t nrows, const in
     if (lane == 0) x[i] = LOWER ? b[i] - acc : (b[i] - acc) / lu[diag[i]];
 }
 
-template <typename TA, typename TB>
+// permuted[i] = original[perm[i]]
+template <typename T>
 __global__ __launch_bounds__(256) void permute_kernel(int64_t n, const int32_t *__restrict__ perm,
-                                                      const TA *__restrict__ a, TB *__restrict__ b,
-                                                      int forward) {
+                                                      const T *__restrict__ a, T *__restrict__ b) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    if (forward) b[i] = TB(a[perm[i]]);   // permuted[i] = original[perm[i]]
-    else b[perm[i]] = TB(a[i]);
+    if (i < n) b[i] = a[perm[i]];
+}
+
+// original[perm[i]] = permuted[i] for the listed permuted rows i
+template <typename T>
+__global__ __launch_bounds__(256) void unpermute_rows_kernel(int64_t n, const int32_t *__restrict__ rows,
+                                                             const int32_t *__restrict__ perm,
+                                                             const T *__restrict__ a, T *__restrict__ b) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k < n) b[perm[rows[k]]] = a[rows[k]];
 }
 
 // ---- arclength continuation vector operations (per sub-problem scalars, masked) ------
@@ -648,10 +655,13 @@ constexpr int kGmresCheck = 8;   // GMRES iterations between host reads of the a
 
 static void ilu_free(KrylovWork *W) {
     IluPlan &L = W->ilu;
-    void *ptrs[] = {L.perm, L.rs, L.col, L.src, L.diag, L.lo_rows, L.up_rows, L.lu,
-                    L.tmp64, L.tmp64b, L.tmp32, L.tmp32b};
-    for (void *q : ptrs)
-        if (q) (void)hipFree(q);
+    void *ptrs[] = {L.perm, L.rs, L.col, L.src, L.diag, L.lo_rows, L.lu, L.tmp64, L.tmp64b, L.tmp32, L.tmp32b,
+                    L.ssubs, L.srow0, L.srows, L.sdsrc, L.sdiag, L.big_lo, L.big_up};
+    for (void *q : ptrs) dfree(q);
+    for (IluPlan::Side *S : {&L.slo, &L.sup}) {
+        void *sp[] = {S->nlev, S->chunk0, S->src, S->idx, S->val};
+        for (void *q : sp) dfree(q);
+    }
     L = IluPlan();
 }
 
@@ -696,27 +706,67 @@ static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
         set_error(err);
         return PYHIP_ERR_BREAKDOWN;
     }
-    const auto &perm = H.perm, &prs = H.prs, &pcol = H.pcol, &psrc = H.psrc, &pdiag = H.pdiag;
-    const auto &lo_rows = H.lo_rows, &up_rows = H.up_rows;
+    // sub-problems whose vector fits one CU's LDS are solved in one workgroup each
+    int lds = 0, dev = 0;
+    PYHIP_CHECK_HIP(hipGetDevice(&dev));
+    PYHIP_CHECK_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    IluSlicedPlan Q;
+    if (ilu_sliced_host(H, p->dof_off_h, std::max(0, std::min<int>(kIluSlicedRows, lds / (int)sizeof(double) - 1)), Q,
+                        err)) {
+        set_error(err);
+        return PYHIP_ERR_INVALID;
+    }
     L.lo_ptr = H.lo_ptr;
-    L.up_ptr = H.up_ptr;
+    L.lo_solve = Q.big_lo_ptr;
+    L.up_solve = Q.big_up_ptr;
     L.requested = W->ilu_order;
     L.multicolor = H.multicolor;
+    L.nsliced = (int)Q.subs.size();
+    L.max_rows = Q.max_rows;
     int rc;
 #define LUP(dst, v)                                                                        \
     if ((rc = kalloc(&(dst), (v).size(), W))) return rc;                                   \
-    PYHIP_CHECK_HIP(hipMemcpy(dst, (v).data(), (v).size() * sizeof((v)[0]), hipMemcpyHostToDevice));
-    LUP(L.perm, perm);
-    LUP(L.rs, prs);
-    LUP(L.col, pcol);
-    LUP(L.src, psrc);
-    LUP(L.diag, pdiag);
-    LUP(L.lo_rows, lo_rows);
-    LUP(L.up_rows, up_rows);
+    if (!(v).empty())                                                                      \
+        PYHIP_CHECK_HIP(hipMemcpy(dst, (v).data(), (v).size() * sizeof((v)[0]), hipMemcpyHostToDevice));
+    LUP(L.perm, H.perm);
+    LUP(L.rs, H.prs);
+    LUP(L.col, H.pcol);
+    LUP(L.src, H.psrc);
+    LUP(L.diag, H.pdiag);
+    LUP(L.lo_rows, H.lo_rows);
+    if (L.nsliced) {
+        LUP(L.ssubs, Q.subs);
+        LUP(L.srow0, Q.row0);
+        LUP(L.srows, Q.rows);
+        // the pivot of each lane's row on the upper side
+        std::vector<int32_t> dsrc(Q.up.idx.size() / 8, -1);
+        for (size_t t = 0; t < Q.subs.size(); t++) {
+            const int64_t c0 = Q.up.chunk0[t * kIluSliceWaves], c1 = Q.up.chunk0[(t + 1) * kIluSliceWaves];
+            for (int64_t k = c0 * kIluSliceLanes; k < c1 * kIluSliceLanes; k++) {
+                const uint16_t r = Q.up.idx[k * 8 + kIluChunk];
+                if (r != kIluNoRow) dsrc[k] = H.pdiag[Q.row0[t] + r];
+            }
+        }
+        LUP(L.sdsrc, dsrc);
+        L.ndiag = (int64_t)dsrc.size();
+        auto side = [&](IluPlan::Side &D, const IluSlicedSide &S) -> int {
+            LUP(D.nlev, S.nlev);
+            LUP(D.chunk0, S.chunk0);
+            LUP(D.src, S.src);
+            LUP(D.idx, S.idx);
+            D.nval = (int64_t)S.src.size();
+            return PYHIP_OK;
+        };
+        if ((rc = side(L.slo, Q.lo)) || (rc = side(L.sup, Q.up))) return rc;
+    }
+    if (!Q.big_lo.empty()) {
+        LUP(L.big_lo, Q.big_lo);
+        LUP(L.big_up, Q.big_up);
+        if ((rc = kalloc(&L.tmp64, n, W)) || (rc = kalloc(&L.tmp64b, n, W)) || (rc = kalloc(&L.tmp32, n, W)) ||
+            (rc = kalloc(&L.tmp32b, n, W)))
+            return rc;
+    }
 #undef LUP
-    if ((rc = kalloc(&L.tmp64, n, W)) || (rc = kalloc(&L.tmp64b, n, W)) ||
-        (rc = kalloc(&L.tmp32, n, W)) || (rc = kalloc(&L.tmp32b, n, W)))
-        return rc;
     L.n = n;
     L.nnz = p->nnz;
     L.built = true;
@@ -731,7 +781,22 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
     if (L.lu_prec != prec) {
         dfree(L.lu);
         L.lu = nullptr;
+        L.lu_prec = -1;
         if ((rc = dev_alloc((T **)&L.lu, L.nnz, W->bytes))) return rc;
+        for (void **q : {&L.slo.val, &L.sup.val, &L.sdiag}) {
+            dfree(*q);
+            *q = nullptr;
+        }
+        if (L.nsliced) {
+            if ((rc = dev_alloc((T **)&L.slo.val, L.slo.nval, W->bytes)) ||
+                (rc = dev_alloc((T **)&L.sup.val, L.sup.nval, W->bytes)) ||
+                (rc = dev_alloc((T **)&L.sdiag, L.ndiag, W->bytes)))
+                return rc;
+            // the solve's vector takes most of a CU's LDS
+            PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ilu_sliced_apply_kernel<T>),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                (int)((L.max_rows + 1) * sizeof(T))));
+        }
         L.lu_prec = prec;
     }
     T *lu = (T *)L.lu;
@@ -745,6 +810,14 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
                            L.lo_rows + L.lo_ptr[l], L.rs, L.col, L.diag, lu, W->nactive_d, L.perm, p->dof_sub,
                            need);
     }
+    auto fill = [&](int64_t m, const int32_t *src, void *val, int reciprocal) {
+        if (m)
+            hipLaunchKernelGGL((ilu_sliced_fill_kernel<T>), dim3(nblk(m)), dim3(256), 0, p->st, m, src, lu, (T *)val,
+                               reciprocal);
+    };
+    fill(L.slo.nval, L.slo.src, L.slo.val, 0);
+    fill(L.sup.nval, L.sup.src, L.sup.val, 0);
+    fill(L.ndiag, L.sdsrc, L.sdiag, 1);
     KCHECK();
     PYHIP_CHECK_HIP(hipMemcpyAsync(W->nactive_h, W->nactive_d, sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
     PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
@@ -755,25 +828,39 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
     return PYHIP_OK;
 }
 
+// z = (L U)^-1 v: the sub-problems of at most kIluSlicedRows rows in one launch, a workgroup
+// each (with act, those with act[s] != 0); the larger ones level by level.
 template <typename T>
-static int ilu_apply(pyhip_problem *p, KrylovWork *W, const T *v, T *z) {
+static int ilu_apply(pyhip_problem *p, KrylovWork *W, const T *v, T *z, const int32_t *act) {
     IluPlan &L = W->ilu;
     const T *lu = (const T *)L.lu;
+    const int64_t n = L.n;
+    if (L.nsliced) {
+        auto dev = [](const IluPlan::Side &S, const T *rdiag) {
+            return IluSlicedDev<T>{S.nlev, S.chunk0, S.idx, (const T *)S.val, rdiag};
+        };
+        hipLaunchKernelGGL((ilu_sliced_apply_kernel<T>), dim3(L.nsliced), dim3(kIluSlicedThreads),
+                           (size_t)(L.max_rows + 1) * sizeof(T), p->st, L.ssubs, L.srow0, L.srows, L.perm,
+                           dev(L.slo, nullptr), dev(L.sup, (const T *)L.sdiag), v, z, act);
+        KCHECK();
+    }
+    if (!L.big_lo) return PYHIP_OK;
     T *a = std::is_same<T, float>::value ? (T *)L.tmp32 : (T *)L.tmp64;
     T *b = std::is_same<T, float>::value ? (T *)L.tmp32b : (T *)L.tmp64b;
-    const int64_t n = L.n;
-    hipLaunchKernelGGL((permute_kernel<T, T>), dim3(nblk(n)), dim3(256), 0, p->st, n, L.perm, v, a, 1);
-    for (size_t l = 0; l + 1 < L.lo_ptr.size(); l++) {
-        const int64_t nr = L.lo_ptr[l + 1] - L.lo_ptr[l];
+    hipLaunchKernelGGL((permute_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, L.perm, v, a);
+    for (size_t l = 0; l + 1 < L.lo_solve.size(); l++) {
+        const int64_t nr = L.lo_solve[l + 1] - L.lo_solve[l];
         hipLaunchKernelGGL((trsv_level_kernel<T, true>), dim3(nblk(nr, 16)), dim3(256), 0, p->st, nr,
-                           L.lo_rows + L.lo_ptr[l], L.rs, L.col, L.diag, lu, a, b);
+                           L.big_lo + L.lo_solve[l], L.rs, L.col, L.diag, lu, a, b);
     }
-    for (size_t l = 0; l + 1 < L.up_ptr.size(); l++) {
-        const int64_t nr = L.up_ptr[l + 1] - L.up_ptr[l];
+    for (size_t l = 0; l + 1 < L.up_solve.size(); l++) {
+        const int64_t nr = L.up_solve[l + 1] - L.up_solve[l];
         hipLaunchKernelGGL((trsv_level_kernel<T, false>), dim3(nblk(nr, 16)), dim3(256), 0, p->st, nr,
-                           L.up_rows + L.up_ptr[l], L.rs, L.col, L.diag, lu, b, a);
+                           L.big_up + L.up_solve[l], L.rs, L.col, L.diag, lu, b, a);
     }
-    hipLaunchKernelGGL((permute_kernel<T, T>), dim3(nblk(n)), dim3(256), 0, p->st, n, L.perm, a, z, 0);
+    // back to the problem's order, the rows of the big sub-problems only
+    const int64_t nb = L.up_solve.back();
+    hipLaunchKernelGGL((unpermute_rows_kernel<T>), dim3(nblk(nb)), dim3(256), 0, p->st, nb, L.big_up, L.perm, a, z);
     KCHECK();
     return PYHIP_OK;
 }
@@ -968,13 +1055,13 @@ static int blk_apply(pyhip_problem *p, KrylovWork *W, const double *r, double *z
 }
 
 template <typename T>
-// z = M^-1 v. The multigrid V-cycle computes only the rows of sub-problems with
-// act[s] != 0 when act (device, host copy act_h) is given; the other preconditioners
-// compute every row.
+// z = M^-1 v. With act (device, host copy act_h) the multigrid V-cycle and the one-workgroup
+// ILU(0) solves compute only the rows of sub-problems with act[s] != 0; the other
+// preconditioners compute every row.
 static int precond_apply(pyhip_problem *p, KrylovWork *W, int pc, const T *v, T *z, const int32_t *act = nullptr,
                          const int32_t *act_h = nullptr, bool x0_ready = false) {
     TimeScope ts(&p->timer, "precond", p->st);
-    if (pc == PYHIP_PRECOND_ILU0) return ilu_apply<T>(p, W, v, z);
+    if (pc == PYHIP_PRECOND_ILU0) return ilu_apply<T>(p, W, v, z, act);
     if (pc == PYHIP_PRECOND_BLOCK) {
         if constexpr (std::is_same<T, double>::value) return blk_apply(p, W, v, z, act, act_h);
         set_error("the block preconditioner runs FP64 solves");
@@ -2021,9 +2108,7 @@ void pyhip_krylov_free(pyhip_problem *p) {
                     W->y, W->V, W->r64, W->x64, W->d64, W->b64, W->r32, W->d32, W->w32, W->t32,
                     W->w64, W->t64, W->vals32, W->vals64, W->res64, W->maxres, W->sub_scalar,
                     W->jdiag64, W->jdiag32, W->dof_mask, W->need, W->cg_rz, W->cg_pq,
-                    W->cg_beta, W->nfail_d, W->ilu.perm, W->ilu.rs, W->ilu.col,
-                    W->ilu.src, W->ilu.diag, W->ilu.lo_rows, W->ilu.up_rows, W->ilu.lu,
-                    W->ilu.tmp64, W->ilu.tmp64b, W->ilu.tmp32, W->ilu.tmp32b, W->achunk,
+                    W->cg_beta, W->nfail_d, W->achunk,
                     W->gpart, W->cg_iters, W->cg_iters2, W->cg_fail, W->ac_cur, W->ac_der, W->ac_y, W->ac_z,
                     W->ac_t, W->ac_zs, W->ac_alpha, W->ac_mask, W->amg_conv64};
     for (void *q : ptrs)
@@ -2033,6 +2118,7 @@ void pyhip_krylov_free(pyhip_problem *p) {
     if (W->maxres_h) (void)hipHostFree(W->maxres_h);
     amg_free(W->amg);
     blk_free(W);
+    ilu_free(W);
     if (W->achunk_h) (void)hipHostFree(W->achunk_h);
     if (W->flags_h) (void)hipHostFree(W->flags_h);
     delete W;

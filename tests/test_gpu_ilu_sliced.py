@@ -1,0 +1,51 @@
+"""One-workgroup ILU(0) solves (ilu_sliced.h): sub-problems on both sides of the rule that
+hands them a workgroup, alone and mixed in one batch, and in the solver plugin."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as sl
+
+pytestmark = pytest.mark.gpu
+
+
+def _solve(parts, precision="f64"):
+    from pyoomph_amd.problem import Problem
+    P = Problem(parts)
+    P.preconditioner = "ilu0"
+    if precision == "f32":
+        P.linear_precision = "f32"
+    st = P.solve()
+    x = P.get_current_dofs()
+    assert all(s["converged"] and s["linear_failures"] == 0 for s in st)
+    return [P.sub_dofs(i, x) for i in range(len(parts))]
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_batch_of_handled_and_level_scheduled_problems_equals_each_alone(gpu, precision):
+    from pyoomph_amd import workloads as wl
+    # 64^2 P2: more entries than a workgroup takes; the others: one workgroup each, natural
+    # order up to N = 17 P2, multicolour above; 2^2 P1: a single unknown
+    parts = [wl.bratu(17, "C2", 1.5), wl.bratu(64, "C2", 1.0), wl.bratu(2, "C1", 2.0), wl.bratu(33, "C1", 0.7),
+             wl.bratu(23, "C2", 2.5)]
+    together = _solve(parts, precision)
+    for mp, x in zip(parts, together):
+        assert np.array_equal(x, _solve([mp], precision)[0])
+
+
+@pytest.mark.parametrize("n,band", [(1, 1), (63, 3), (65, 64), (1500, 40), (20001, 2)])
+def test_plugin_solves_matrices_at_the_edges_of_the_rule(gpu, n, band):
+    """One row; rows of a slice and of a level that do not fill it; dense rows, many lanes
+    each; one row more than a workgroup's LDS holds."""
+    from pyoomph_amd.plugins import HIPKrylovSerial
+    rng = np.random.default_rng(n)
+    offs = [k for k in range(-band, band + 1) if abs(k) < n]
+    A = sp.diags([rng.uniform(-1, 1, n - abs(k)) for k in offs], offs, shape=(n, n)).tolil()
+    A.setdiag(2.0 * band + 2.0)
+    A = A.tocsr()
+    b = rng.standard_normal(n)
+    x = b.copy()
+    S = HIPKrylovSerial(None)
+    S.solve_serial(1, n, A.nnz, 1, A.data, A.indices, A.indptr, None, n, 1)
+    S.solve_serial(2, n, A.nnz, 1, None, None, None, x, n, 1)
+    want = sl.spsolve(A.tocsc(), b)
+    assert np.linalg.norm(x - want) <= 1e-9 * np.linalg.norm(want)

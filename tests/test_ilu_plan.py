@@ -227,3 +227,91 @@ def test_level_schedule_solves_like_a_sequential_sweep():
     for i in range(n - 1, -1, -1):
         xs[i] = (y[i] - (Us[i] @ xs)[0]) / d[i]
     assert np.allclose(x, xs, rtol=1e-13, atol=1e-13)
+
+
+def _sliced(P_args, off, cap, side):
+    """Copy of one side (0 lower, 1 upper) of the sliced plan (ilu_sliced_host)."""
+    L = _lib_ilu()
+    A, grp, order = P_args
+    rs, col = np.ascontiguousarray(A.indptr, np.int32), np.ascontiguousarray(A.indices, np.int32)
+    so, g = np.ascontiguousarray(off, np.int64), np.ascontiguousarray(grp, np.int8)
+    h = L.pyhip_ilu_plan_new(len(rs) - 1, rs.ctypes.data_as(_lib.c_i32p), col.ctypes.data_as(_lib.c_i32p), len(so) - 1,
+                             so.ctypes.data_as(_lib.c_i64p), g.ctypes.data_as(ctypes.POINTER(ctypes.c_int8)), order, 64)
+    assert h
+    vp = ctypes.c_void_p
+    f = L.pyhip_ilu_sliced_copy
+    f.argtypes = [vp, ctypes.c_int, _lib.c_i64p, ctypes.c_int, ctypes.c_int, _lib.c_i64p] + [vp] * 7
+    sz = np.zeros(4, np.int64)
+    head = [h, len(so) - 1, so.ctypes.data_as(_lib.c_i64p), cap, side, sz.ctypes.data_as(_lib.c_i64p)]
+    assert f(*head, *[None] * 7) == 0
+    ns, nc, nb, nbl = (int(v) for v in sz)
+    out = dict(subs=np.zeros(ns, np.int32), nlev=np.zeros(ns, np.int32), chunk0=np.zeros(16 * ns + 1, np.int32),
+               idx=np.zeros((nc, 64, 8), np.uint16), src=np.zeros((nc, 3, 64, 2), np.int32), big=np.zeros(nb, np.int32),
+               big_ptr=np.zeros(nbl + 1, np.int64))
+    assert f(*head, *[v.ctypes.data for v in out.values()]) == 0
+    L.pyhip_ilu_plan_free(h)
+    return out
+
+
+@pytest.mark.parametrize("cap", [0, 60, 1000])
+@pytest.mark.parametrize("order", [AUTO, NATURAL, MULTICOLOR])
+def test_sliced_solve_emulated_equals_the_triangular_solves(order, cap):
+    """The slices, walked as the one-workgroup solve walks them, give the triangular solves
+    of the permuted factor; sub-problems above the cap stay in the level lists."""
+    import scipy.sparse.linalg as sl
+    parts = [oracle_problem("ns", N=6), oracle_problem("bratu", N=9, space="C1", lam=1.0), oracle_problem("poisson", N=2),
+             oracle_problem("poisson", N=11)]
+    A, off, grp = _batch(parts)
+    P = _plan(A.indptr, A.indices, off, is_p=grp, order=order)
+    n = A.shape[0]
+    rng = np.random.default_rng(1)
+    lu = rng.uniform(-0.05, 0.05, len(P["pcol"]))
+    lu[P["pdiag"]] = rng.uniform(1.0, 2.0, n)
+    b = rng.standard_normal(n)
+    F = sp.csr_matrix((lu, P["pcol"], P["prs"]), shape=(n, n))
+    D = sp.diags(lu[P["pdiag"]])
+    want = {0: sl.spsolve_triangular((sp.tril(F, -1) + sp.eye(n)).tocsr(), b, lower=True),
+            1: sl.spsolve_triangular((sp.triu(F, 1) + D).tocsr(), b, lower=False)}
+    small = [s for s in range(len(parts)) if off[s + 1] - off[s] <= cap]
+    for side in (0, 1):
+        S = _sliced((A, grp, order), off, cap, side)
+        assert sorted(S["subs"]) == small
+        # rows of the other sub-problems, every one in a level of its own side
+        rest = np.concatenate([np.arange(off[s], off[s + 1]) for s in range(len(parts)) if s not in small] or [[]])
+        assert np.array_equal(np.sort(S["big"]), rest) and S["big_ptr"][-1] == len(rest)
+        for t, s in enumerate(S["subs"]):
+            r0, m = off[s], off[s + 1] - off[s]
+            x = np.append(b[r0:r0 + m], 0.0)
+            seen = np.zeros(m, int)
+            for lv in range(S["nlev"][t]):
+                new = {}
+                for wave in range(16 * t, 16 * t + 16):
+                    lo, hi = S["chunk0"][wave:wave + 2]
+                    assert (hi - lo) % 3 == 0
+                    marks = S["idx"][lo:hi, :, 7].astype(int)
+                    assert np.all(marks == marks[:, :1]) and np.all(np.diff(marks[:, 0] & 0xfff) >= 0)
+                    acc = np.zeros(64)
+                    for ch in range(lo, hi):
+                        mark = int(S["idx"][ch, 0, 7])
+                        if mark & 0xfff != lv:
+                            continue
+                        lanes = 1 << ((mark >> 12) & 7)
+                        c = S["idx"][ch, :, :6].astype(int).T            # [step][lane]
+                        q = S["src"][ch].transpose(0, 2, 1).reshape(6, 64)
+                        assert lanes <= 16 and np.all(c <= m) and np.all((q < 0) == (c == m))
+                        acc += (np.where(q >= 0, lu[q], 0.0) * x[c]).sum(0)
+                        if mark >> 15:
+                            continue
+                        lane, acc, row = acc, np.zeros(64), S["idx"][ch, :, 6]
+                        for g in range(0, 64, lanes):
+                            if row[g] == 0xffff:
+                                continue
+                            assert np.all(row[g:g + lanes] == row[g])
+                            r = int(row[g])
+                            v = x[r] - lane[g:g + lanes].sum()
+                            new[r] = v / lu[P["pdiag"][r0 + r]] if side else v
+                            seen[r] += 1
+                for r, v in new.items():   # rows of one level do not read each other
+                    x[r] = v
+            assert np.all(seen == 1)
+            assert np.allclose(x[:m], want[side][r0:r0 + m], rtol=1e-12, atol=1e-13)
