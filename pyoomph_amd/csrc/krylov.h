@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "amg.h"
+#include "gmres_kernels.h"
 #include "problem.h"
 
 namespace pyhip {
@@ -83,6 +84,13 @@ struct KrylovWork {
     int32_t *sub_chunk_ptr = nullptr; // [nsub+1]
     double *partial = nullptr;        // [nchunk][m+2]
     double *dots = nullptr;           // [m+2][nsub]
+    // GMRES orthogonalisation (gmres_kernels.h): its chunks and their partial sums
+    int64_t *gs_begin = nullptr, *gs_end = nullptr;
+    int32_t *gs_sub = nullptr, *gs_ptr = nullptr;
+    int64_t gs_count = 0;
+    int gs_max = 0;                   // chunks of the largest sub-problem
+    double *gs_part1 = nullptr, *gs_part2 = nullptr;   // [m+1][gs_count]
+    GsChunks gs_chunks() const { return GsChunks{gs_begin, gs_end, gs_sub, gs_ptr, gs_count}; }
     // GMRES state per sub-problem
     double *H = nullptr;              // [nsub][m+1][m]
     double *cs = nullptr, *sn = nullptr;  // [nsub][m]

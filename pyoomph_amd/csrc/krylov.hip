@@ -105,23 +105,6 @@ __global__ __launch_bounds__(64) void reduce_partials_kernel(int nvec, int nsub,
     if (threadIdx.x == 0) out[j * nsub + s] = acc;
 }
 
-// w -= sum_j h[j][sub] V_j  (h = dots of this Gram-Schmidt pass)
-template <typename T>
-__global__ __launch_bounds__(256) void cgs_update_kernel(int64_t n, int nvec, int nsub,
-                                                         const T *__restrict__ V, int64_t ldv,
-                                                         const double *__restrict__ h,
-                                                         const int32_t *__restrict__ dsub,
-                                                         const int32_t *__restrict__ active,
-                                                         T *__restrict__ w) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int s = dsub[i];
-    if (!active[s]) return;
-    double acc = double(w[i]);
-    for (int j = 0; j < nvec; j++) acc -= h[j * nsub + s] * double(V[(int64_t)j * ldv + i]);
-    w[i] = T(acc);
-}
-
 // out = in * (1 / nrm[sub]) (0 where nrm == 0); only active sub-problems
 template <typename T>
 __global__ __launch_bounds__(256) void scale_kernel(int64_t n, const T *in,
@@ -151,7 +134,7 @@ __global__ void gmres_start_kernel(int nsub, int m, const double *__restrict__ n
                                    const double *__restrict__ bnorm, double tol, double stag, int first,
                                    const int32_t *__restrict__ need, double *__restrict__ g,
                                    int32_t *__restrict__ active, int32_t *__restrict__ kcols,
-                                   double *__restrict__ beta0, int32_t *__restrict__ nactive) {
+                                   double *__restrict__ beta0) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nsub) return;
     const double beta = sqrt(nrm2[s]);
@@ -162,68 +145,6 @@ __global__ void gmres_start_kernel(int nsub, int m, const double *__restrict__ n
     g[s * (m + 1)] = beta;
     const int a = need[s] && (beta > tol * bnorm[s]) && isfinite(beta) && !stalled;
     active[s] = a;
-    if (a) atomicAdd(nactive, 1);
-}
-
-// Column k of the Hessenberg: h[0..k] = dots (CGS pass 1 + pass 2), h[k+1] = |w|.
-// m: stride of the per-sub-problem Hessenberg / Givens arrays (the workspace's restart
-// capacity); mr <= m: the restart length of this solve (the cycle ends after column mr-1).
-__global__ void gmres_givens_kernel(int nsub, int m, int mr, int k, const double *__restrict__ d1,
-                                    const double *__restrict__ d2, const double *__restrict__ wn2,
-                                    double *__restrict__ H, double *__restrict__ cs,
-                                    double *__restrict__ sn, double *__restrict__ g,
-                                    const double *__restrict__ bnorm, double tol,
-                                    int32_t *__restrict__ active, int32_t *__restrict__ kcols,
-                                    int32_t *__restrict__ nactive) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsub || !active[s]) return;
-    double *Hs = H + (int64_t)s * (m + 1) * m;
-    double *cs_s = cs + (int64_t)s * m, *sn_s = sn + (int64_t)s * m, *gs = g + (int64_t)s * (m + 1);
-    // column k is rotated in place: Hs[i * m + k], i = 0..k (row k + 1 is only carried in
-    // a register, since the rotation zeroes it)
-    double hi = d1[s] + d2[s];
-    for (int i = 0; i < k; i++) {
-        const double hn = d1[(i + 1) * nsub + s] + d2[(i + 1) * nsub + s];
-        Hs[i * m + k] = cs_s[i] * hi + sn_s[i] * hn;
-        hi = -sn_s[i] * hi + cs_s[i] * hn;
-    }
-    const double hk1 = sqrt(wn2[s]);
-    const double den = hypot(hi, hk1);
-    double c = 1.0, sv = 0.0;
-    if (den > 0.0) {
-        c = hi / den;
-        sv = hk1 / den;
-    }
-    cs_s[k] = c;
-    sn_s[k] = sv;
-    Hs[k * m + k] = den;
-    gs[k + 1] = -sv * gs[k];
-    gs[k] = c * gs[k];
-    kcols[s] = k + 1;
-    const bool done = !(fabs(gs[k + 1]) > tol * bnorm[s]) || hk1 == 0.0 || den == 0.0 ||
-                      !isfinite(gs[k + 1]) || (k + 1 == mr);
-    if (done) active[s] = 0;
-    else atomicAdd(nactive, 1);
-}
-
-// y = R^{-1} g (upper triangular back substitution of the rotated Hessenberg)
-__global__ void gmres_backsolve_kernel(int nsub, int m, const double *__restrict__ H,
-                                       const double *__restrict__ g,
-                                       const int32_t *__restrict__ kcols,
-                                       double *__restrict__ y) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsub) return;
-    const double *Hs = H + (int64_t)s * (m + 1) * m;
-    const double *gs = g + (int64_t)s * (m + 1);
-    double *ys = y + (int64_t)s * m;
-    const int k = kcols[s];
-    for (int i = k - 1; i >= 0; i--) {
-        double acc = gs[i];
-        for (int j = i + 1; j < k; j++) acc -= Hs[i * m + j] * ys[j];
-        const double d = Hs[i * m + i];
-        ys[i] = d != 0.0 ? acc / d : 0.0;
-    }
-    for (int i = k; i < m; i++) ys[i] = 0.0;
 }
 
 // t = sum_{j < kcols[sub]} y_j V_j
@@ -456,6 +377,27 @@ static int krylov_setup(pyhip_problem *p, int m) {
         KUP(W->chunk_begin, cb);
         KUP(W->chunk_end, ce);
         KUP(W->sub_chunk_ptr, scp);
+        // chunks of the GMRES orthogonalisation, rows per chunk by the sub-problem's rows
+        {
+            std::vector<int64_t> gb, ge;
+            std::vector<int32_t> gsub, gptr(p->nsub + 1, 0);
+            for (int s = 0; s < p->nsub; s++) {
+                gptr[s] = (int32_t)gb.size();
+                const int step = gs_chunk_rows(p->dof_off_h[s + 1] - p->dof_off_h[s]);
+                for (int64_t b = p->dof_off_h[s]; b < p->dof_off_h[s + 1]; b += step) {
+                    gb.push_back(b);
+                    ge.push_back(std::min<int64_t>(b + step, p->dof_off_h[s + 1]));
+                    gsub.push_back(s);
+                }
+                W->gs_max = std::max(W->gs_max, (int)gb.size() - gptr[s]);
+            }
+            gptr[p->nsub] = (int32_t)gb.size();
+            W->gs_count = (int64_t)gb.size();
+            KUP(W->gs_begin, gb);
+            KUP(W->gs_end, ge);
+            KUP(W->gs_sub, gsub);
+            KUP(W->gs_ptr, gptr);
+        }
 #undef KUP
         const int64_t n = W->n, ns = W->nsub;
         if ((rc = kalloc(&W->beta0, ns, W)) || (rc = kalloc(&W->bnorm, ns, W)) ||
@@ -501,6 +443,8 @@ static int krylov_setup(pyhip_problem *p, int m) {
     dfree(W->sn);
     dfree(W->g);
     dfree(W->y);
+    dfree(W->gs_part1);
+    dfree(W->gs_part2);
     dfree(W->V);
     W->V = nullptr;
     W->vprec = -1;
@@ -510,7 +454,8 @@ static int krylov_setup(pyhip_problem *p, int m) {
         (rc = kalloc(&W->dots, (size_t)3 * (m + 2) * ns, W)) ||
         (rc = kalloc(&W->H, (size_t)ns * (m + 1) * m, W)) || (rc = kalloc(&W->cs, (size_t)ns * m, W)) ||
         (rc = kalloc(&W->sn, (size_t)ns * m, W)) || (rc = kalloc(&W->g, (size_t)ns * (m + 1), W)) ||
-        (rc = kalloc(&W->y, (size_t)ns * m, W)))
+        (rc = kalloc(&W->y, (size_t)ns * m, W)) || (rc = kalloc(&W->gs_part1, (size_t)(m + 1) * W->gs_count, W)) ||
+        (rc = kalloc(&W->gs_part2, (size_t)(m + 1) * W->gs_count, W)))
         return rc;
     W->m = m;
     return PYHIP_OK;
@@ -1182,83 +1127,82 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     KCHECK();
     // x0 = 0
     PYHIP_CHECK_HIP(hipMemsetAsync(x, 0, n * sizeof(T), p->st));
-    int total = 0;
+    // running sub-problems: the flags come to the host now and then; between reads they only
+    // lose sub-problems, so the host copy stays a superset (it sizes the byte counts of the
+    // filtered launches; the device flags decide which rows are computed)
+    int32_t *act_h = W->act_h;
+    auto read_active = [&](int *count) -> int {
+        PYHIP_CHECK_HIP(hipMemcpyAsync(act_h, W->active, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
+        PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
+        *count = 0;
+        for (int s = 0; s < ns; s++) *count += act_h[s] != 0;
+        return PYHIP_OK;
+    };
+    const GsChunks C = W->gs_chunks();
+    const bool reduced = W->gs_max > kGsFusedChunks;
+    PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gs_backsolve_kernel),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)gs_backsolve_lds(m, mr)));
+    int total = 0, nact = 0;
     const int max_cycles = std::max(1, (o.max_iters + mr - 1) / mr);
     for (int cyc = 0; cyc < max_cycles; cyc++) {
         // r = b - A x  -> V_0 (unnormalised)
         if ((rc = spmv<TV, T, T>(p, vals, x, V, b))) return rc;
         if ((rc = batched_dots<T>(p, W, 1, V, n, V, d3))) return rc;
-        PYHIP_CHECK_HIP(hipMemsetAsync(W->nactive_d, 0, sizeof(int32_t), p->st));
         hipLaunchKernelGGL(gmres_start_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, d3,
-                           W->bnorm, rtol, stag, cyc == 0 ? 1 : 0, need, W->g, W->active, W->kcols, W->beta0,
-                           W->nactive_d);
+                           W->bnorm, rtol, stag, cyc == 0 ? 1 : 0, need, W->g, W->active, W->kcols, W->beta0);
         KCHECK();
-        // the running flags come to the host with the count: between reads they only lose
-        // sub-problems, so the host copy stays a superset (it sizes the byte counts of the
-        // filtered launches; the device flags decide which rows are computed)
-        int32_t *act_h = W->act_h;
-        PYHIP_CHECK_HIP(hipMemcpyAsync(W->nactive_h, W->nactive_d, sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-        PYHIP_CHECK_HIP(hipMemcpyAsync(act_h, W->active, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-        PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
+        if ((rc = read_active(&nact))) return rc;
         if (debug_enabled()) {
             double b0 = 0, bn = 0;
             (void)hipMemcpy(&b0, W->beta0, sizeof(double), hipMemcpyDeviceToHost);
             (void)hipMemcpy(&bn, W->bnorm, sizeof(double), hipMemcpyDeviceToHost);
             fprintf(stderr, "[pyhip] gmres cycle %d: active %d |r| %.3e |b| %.3e iters %d\n", cyc,
-                    *W->nactive_h, b0, bn, total);
+                    nact, b0, bn, total);
         }
-        if (*W->nactive_h == 0) break;
+        if (nact == 0) break;
         hipLaunchKernelGGL((scale_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, V, d3, p->dof_sub,
                            W->active, V);
         KCHECK();
         int k = 0;
         for (; k < mr; k++) {
             T *vk = V + (int64_t)k * n;
-            // the preconditioner (multigrid) and the spmv skip the rows of stopped
-            // sub-problems: nothing reads their t and w
+            // the preconditioner and the spmv skip the rows of stopped sub-problems: nothing
+            // reads their t and w
             if ((rc = precond_apply<T>(p, W, o.precond, vk, t, W->active, act_h))) return rc;
             if ((rc = spmv<TV, T, T>(p, vals, t, w, (const T *)nullptr, W->active, act_h))) return rc;
-            // CGS2
-            // (the Gram-Schmidt dots skip the sub-problems that have stopped: every kernel
-            // that reads them skips those too)
-            if ((rc = batched_dots<T>(p, W, k + 1, V, n, w, d1, W->active))) return rc;
             {
                 TimeScope tsu(&p->timer, "vector", p->st);
-                hipLaunchKernelGGL((cgs_update_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, k + 1, ns, V,
-                                   n, d1, p->dof_sub, W->active, w);
+                const dim3 grid((unsigned)C.count), thr(kGsThreads);
+                const size_t lds = gs_update_lds(k + 1, sizeof(T));
+                auto reduce = [&](const double *part, double *out) {
+                    if (reduced)
+                        hipLaunchKernelGGL(gs_reduce_kernel, dim3((unsigned)((k + 1) * ns)), dim3(64), 0, p->st, ns, C,
+                                           W->active, part, out);
+                };
+                hipLaunchKernelGGL((gs_dot_kernel<T>), grid, thr, 0, p->st, k + 1, V, n, w, C, W->active, W->gs_part1);
+                reduce(W->gs_part1, d1);
+                hipLaunchKernelGGL((gs_update_kernel<T, false>), grid, thr, lds, p->st, k + 1, ns, V, n, w, C, W->active,
+                                   W->gs_part1, d1, reduced ? 1 : 0, W->gs_part2);
+                reduce(W->gs_part2, d2);
+                hipLaunchKernelGGL((gs_update_kernel<T, true>), grid, thr, lds, p->st, k + 1, ns, V, n, w, C, W->active,
+                                   W->gs_part2, d2, reduced ? 1 : 0, W->gs_part1);
+                hipLaunchKernelGGL((gs_finish_kernel<T>), grid, thr, 3 * (size_t)(m + 1) * sizeof(double), p->st, ns, m,
+                                   mr, k, w, V + (int64_t)(k + 1) * n, C, W->gs_part1, d1, d2, W->H, W->cs, W->sn, W->g,
+                                   W->bnorm, rtol, W->active, W->kcols);
             }
-            if ((rc = batched_dots<T>(p, W, k + 1, V, n, w, d2, W->active))) return rc;
-            {
-                TimeScope tsu(&p->timer, "vector", p->st);
-                hipLaunchKernelGGL((cgs_update_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, k + 1, ns, V,
-                                   n, d2, p->dof_sub, W->active, w);
-            }
-            if ((rc = batched_dots<T>(p, W, 1, w, n, w, d3, W->active))) return rc;
-            {
-                TimeScope tsu(&p->timer, "vector", p->st);
-                hipLaunchKernelGGL((scale_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, w, d3, p->dof_sub,
-                                   W->active, V + (int64_t)(k + 1) * n);
-            }
-            PYHIP_CHECK_HIP(hipMemsetAsync(W->nactive_d, 0, sizeof(int32_t), p->st));
-            hipLaunchKernelGGL(gmres_givens_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, mr, k, d1, d2,
-                               d3, W->H, W->cs, W->sn, W->g, W->bnorm, rtol, W->active, W->kcols,
-                               W->nactive_d);
             KCHECK();
             total++;
-            // the host reads the number of sub-problems still iterating every kGmresCheck
-            // iterations (and at the end of the cycle); in between, a sub-problem that
-            // has converged keeps its state (every kernel skips it) while the others go on
+            // the host reads the flags every kGmresCheck iterations (and at the end of the
+            // cycle); in between, a sub-problem that has converged keeps its state (every
+            // kernel skips it) while the others go on
             if ((k + 1) % kGmresCheck == 0 || k + 1 == mr) {
-                PYHIP_CHECK_HIP(hipMemcpyAsync(W->nactive_h, W->nactive_d, sizeof(int32_t), hipMemcpyDeviceToHost,
-                                               p->st));
-                PYHIP_CHECK_HIP(hipMemcpyAsync(act_h, W->active, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-                PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
-                if (*W->nactive_h == 0) break;
+                if ((rc = read_active(&nact))) return rc;
+                if (nact == 0) break;
             }
         }
         // x += M^{-1} V y
-        hipLaunchKernelGGL(gmres_backsolve_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, W->H, W->g,
-                           W->kcols, W->y);
+        hipLaunchKernelGGL(gs_backsolve_kernel, dim3(ns), dim3(64), gs_backsolve_lds(m, mr), p->st, m, W->H, W->g,
+                           W->kcols, std::min(mr, kGsBackCols), W->y);
         hipLaunchKernelGGL((combine_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, m, V, n, W->y,
                            W->kcols, p->dof_sub, w);
         KCHECK();
@@ -1271,16 +1215,13 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     // sub-problems still above tolerance (true residual of the returned x)
     if ((rc = spmv<TV, T, T>(p, vals, x, V, b))) return rc;
     if ((rc = batched_dots<T>(p, W, 1, V, n, V, d3))) return rc;
-    PYHIP_CHECK_HIP(hipMemsetAsync(W->nactive_d, 0, sizeof(int32_t), p->st));
     hipLaunchKernelGGL(gmres_start_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, d3, W->bnorm,
-                       rtol * 1.01, 0.0, 1, need, W->g, W->active, W->kcols, W->beta0, W->nactive_d);
+                       rtol * 1.01, 0.0, 1, need, W->g, W->active, W->kcols, W->beta0);
     KCHECK();
-    PYHIP_CHECK_HIP(hipMemcpyAsync(W->nactive_h, W->nactive_d, sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-    PYHIP_CHECK_HIP(hipMemcpyAsync(W->act_h, W->active, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-    PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
+    if ((rc = read_active(&nact))) return rc;
     // a sub-problem still marked active is above its tolerance
-    W->lfail_h.assign(W->act_h, W->act_h + ns);
-    *failed = *W->nactive_h;
+    W->lfail_h.assign(act_h, act_h + ns);
+    *failed = nact;
     *iters = total;
     return PYHIP_OK;
 }
@@ -2104,7 +2045,7 @@ void pyhip_krylov_free(pyhip_problem *p) {
     KrylovWork *W = p->kw;
     if (!W) return;
     void *ptrs[] = {W->chunk_sub, W->chunk_begin, W->chunk_end, W->sub_chunk_ptr, W->partial, W->dots,
-                    W->H, W->cs, W->sn, W->g, W->beta0, W->bnorm, W->kcols, W->active, W->nactive_d,
+                    W->gs_begin, W->gs_end, W->gs_sub, W->gs_ptr, W->gs_part1, W->gs_part2, W->H, W->cs, W->sn, W->g, W->beta0, W->bnorm, W->kcols, W->active, W->nactive_d,
                     W->y, W->V, W->r64, W->x64, W->d64, W->b64, W->r32, W->d32, W->w32, W->t32,
                     W->w64, W->t64, W->vals32, W->vals64, W->res64, W->maxres, W->sub_scalar,
                     W->jdiag64, W->jdiag32, W->dof_mask, W->need, W->cg_rz, W->cg_pq,
