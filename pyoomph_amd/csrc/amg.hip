@@ -577,9 +577,9 @@ static int64_t active_sum(const std::vector<int64_t> &v, const int32_t *act_h) {
 }
 
 
-// Variants of each level's three spmv launches: the fastest of the canonical spmv's
-// variants (1, 2, 4, 8 lanes per row, LDS staging) over two timed launches each, once per
-// hierarchy (every variant gives the same bits, so the choice changes no result), or
+// Variants of each level's three spmv launches: by rule for small matrices
+// (spmv_small_variant), else the fastest of the canonical spmv's variants over two timed
+// launches each, once per hierarchy (every variant gives the same bits, so the choice changes no result), or
 // PYHIP_SPMV_LPR for all of them. The outputs are scratch vectors of the level.
 static int tune_levels(AmgDev &A, hipStream_t st) {
     if (const char *e = getenv("PYHIP_SPMV_LPR")) {
@@ -592,7 +592,8 @@ static int tune_levels(AmgDev &A, hipStream_t st) {
     hipEvent_t e0, e1;
     PYHIP_CHECK_HIP(hipEventCreate(&e0));
     PYHIP_CHECK_HIP(hipEventCreate(&e1));
-    auto pick = [&](auto &&launch) {
+    auto pick = [&](int64_t n, int64_t nnz, auto &&launch) {
+        if (const int v = spmv_small_variant(n, nnz)) return v;
         float best = 1e30f;
         int arg = 8;
         for (int lpr : kSpmvVariants) {
@@ -612,14 +613,14 @@ static int tune_levels(AmgDev &A, hipStream_t st) {
     for (size_t l = 0; l < A.lv.size(); l++) {
         AmgDevLevel &L = A.lv[l];
         AmgDevLevel &C = (l + 1 < A.lv.size()) ? A.lv[l + 1] : A.bot;
-        L.lpr_a = pick([&](int lpr) {
+        L.lpr_a = pick(L.n, L.nnz, [&](int lpr) {
             launch_spmv<double, double, double>(lpr, st, L.n, L.rs, L.col, L.vals, L.b, L.r, nullptr);
         });
         if (L.nc) {
-            L.lpr_t = pick([&](int lpr) {
+            L.lpr_t = pick(L.nc, L.nnzp, [&](int lpr) {
                 launch_spmv<double, double, double>(lpr, st, L.nc, L.trs, L.trow, L.ptv, L.r, C.b, nullptr);
             });
-            L.lpr_p = pick([&](int lpr) {
+            L.lpr_p = pick(L.n, L.nnzp, [&](int lpr) {
                 launch_spmv_add<double, double, double>(lpr, st, L.n, L.prs, L.pcol, L.pv, C.x, L.x2, L.x2);
             });
         }

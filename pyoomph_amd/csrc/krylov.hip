@@ -509,9 +509,10 @@ int batched_maxabs(pyhip_problem *p, const double *v, double *out) {
     return PYHIP_OK;
 }
 
-// Variant of this problem's spmv: the fastest of the canonical spmv's variants (1, 2, 4 or
-// 8 lanes per row, LDS staging) over two timed launches each, all giving the same bits, or
-// PYHIP_SPMV_LPR. The work-list CG kernel takes the fastest lane count. y is scratch here.
+// Variant of this problem's spmv: by rule for small matrices (spmv_small_variant), else the
+// fastest of the canonical spmv's variants over two timed launches each, all giving the same
+// bits, or PYHIP_SPMV_LPR. The work-list CG kernel takes the fastest of its lane counts (1, 2,
+// 4, 8; small matrices: by the mean row length). y is scratch here.
 template <typename TV, typename TX, typename TY>
 static int spmv_tune(pyhip_problem *p, KrylovWork *W, const TV *vals, const TX *x, TY *y) {
     if (W->smode) return PYHIP_OK;
@@ -526,6 +527,11 @@ static int spmv_tune(pyhip_problem *p, KrylovWork *W, const TV *vals, const TX *
     const int64_t n = p->ndof;
     W->smode = W->lpr = 8;
     if (n == 0) return PYHIP_OK;
+    if (const int v = spmv_small_variant(n, p->nnz)) {
+        W->smode = v;
+        W->lpr = p->nnz <= 12 * n ? 4 : 8;
+        return PYHIP_OK;
+    }
     hipEvent_t e0, e1;
     PYHIP_CHECK_HIP(hipEventCreate(&e0));
     PYHIP_CHECK_HIP(hipEventCreate(&e1));

@@ -15,23 +15,24 @@ __device__ __forceinline__ float fmadd(float a, float b, float c) { return __bui
 // combine as ((S0+S4)+(S2+S6)) + ((S1+S5)+(S3+S7)). LPR lanes per row (1, 2, 4 or 8;
 // lane l owns stripes l, l+LPR, ...) all give the same bits, so the lane count can be
 // tuned per problem without changing any result.
-// A thread serves LPR rows of a 256-row block (rows r0 + p*(256/LPR) + threadIdx.x/LPR,
-// p = 0..LPR-1) and issues the loads of all of them together: 8 (row, stripe) streams in
-// flight per thread, whatever LPR. All lanes of a row call this; out[p] is the sum of
-// row p (rows at or past r1: 0). With a row filter (rsub, act non-null) a row whose
-// sub-problem rsub[row] has act[...] == 0 is skipped: live[p] tells which rows to store.
-template <typename TV, typename TX, typename TY, int LPR>
+// A thread serves NR rows of a block of NR * (256 / LPR) rows (rows r0 + p*(256/LPR) +
+// threadIdx.x/LPR, p = 0..NR-1) and issues the loads of all of them together, NU entries of
+// each stripe at a time: NR * NU * 8 / LPR (row, entry) loads in flight per thread. All lanes
+// of a row call this; out[p] is the sum of row p (rows at or past r1: 0). With a row filter
+// (rsub, act non-null) a row whose sub-problem rsub[row] has act[...] == 0 is skipped:
+// live[p] tells which rows to store.
+template <typename TV, typename TX, typename TY, int LPR, int NR = LPR, int NU = 1>
 __device__ __forceinline__ void rows_dot(int64_t r0, int64_t r1, const int32_t *__restrict__ rs,
                                          const int32_t *__restrict__ col, const TV *__restrict__ val,
                                          const TX *__restrict__ x, const int32_t *__restrict__ rsub,
-                                         const int32_t *__restrict__ act, TY (&out)[LPR],
-                                         bool (&live)[LPR]) {
+                                         const int32_t *__restrict__ act, TY (&out)[NR],
+                                         bool (&live)[NR]) {
     constexpr int NS = 8 / LPR, RPP = 256 / LPR;
     const int lane = threadIdx.x % LPR;
-    int32_t k0[LPR], k1[LPR];
+    int32_t k0[NR], k1[NR];
     int32_t len = 0;
 #pragma unroll
-    for (int p = 0; p < LPR; p++) {
+    for (int p = 0; p < NR; p++) {
         const int64_t row = r0 + p * RPP + threadIdx.x / LPR;
         const bool ok = row < r1 && (act == nullptr || act[rsub[row]] != 0);
         live[p] = ok;
@@ -39,35 +40,41 @@ __device__ __forceinline__ void rows_dot(int64_t r0, int64_t r1, const int32_t *
         k1[p] = ok ? rs[row + 1] : 0;
         len = max(len, k1[p] - k0[p]);
     }
-    TY acc[LPR][NS];
+    TY acc[NR][NS];
 #pragma unroll
-    for (int p = 0; p < LPR; p++)
+    for (int p = 0; p < NR; p++)
 #pragma unroll
         for (int j = 0; j < NS; j++) acc[p][j] = TY(0);
-    for (int32_t base = lane; base < len; base += 8) {
-        int32_t cc[LPR][NS];
-        TY vv[LPR][NS], xx[LPR][NS];
+    for (int32_t base = lane; base < len; base += 8 * NU) {
+        int32_t cc[NR][NU][NS];
+        TY vv[NR][NU][NS], xx[NR][NU][NS];
 #pragma unroll
-        for (int p = 0; p < LPR; p++)
+        for (int p = 0; p < NR; p++)
 #pragma unroll
-            for (int j = 0; j < NS; j++) {
-                const int32_t k = k0[p] + base + j * LPR;
-                const bool in = k < k1[p];
-                cc[p][j] = in ? col[k] : -1;
-                vv[p][j] = in ? TY(val[k]) : TY(0);
-            }
+            for (int u = 0; u < NU; u++)
 #pragma unroll
-        for (int p = 0; p < LPR; p++)
+                for (int j = 0; j < NS; j++) {
+                    const int32_t k = k0[p] + base + 8 * u + j * LPR;
+                    const bool in = k < k1[p];
+                    cc[p][u][j] = in ? col[k] : -1;
+                    vv[p][u][j] = in ? TY(val[k]) : TY(0);
+                }
 #pragma unroll
-            for (int j = 0; j < NS; j++) xx[p][j] = cc[p][j] >= 0 ? TY(x[cc[p][j]]) : TY(0);
+        for (int p = 0; p < NR; p++)
 #pragma unroll
-        for (int p = 0; p < LPR; p++)
+            for (int u = 0; u < NU; u++)
 #pragma unroll
-            for (int j = 0; j < NS; j++)
-                if (cc[p][j] >= 0) acc[p][j] = fmadd(vv[p][j], xx[p][j], acc[p][j]);
+                for (int j = 0; j < NS; j++) xx[p][u][j] = cc[p][u][j] >= 0 ? TY(x[cc[p][u][j]]) : TY(0);
+#pragma unroll
+        for (int p = 0; p < NR; p++)
+#pragma unroll
+            for (int u = 0; u < NU; u++)
+#pragma unroll
+                for (int j = 0; j < NS; j++)
+                    if (cc[p][u][j] >= 0) acc[p][j] = fmadd(vv[p][u][j], xx[p][u][j], acc[p][j]);
     }
 #pragma unroll
-    for (int p = 0; p < LPR; p++) {
+    for (int p = 0; p < NR; p++) {
         TY v;
         if constexpr (LPR == 8) v = acc[p][0];
         else if constexpr (LPR == 4) v = acc[p][0] + acc[p][1];
@@ -99,9 +106,9 @@ __device__ __forceinline__ void spmv_store(int64_t row, TY v, const TX *x, TY *y
     }
 }
 
-// 256 rows per block (rows_dot); the grid is a multiple of 8 (spmv_grid). Rows the filter
-// skips keep their outputs.
-template <typename TV, typename TX, typename TY, int LPR, int EPI>
+// NR * (256 / LPR) rows per block (rows_dot); the grid is a multiple of 8 (spmv_grid). Rows
+// the filter skips keep their outputs.
+template <typename TV, typename TX, typename TY, int LPR, int EPI, int NR = LPR, int NU = 1>
 __global__ __launch_bounds__(256) void spmv_kernel(int64_t n, const int32_t *__restrict__ rs,
                                                    const int32_t *__restrict__ col,
                                                    const TV *__restrict__ val,
@@ -109,18 +116,18 @@ __global__ __launch_bounds__(256) void spmv_kernel(int64_t n, const int32_t *__r
                                                    const TY *__restrict__ w, TY *__restrict__ out,
                                                    const int32_t *__restrict__ rsub,
                                                    const int32_t *__restrict__ act) {
-    constexpr int RPP = 256 / LPR;
+    constexpr int RPP = 256 / LPR, RPB = NR * RPP;
     // blocks round-robin over the 8 XCDs: XCD x gets the contiguous block range x*per..
-    const int64_t nb = (n + 255) / 256, per = (nb + 7) / 8, k = blockIdx.x / 8;
+    const int64_t nb = (n + RPB - 1) / RPB, per = (nb + 7) / 8, k = blockIdx.x / 8;
     const int64_t lb = (int64_t)(blockIdx.x % 8) * per + k;
     if (k >= per || lb >= nb) return;
-    const int64_t r0 = lb * 256;
-    TY v[LPR];
-    bool live[LPR];
-    rows_dot<TV, TX, TY, LPR>(r0, n, rs, col, val, x, rsub, act, v, live);
+    const int64_t r0 = lb * RPB;
+    TY v[NR];
+    bool live[NR];
+    rows_dot<TV, TX, TY, LPR, NR, NU>(r0, n, rs, col, val, x, rsub, act, v, live);
     if (threadIdx.x % LPR == 0) {
 #pragma unroll
-        for (int p = 0; p < LPR; p++) {
+        for (int p = 0; p < NR; p++) {
             const int64_t row = r0 + p * RPP + threadIdx.x / LPR;
             if (live[p]) spmv_store<EPI>(row, v[p], x, y, b, w, out);
         }
@@ -198,19 +205,32 @@ __global__ __launch_bounds__(256) void spmv_lds_kernel(int64_t n, const int32_t 
     }
 }
 
-// Variants of the canonical spmv (all give the same bits): 1, 2, 4, 8 lanes per row
-// (spmv_kernel), or LDS staging with chunks of 512, 1024, 2048 or 4096 entries
-// (spmv_lds_kernel).
-enum { kSpmvLds512 = 16, kSpmvLds1K = 32, kSpmvLds2K = 64, kSpmvLds4K = 128 };
-static constexpr int kSpmvVariants[] = {1, 2, 4, 8, kSpmvLds512, kSpmvLds1K, kSpmvLds2K, kSpmvLds4K};
+// Variants of the canonical spmv (all give the same bits): 1, 2, 4, 8 lanes per row, 256 rows
+// per block (spmv_kernel); 2, 4, 8 lanes per row with one row per lane group (128, 64 or 32
+// rows per block, several entries of a row in flight per lane): matrices of some thousand
+// rows then spread over all CUs instead of one 256-row block on each of a few; or LDS staging
+// with chunks of 512, 1024, 2048 or 4096 entries (spmv_lds_kernel).
+enum { kSpmvOne2 = 9, kSpmvOne4 = 10, kSpmvOne8 = 11, kSpmvLds512 = 16, kSpmvLds1K = 32, kSpmvLds2K = 64, kSpmvLds4K = 128 };
+static constexpr int kSpmvVariants[] = {1, 2, 4, 8, kSpmvOne2, kSpmvOne4, kSpmvOne8,
+                                        kSpmvLds512, kSpmvLds1K, kSpmvLds2K, kSpmvLds4K};
 static inline bool spmv_variant_ok(int v) {
     for (int w : kSpmvVariants)
         if (v == w) return true;
     return false;
 }
 
-static inline unsigned spmv_grid(int64_t n) {
-    const int64_t nb = std::max<int64_t>(1, (n + 255) / 256);
+// Matrices of up to kSpmvOneRows rows take one row per lane group, untimed: 256-row blocks
+// would leave most CUs without one and run a block's rows one after another (Taylor-Hood
+// 26^2, 5930 rows of 40 entries: 14.0 us against 4.7 us; the variants' times there differ by
+// less than the timing of two launches does). Lanes by the mean row length. 0: time them.
+constexpr int64_t kSpmvOneRows = 16384;
+static inline int spmv_small_variant(int64_t n, int64_t nnz) {
+    if (n > kSpmvOneRows) return 0;
+    return nnz <= 4 * n ? kSpmvOne2 : nnz <= 14 * n ? kSpmvOne4 : kSpmvOne8;
+}
+
+static inline unsigned spmv_grid(int64_t n, int rows) {
+    const int64_t nb = std::max<int64_t>(1, (n + rows - 1) / rows);
     return (unsigned)(((nb + 7) / 8) * 8);
 }
 
@@ -218,7 +238,10 @@ template <typename TV, typename TX, typename TY, int EPI>
 static void launch_spmv_epi(int variant, hipStream_t st, int64_t n, const int32_t *rs, const int32_t *col,
                             const TV *vals, const TX *x, TY *y, const TY *b, const TY *w, TY *out,
                             const int32_t *rsub, const int32_t *act) {
-    const dim3 g(spmv_grid(n)), t(256);
+    const dim3 g(spmv_grid(n, 256)), t(256);
+#define PYHIP_SPMV_ONE(L, NU)                                                                                 \
+    hipLaunchKernelGGL((spmv_kernel<TV, TX, TY, L, EPI, 1, NU>), dim3(spmv_grid(n, 256 / L)), t, 0, st, n, rs, col, \
+                       vals, x, y, b, w, out, rsub, act)
 #define PYHIP_SPMV_LANES(L)                                                                                   \
     hipLaunchKernelGGL((spmv_kernel<TV, TX, TY, L, EPI>), g, t, 0, st, n, rs, col, vals, x, y, b, w, out, rsub, act)
 #define PYHIP_SPMV_LDS(C)                                                                                     \
@@ -228,12 +251,16 @@ static void launch_spmv_epi(int variant, hipStream_t st, int64_t n, const int32_
     case 1: PYHIP_SPMV_LANES(1); break;
     case 2: PYHIP_SPMV_LANES(2); break;
     case 4: PYHIP_SPMV_LANES(4); break;
+    case kSpmvOne2: PYHIP_SPMV_ONE(2, 2); break;
+    case kSpmvOne4: PYHIP_SPMV_ONE(4, 4); break;
+    case kSpmvOne8: PYHIP_SPMV_ONE(8, 4); break;
     case kSpmvLds512: PYHIP_SPMV_LDS(512); break;
     case kSpmvLds1K: PYHIP_SPMV_LDS(1024); break;
     case kSpmvLds2K: PYHIP_SPMV_LDS(2048); break;
     case kSpmvLds4K: PYHIP_SPMV_LDS(4096); break;
     default: PYHIP_SPMV_LANES(8); break;
     }
+#undef PYHIP_SPMV_ONE
 #undef PYHIP_SPMV_LANES
 #undef PYHIP_SPMV_LDS
 }
