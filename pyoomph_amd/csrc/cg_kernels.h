@@ -1,15 +1,15 @@
 // Vector work of preconditioned conjugate gradients in four launches per iteration, per
 // sub-problem, on the chunks of gmres_kernels.h (256, 512 or 1024 rows of one sub-problem):
-//   cg_pq    partials of (p, q), q = A p
+//   cg_dots  partials of (p, q), q = A p
 //   cg_step  alpha = rz / (p, q);  x += alpha p, r -= alpha q [, x0 = W r]
-//   cg_rz    partials of (r, r) and (r, z), z = M^-1 r
+//   cg_dots  partials of (r, r) and (r, z), z = M^-1 r
 //   cg_dir   convergence test on (r, r), beta = rz_new / rz;  p = z + beta p
 // cg_step and cg_dir sum the partials of their sub-problem in every block (lane-strided over
 // its chunks, then an xor tree) and derive the scalars there; the sub-problem's first block
 // stores them. That replaces two reductions and two scalar launches, 1.4-3 us each, of an
 // iteration. rz alternates between two arrays, since a first block may store the new value
 // while other blocks still read the old one. Sub-problems of more than kGsFusedChunks chunks
-// get their sums from a launch of cg_reduce (same order, same bits).
+// get their sums from a launch of cg_sums (same order, same bits).
 // Bound: HBM (cg_step 5-6 vectors, cg_dir 3, the dots 2 each); launches for small systems.
 #pragma once
 #include "gmres_kernels.h"
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_dots_kernel(const T *__restrict
 }
 
 // sums[v][s] of the partials' row v (nv rows) for every sub-problem, one wave each
-__global__ __launch_bounds__(64) void cg_reduce_kernel2(int nsub, GsChunks C, const int32_t *__restrict__ active,
+__global__ __launch_bounds__(64) void cg_sums_kernel(int nsub, GsChunks C, const int32_t *__restrict__ active,
                                                         const double *__restrict__ part, double *__restrict__ sums) {
     const int v = blockIdx.x / nsub, s = blockIdx.x % nsub;
     if (active && !active[s]) return;

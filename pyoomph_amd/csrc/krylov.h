@@ -3,6 +3,7 @@
 #include <vector>
 
 #include "amg.h"
+#include "cg_kernels.h"
 #include "gmres_kernels.h"
 #include "problem.h"
 
@@ -120,7 +121,6 @@ struct KrylovWork {
     int32_t *dof_mask = nullptr;      // [nsub] Newton: 1 if the sub-problem takes a step
     int32_t *need = nullptr;          // [nsub] refinement: sub-problems still refining
     double *cg_rz = nullptr, *cg_pq = nullptr, *cg_beta = nullptr;   // [nsub]
-    int32_t *nfail_d = nullptr;       // breakdown / non-convergence counter
     // single-reduction CG (work list over active chunks)
     int32_t *achunk = nullptr;        // [nchunk] chunks of the sub-problems iterating
     int32_t *achunk_h = nullptr;      // pinned [nchunk]

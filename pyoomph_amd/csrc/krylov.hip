@@ -412,7 +412,7 @@ static int krylov_setup(pyhip_problem *p, int m) {
             (rc = kalloc(&W->jdiag64, n, W)) || (rc = kalloc(&W->jdiag32, n, W)) ||
             (rc = kalloc(&W->dof_mask, ns, W)) || (rc = kalloc(&W->need, ns, W)) ||
             (rc = kalloc(&W->cg_rz, ns, W)) || (rc = kalloc(&W->cg_pq, ns, W)) ||
-            (rc = kalloc(&W->cg_beta, ns, W)) || (rc = kalloc(&W->nfail_d, 1, W)))
+            (rc = kalloc(&W->cg_beta, ns, W)))
             return rc;
         // single-reduction CG work list
         W->sub_nnz_h.resize(ns);
@@ -1108,6 +1108,15 @@ static int precond_setup(pyhip_problem *p, KrylovWork *W, int pc, const TV *vals
     return PYHIP_OK;
 }
 
+// W->act_h = the running flags of the sub-problems, *count of them set (waits for the stream)
+static int read_active(pyhip_problem *p, KrylovWork *W, int *count) {
+    PYHIP_CHECK_HIP(hipMemcpyAsync(W->act_h, W->active, W->nsub * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
+    PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
+    *count = 0;
+    for (int s = 0; s < W->nsub; s++) *count += W->act_h[s] != 0;
+    return PYHIP_OK;
+}
+
 // GMRES in precision T on matrix values TV: x = A^{-1} b per sub-problem with need[s].
 // b, x: device vectors of type T. Returns the iterations of the longest-running one.
 template <typename T, typename TV>
@@ -1137,13 +1146,6 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     // lose sub-problems, so the host copy stays a superset (it sizes the byte counts of the
     // filtered launches; the device flags decide which rows are computed)
     int32_t *act_h = W->act_h;
-    auto read_active = [&](int *count) -> int {
-        PYHIP_CHECK_HIP(hipMemcpyAsync(act_h, W->active, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-        PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
-        *count = 0;
-        for (int s = 0; s < ns; s++) *count += act_h[s] != 0;
-        return PYHIP_OK;
-    };
     const GsChunks C = W->gs_chunks();
     const bool reduced = W->gs_max > kGsFusedChunks;
     PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gs_backsolve_kernel),
@@ -1157,7 +1159,7 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
         hipLaunchKernelGGL(gmres_start_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, d3,
                            W->bnorm, rtol, stag, cyc == 0 ? 1 : 0, need, W->g, W->active, W->kcols, W->beta0);
         KCHECK();
-        if ((rc = read_active(&nact))) return rc;
+        if ((rc = read_active(p, W, &nact))) return rc;
         if (debug_enabled()) {
             double b0 = 0, bn = 0;
             (void)hipMemcpy(&b0, W->beta0, sizeof(double), hipMemcpyDeviceToHost);
@@ -1202,7 +1204,7 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
             // cycle); in between, a sub-problem that has converged keeps its state (every
             // kernel skips it) while the others go on
             if ((k + 1) % kGmresCheck == 0 || k + 1 == mr) {
-                if ((rc = read_active(&nact))) return rc;
+                if ((rc = read_active(p, W, &nact))) return rc;
                 if (nact == 0) break;
             }
         }
@@ -1224,7 +1226,7 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     hipLaunchKernelGGL(gmres_start_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, d3, W->bnorm,
                        rtol * 1.01, 0.0, 1, need, W->g, W->active, W->kcols, W->beta0);
     KCHECK();
-    if ((rc = read_active(&nact))) return rc;
+    if ((rc = read_active(p, W, &nact))) return rc;
     // a sub-problem still marked active is above its tolerance
     W->lfail_h.assign(act_h, act_h + ns);
     *failed = nact;
@@ -1268,22 +1270,10 @@ __global__ __launch_bounds__(256) void dot2_kernel(const T *__restrict__ a, cons
     }
 }
 
-// nactive = number of sub-problems with active[s] != 0 (one block, fixed order)
-__global__ __launch_bounds__(256) void count_active_kernel(int nsub, const int32_t *__restrict__ active,
-                                                           int32_t *__restrict__ nactive) {
-    __shared__ int32_t c[256];
-    int32_t k = 0;
-    for (int s = threadIdx.x; s < nsub; s += 256) k += active[s] != 0;
-    c[threadIdx.x] = k;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if (threadIdx.x < h) c[threadIdx.x] += c[threadIdx.x + h];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *nactive = c[0];
-}
-
-constexpr int kPcgRead = 4;   // preconditioned-CG iterations between host reads of the flags
+// preconditioned-CG iterations between host reads of the flags: at least kPcgRead, an eighth
+// of the iterations done so far up to kPcgReadMax (a read leaves the GPU idle for ~10 us; the
+// iterations after the last sub-problem's stop are empty launches)
+constexpr int kPcgRead = 4, kPcgReadMax = 16;
 
 __global__ void zero_i32_kernel(int n, int32_t *__restrict__ v) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1293,82 +1283,13 @@ __global__ void zero_i32_kernel(int n, int32_t *__restrict__ v) {
 // start: bnorm = |r0|, rz = (r0, z0); active where needed and |b| > 0
 __global__ void cg_start_kernel(int nsub, const double *__restrict__ d2,
                                 const int32_t *__restrict__ need, double *__restrict__ bnorm,
-                                double *__restrict__ rz, int32_t *__restrict__ active,
-                                int32_t *__restrict__ nactive) {
+                                double *__restrict__ rz, int32_t *__restrict__ active) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nsub) return;
     bnorm[s] = sqrt(d2[s]);
     rz[s] = d2[nsub + s];
     const int a = need[s] && d2[s] > 0.0 && isfinite(d2[s]);
     active[s] = a;
-    if (a) atomicAdd(nactive, 1);
-}
-
-// alpha = rz / (p, Ap); a non-positive curvature stops the sub-problem (breakdown)
-// (also counts, per sub-problem, the iterations whose spmv visited it)
-__global__ void cg_alpha_kernel(int nsub, const double *__restrict__ pq_in, double *__restrict__ pq,
-                                int32_t *__restrict__ active, int32_t *__restrict__ nfail,
-                                int32_t *__restrict__ fail, int32_t *__restrict__ nspmv) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsub || !active[s]) return;
-    nspmv[s] += 1;
-    const double v = pq_in[s];
-    pq[s] = v;
-    if (!(v > 0.0) || !isfinite(v)) {
-        active[s] = 0;
-        fail[s] = 1;
-        atomicAdd(nfail, 1);
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void cg_xr_kernel(int64_t n, const T *__restrict__ p,
-                                                    const T *__restrict__ q, T *__restrict__ x,
-                                                    T *__restrict__ r, const double *__restrict__ rz,
-                                                    const double *__restrict__ pq,
-                                                    const int32_t *__restrict__ dsub,
-                                                    const int32_t *__restrict__ active,
-                                                    const double *__restrict__ w0, double *__restrict__ x0) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int s = dsub[i];
-    if (!active[s]) return;
-    const double a = rz[s] / pq[s];
-    x[i] = T(double(x[i]) + a * double(p[i]));
-    const T rn = T(double(r[i]) - a * double(q[i]));
-    r[i] = rn;
-    // the multigrid V-cycle's first smoothing x0 = W r of the new residual
-    if (x0) x0[i] = w0[i] * double(rn);
-}
-
-// convergence test on |r|, then beta = (r,z)_new / (r,z)_old (also counts, per
-// sub-problem, the preconditioner applies that visited it)
-__global__ void cg_check_kernel(int nsub, const double *__restrict__ d2,
-                                const double *__restrict__ bnorm, double rtol,
-                                double *__restrict__ rz, double *__restrict__ beta,
-                                int32_t *__restrict__ active, int32_t *__restrict__ nprec) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsub || !active[s]) return;
-    nprec[s] += 1;
-    const double rr = d2[s], rzn = d2[nsub + s];
-    if (!(sqrt(rr) > rtol * bnorm[s]) || !isfinite(rr)) {
-        active[s] = 0;
-        return;
-    }
-    beta[s] = rzn / rz[s];
-    rz[s] = rzn;
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void cg_p_kernel(int64_t n, const T *__restrict__ z,
-                                                   T *__restrict__ p, const double *__restrict__ beta,
-                                                   const int32_t *__restrict__ dsub,
-                                                   const int32_t *__restrict__ active) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int s = dsub[i];
-    if (!active[s]) return;
-    p[i] = T(double(z[i]) + beta[s] * double(p[i]));
 }
 
 template <typename T>
@@ -1383,16 +1304,6 @@ static int batched_dot2(pyhip_problem *p, KrylovWork *W, const T *a, const T *b,
     hipLaunchKernelGGL(reduce_partials_kernel, dim3((unsigned)(2 * W->nsub)), dim3(64), 0, p->st, 2,
                        W->nsub, W->sub_chunk_ptr, W->partial, pstride, out, 0);
     KCHECK();
-    return PYHIP_OK;
-}
-
-static int read_counter(pyhip_problem *p, KrylovWork *W, int32_t *dev, int32_t *out,
-                        const int32_t *flags = nullptr, int32_t *flags_h = nullptr) {
-    PYHIP_CHECK_HIP(hipMemcpyAsync(W->nactive_h, dev, sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-    if (flags)
-        PYHIP_CHECK_HIP(hipMemcpyAsync(flags_h, flags, W->nsub * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-    PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
-    *out = *W->nactive_h;
     return PYHIP_OK;
 }
 
@@ -1421,15 +1332,15 @@ static int cg_generic(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *
     PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
     if ((rc = precond_apply<T>(p, W, o.precond, r, z, need, act_h))) return rc;
     if ((rc = batched_dot2<T>(p, W, r, r, r, z, d2))) return rc;
-    PYHIP_CHECK_HIP(hipMemsetAsync(W->nactive_d, 0, sizeof(int32_t), p->st));
-    PYHIP_CHECK_HIP(hipMemsetAsync(W->nfail_d, 0, sizeof(int32_t), p->st));
-    PYHIP_CHECK_HIP(hipMemsetAsync(W->cg_fail, 0, ns * sizeof(int32_t), p->st));
+    hipLaunchKernelGGL(zero_i32_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, W->cg_fail);
+    // (r, z) alternates between two arrays (cg_kernels.h)
+    double *rz[2] = {W->cg_rz, W->cg_beta};
     hipLaunchKernelGGL(cg_start_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, d2, need, W->bnorm,
-                       W->cg_rz, W->active, W->nactive_d);
+                       rz[0], W->active);
     hipLaunchKernelGGL((convert_kernel<T, T>), dim3(nblk(n)), dim3(256), 0, p->st, n, z, pv);
     KCHECK();
-    int32_t nact = 0;
-    if ((rc = read_counter(p, W, W->nactive_d, &nact, W->active, act_h))) return rc;
+    int nact = 0;
+    if ((rc = read_active(p, W, &nact))) return rc;
     // with the multigrid preconditioner the x/r update also writes the V-cycle's first
     // smoothing W r of the finest level
     const double *w0 = nullptr;
@@ -1449,41 +1360,43 @@ static int cg_generic(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *
     hipLaunchKernelGGL(zero_i32_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, nprec);
     const bool defer_saved = p->timer.defer;
     p->timer.defer = true;
+    const GsChunks C = W->gs_chunks();
+    const dim3 grid((unsigned)C.count), thr(kCgThreads);
+    double *part = W->gs_part1, *sums = W->gs_max > kGsFusedChunks ? d2 : nullptr;
+    auto dots = [&](const T *a, const T *b2, const T *c, const T *d) {
+        hipLaunchKernelGGL((cg_dots_kernel<T>), grid, thr, 0, p->st, a, b2, c, d, C, W->active, part);
+        if (sums)
+            hipLaunchKernelGGL(cg_sums_kernel, dim3((unsigned)((c ? 2 : 1) * ns)), dim3(64), 0, p->st, ns, C, W->active,
+                               part, sums);
+    };
     int it = 0;
     while (nact > 0 && it < o.max_iters) {
-        const int batch = std::min(kPcgRead, o.max_iters - it);
+        const int batch = std::min(std::min(kPcgReadMax, std::max(kPcgRead, it / 8)), o.max_iters - it);
         for (int k = 0; k < batch; k++, it++) {
             if ((rc = spmv<TV, T, T>(p, vals, pv, qv, (const T *)nullptr, W->active, act_h))) return rc;
-            if ((rc = batched_dots<T>(p, W, 1, pv, n, qv, d2 + 2 * ns, W->active))) return rc;
-            hipLaunchKernelGGL(cg_alpha_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, d2 + 2 * ns,
-                               W->cg_pq, W->active, W->nfail_d, W->cg_fail, nspmv);
             {
                 TimeScope ts(&p->timer, "vector", p->st);
-                hipLaunchKernelGGL((cg_xr_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, pv, qv, x, r,
-                                   W->cg_rz, W->cg_pq, p->dof_sub, W->active, w0, x0);
+                dots(pv, qv, nullptr, nullptr);
+                hipLaunchKernelGGL((cg_step_kernel<T>), grid, thr, 0, p->st, ns, pv, qv, x, r, rz[it & 1], C, part,
+                                   sums, W->active, W->cg_fail, nspmv, w0, x0);
             }
             KCHECK();
             if ((rc = precond_apply<T>(p, W, o.precond, r, z, W->active, act_h, x0 != nullptr))) return rc;
-            if ((rc = batched_dot2<T>(p, W, r, r, r, z, d2, W->active))) return rc;
-            hipLaunchKernelGGL(cg_check_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, d2, W->bnorm, rtol,
-                               W->cg_rz, W->cg_beta, W->active, nprec);
             {
                 TimeScope ts(&p->timer, "vector", p->st);
-                hipLaunchKernelGGL((cg_p_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, z, pv, W->cg_beta,
-                                   p->dof_sub, W->active);
+                dots(r, r, r, z);
+                hipLaunchKernelGGL((cg_dir_kernel<T>), grid, thr, 0, p->st, ns, z, pv, rz[it & 1], rz[(it & 1) ^ 1], C,
+                                   part, sums, W->bnorm, rtol, W->active, nprec);
             }
             KCHECK();
         }
-        // the running count of this read: recount from the flags
-        hipLaunchKernelGGL(count_active_kernel, dim3(1), dim3(256), 0, p->st, ns, W->active, W->nactive_d);
-        if ((rc = read_counter(p, W, W->nactive_d, &nact, W->active, act_h))) return rc;
+        if ((rc = read_active(p, W, &nact))) return rc;
     }
     p->timer.defer = defer_saved;
-    int32_t nf = 0;
     PYHIP_CHECK_HIP(hipMemcpyAsync(W->flags_h, W->cg_fail, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
     PYHIP_CHECK_HIP(hipMemcpyAsync(W->flags_h + ns, nspmv, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
     PYHIP_CHECK_HIP(hipMemcpyAsync(W->flags_h + 2 * ns, nprec, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
-    if ((rc = read_counter(p, W, W->nfail_d, &nf, W->active, act_h))) return rc;
+    if ((rc = read_active(p, W, &nact))) return rc;
     if (p->timer.on) {
         // rows visited: each spmv of the loop (y = A p: matrix, row starts, p, q) and each
         // V-cycle, per sub-problem
@@ -1501,9 +1414,10 @@ static int cg_generic(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *
     // per sub-problem: broke down, or still above tolerance; iterations of the longest-
     // running sub-problem (the loop may have run a few no-op iterations past the last one)
     W->lfail_h.assign(ns, 0);
-    int maxit = 0;
+    int maxit = 0, nf = 0;
     for (int s = 0; s < ns; s++) {
         W->lfail_h[s] = (W->flags_h[s] != 0 || act_h[s] != 0) ? 1 : 0;
+        nf += W->flags_h[s] != 0;
         maxit = std::max(maxit, (int)W->flags_h[ns + s]);
     }
     *iters = maxit;
@@ -2055,7 +1969,7 @@ void pyhip_krylov_free(pyhip_problem *p) {
                     W->y, W->V, W->r64, W->x64, W->d64, W->b64, W->r32, W->d32, W->w32, W->t32,
                     W->w64, W->t64, W->vals32, W->vals64, W->res64, W->maxres, W->sub_scalar,
                     W->jdiag64, W->jdiag32, W->dof_mask, W->need, W->cg_rz, W->cg_pq,
-                    W->cg_beta, W->nfail_d, W->achunk,
+                    W->cg_beta, W->achunk,
                     W->gpart, W->cg_iters, W->cg_iters2, W->cg_fail, W->ac_cur, W->ac_der, W->ac_y, W->ac_z,
                     W->ac_t, W->ac_zs, W->ac_alpha, W->ac_mask, W->amg_conv64};
     for (void *q : ptrs)
