@@ -292,4 +292,57 @@ int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, i
     return rc;
 }
 
+int ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
+                   bool lower, IluLevelSide &out, std::string &err) {
+    out = IluLevelSide();
+    auto len = [&](int32_t r) { return lower ? H.pdiag[r] - H.prs[r] : H.prs[r + 1] - H.pdiag[r] - 1; };
+    std::vector<int32_t> R;
+    for (size_t l = 0; l + 1 < big_ptr.size(); l++) {
+        R.assign(big_rows.begin() + big_ptr[l], big_rows.begin() + big_ptr[l + 1]);
+        auto steps_of = [&](int32_t r) { return (len(r) + 7) / 8; };
+        std::stable_sort(R.begin(), R.end(), [&](int32_t a, int32_t b) { return steps_of(a) > steps_of(b); });
+        IluLevel L;
+        L.rows = (int32_t)R.size();
+        L.row0 = (int32_t)out.row.size();
+        // narrow levels: more lanes per row, for more loads in flight
+        L.lanes = L.rows <= 16384 ? 8 : L.rows <= 65536 ? 4 : 2;
+        const int ns = 8 / L.lanes;
+        for (int32_t b = 0; b < L.rows;) {
+            const int g = L.nseg++, steps = steps_of(R[b]);
+            int32_t e = b;
+            // the last segment takes every row that is left
+            while (e < L.rows && (g == kIluSegments - 1 || steps_of(R[e]) == steps)) e++;
+            L.seg_row[g] = b;
+            L.seg_row[g + 1] = e;
+            L.steps[g] = steps;
+            L.off[g] = (int64_t)out.col.size();
+            const int64_t S = (int64_t)(e - b) * L.lanes;
+            out.col.resize(out.col.size() + S * ns * steps);
+            out.src.resize(out.col.size(), -1);
+            for (int32_t q = b; q < e; q++) {
+                const int32_t r = R[q], k0 = lower ? H.prs[r] : H.pdiag[r] + 1, n = len(r);
+                const int32_t pad = n ? H.perm[H.pcol[k0]] : H.perm[r];
+                for (int k = 0; k < 8 * steps; k++) {
+                    const int st = k % 8, u = st % L.lanes, j = st / L.lanes;
+                    const int64_t at = L.off[g] + ((int64_t)(k / 8) * ns + j) * S + (int64_t)(q - b) * L.lanes + u;
+                    out.col[at] = k < n ? H.perm[H.pcol[k0 + k]] : pad;
+                    out.src[at] = k < n ? k0 + k : -1;
+                }
+            }
+            b = e;
+        }
+        for (const int32_t r : R) {
+            const bool last = lower && H.prs[r + 1] - H.pdiag[r] == 1;
+            out.row.push_back(last ? (H.perm[r] | kIluLast) : H.perm[r]);
+            out.rsrc.push_back(H.pdiag[r]);
+        }
+        out.lev.push_back(L);
+    }
+    if (out.col.size() >= (size_t)INT64_C(1) << 40) {
+        err = "ILU(0) level plan: too many entries";
+        return -1;
+    }
+    return 0;
+}
+
 }  // namespace pyhip

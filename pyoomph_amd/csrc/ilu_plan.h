@@ -71,4 +71,30 @@ constexpr int64_t kIluEntriesPerLevel = 10000;
 int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, int cap, IluSlicedPlan &out,
                     std::string &err);
 
+
+// Level-by-level solves of the other sub-problems, a launch per level, in the problem's own
+// row numbering. A level's rows are sorted by decreasing entry count and cut into segments of
+// equal step counts (a step: 8 entries of a row); `lanes` lanes take a row. Entry e of a row
+// belongs to stripe e mod 8, lane u of the row to the stripes u, u + lanes, ...: stored
+// [step][stripe / lanes][row in segment * lanes + u], so that a thread's entries come from
+// addresses it computes from the segment's numbers alone, without row pointers. Padding
+// repeats the row's first column with factor entry 0.
+constexpr int kIluSegments = 8;
+struct IluLevel {
+    int32_t rows = 0, row0 = 0, lanes = 1, nseg = 0;
+    int32_t seg_row[kIluSegments + 1] = {0};   // first row of each segment within the level
+    int32_t steps[kIluSegments] = {0};
+    int64_t off[kIluSegments] = {0};           // first entry of each segment
+};
+constexpr int32_t kIluLast = INT32_MIN;        // row mark (sign bit): no upper entries
+struct IluLevelSide {
+    std::vector<IluLevel> lev;
+    std::vector<int32_t> row, col, src, rsrc;  // problem rows (lower: | kIluLast where it applies), problem
+                                               // columns, permuted-pattern index of each entry (-1: padding)
+                                               // and of each row's pivot
+};
+// big_rows / big_ptr: the permuted rows by level (IluSlicedPlan). Returns 0 or -1 (err).
+int ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
+                   bool lower, IluLevelSide &out, std::string &err);
+
 }  // namespace pyhip

@@ -95,6 +95,38 @@ int pyhip_ilu_sliced_copy(const void *h, int nsub, const int64_t *sub_off, int c
     return 0;
 }
 
+// The level-by-level layout of one side (0 lower, 1 upper) of the sub-problems above `cap`
+// rows (ilu_level_host). sizes: [0] levels, [1] rows, [2] entries; levels [nlev][4 + 9 + 8 + 8]:
+// rows, row0, lanes, nseg, seg_row, steps, off. Null arrays are not written.
+int pyhip_ilu_level_copy(const void *h, int nsub, const int64_t *sub_off, int cap, int side, int64_t *sizes,
+                         int64_t *levels, int32_t *row, int32_t *col, int32_t *src, int32_t *rsrc) {
+    const IluHostPlan *P = (const IluHostPlan *)h;
+    if (!P || !sizes || !sub_off || nsub < 1) return -1;
+    IluSlicedPlan Q;
+    IluLevelSide S;
+    if (ilu_sliced_host(*P, std::vector<int64_t>(sub_off, sub_off + nsub + 1), cap, Q, g_ilu_err) ||
+        ilu_level_host(*P, side ? Q.big_up : Q.big_lo, side ? Q.big_up_ptr : Q.big_lo_ptr, side == 0, S, g_ilu_err))
+        return -1;
+    sizes[0] = (int64_t)S.lev.size();
+    sizes[1] = (int64_t)S.row.size();
+    sizes[2] = (int64_t)S.col.size();
+    if (levels)
+        for (const IluLevel &L : S.lev) {
+            for (int64_t v : {(int64_t)L.rows, (int64_t)L.row0, (int64_t)L.lanes, (int64_t)L.nseg}) *levels++ = v;
+            for (int32_t v : L.seg_row) *levels++ = v;
+            for (int32_t v : L.steps) *levels++ = v;
+            for (int64_t v : L.off) *levels++ = v;
+        }
+    auto cp = [](auto *dst, const auto &v) {
+        if (dst && !v.empty()) std::memcpy(dst, v.data(), v.size() * sizeof(v[0]));
+    };
+    cp(row, S.row);
+    cp(col, S.col);
+    cp(src, S.src);
+    cp(rsrc, S.rsrc);
+    return 0;
+}
+
 void pyhip_ilu_plan_free(void *h) { delete (IluHostPlan *)h; }
 
 }  // extern "C"

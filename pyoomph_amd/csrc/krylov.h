@@ -5,6 +5,7 @@
 #include "amg.h"
 #include "cg_kernels.h"
 #include "gmres_kernels.h"
+#include "ilu_plan.h"
 #include "problem.h"
 
 namespace pyhip {
@@ -28,12 +29,9 @@ struct IluPlan {
     std::vector<int64_t> lo_ptr;  // factorisation level boundaries (host)
     void *lu = nullptr;           // [nnz] factor values (T)
     int lu_prec = -1;
-    double *tmp64 = nullptr;      // [n] permuted work vectors (allocated with big rows)
-    double *tmp64b = nullptr;
-    float *tmp32 = nullptr;
-    float *tmp32b = nullptr;
-    // sub-problems solved in one workgroup each (ilu_sliced.h); big_lo / big_up with
-    // the level boundaries lo_solve / up_solve hold the rows of the others
+    void *tmp = nullptr;          // [n] (T) lower solve's result (with level-scheduled rows)
+    // sub-problems solved in one workgroup each (ilu_sliced.h); the others level by
+    // level (ilu_levels.h)
     struct Side {
         int32_t *nlev = nullptr, *chunk0 = nullptr, *src = nullptr;
         uint16_t *idx = nullptr;
@@ -45,8 +43,12 @@ struct IluPlan {
     int32_t *sdsrc = nullptr;     // [chunks * 64] pivot of each lane's row in lu (upper side)
     void *sdiag = nullptr;        // [chunks * 64] reciprocal pivots (T)
     int64_t ndiag = 0;
-    int32_t *big_lo = nullptr, *big_up = nullptr;
-    std::vector<int64_t> lo_solve, up_solve;
+    struct Levels {
+        std::vector<IluLevel> lev;
+        int32_t *row = nullptr, *col = nullptr, *src = nullptr, *rsrc = nullptr;
+        void *val = nullptr, *rdiag = nullptr;    // (T)
+        int64_t entries = 0, rows = 0;
+    } llo, lup;
 };
 
 // Block-triangular preconditioner of Taylor-Hood Jacobians [A G; D 0] (block_precond.hip):

@@ -24,6 +24,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "ilu_levels.h"
 #include "ilu_sliced.h"
 #include "krylov.h"
 #include "spmv.h"
@@ -263,45 +264,6 @@ __global__ __launch_bounds__(256) void ilu_factor_level_kernel(int64_t nrows,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     }
     if (lane == 0 && !(double(lu[di]) != 0.0 && isfinite(double(lu[di])))) err[0] = 1;
-}
-
-// One level of L y = b (unit lower) or U z = y; 16 lanes per row.
-template <typename T, bool LOWER>
-__global__ __launch_bounds__(256) void trsv_level_kernel(int64_t nrows, const int32_t *__restrict__ rows,
-                                                         const int32_t *__restrict__ rs,
-                                                         const int32_t *__restrict__ col,
-                                                         const int32_t *__restrict__ diag,
-                                                         const T *__restrict__ lu,
-                                                         const T *__restrict__ b,
-                                                         T *__restrict__ x) {
-    const int64_t w = (int64_t)blockIdx.x * 16 + threadIdx.x / 16;
-    const int lane = threadIdx.x % 16;
-    if (w >= nrows) return;
-    const int32_t i = rows[w];
-    const int32_t k0 = LOWER ? rs[i] : diag[i] + 1;
-    const int32_t k1 = LOWER ? diag[i] : rs[i + 1];
-    T acc = T(0);
-    for (int32_t k = k0 + lane; k < k1; k += 16) acc += lu[k] * x[col[k]];
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 16);
-    if (lane == 0) x[i] = LOWER ? b[i] - acc : (b[i] - acc) / lu[diag[i]];
-}
-
-// permuted[i] = original[perm[i]]
-template <typename T>
-__global__ __launch_bounds__(256) void permute_kernel(int64_t n, const int32_t *__restrict__ perm,
-                                                      const T *__restrict__ a, T *__restrict__ b) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) b[i] = a[perm[i]];
-}
-
-// original[perm[i]] = permuted[i] for the listed permuted rows i
-template <typename T>
-__global__ __launch_bounds__(256) void unpermute_rows_kernel(int64_t n, const int32_t *__restrict__ rows,
-                                                             const int32_t *__restrict__ perm,
-                                                             const T *__restrict__ a, T *__restrict__ b) {
-    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k < n) b[perm[rows[k]]] = a[rows[k]];
 }
 
 // ---- arclength continuation vector operations (per sub-problem scalars, masked) ------
@@ -606,11 +568,15 @@ constexpr int kGmresCheck = 8;   // GMRES iterations between host reads of the a
 
 static void ilu_free(KrylovWork *W) {
     IluPlan &L = W->ilu;
-    void *ptrs[] = {L.perm, L.rs, L.col, L.src, L.diag, L.lo_rows, L.lu, L.tmp64, L.tmp64b, L.tmp32, L.tmp32b,
-                    L.ssubs, L.srow0, L.srows, L.sdsrc, L.sdiag, L.big_lo, L.big_up};
+    void *ptrs[] = {L.perm, L.rs, L.col, L.src, L.diag, L.lo_rows, L.lu, L.tmp, L.ssubs, L.srow0,
+                    L.srows, L.sdsrc, L.sdiag};
     for (void *q : ptrs) dfree(q);
     for (IluPlan::Side *S : {&L.slo, &L.sup}) {
         void *sp[] = {S->nlev, S->chunk0, S->src, S->idx, S->val};
+        for (void *q : sp) dfree(q);
+    }
+    for (IluPlan::Levels *S : {&L.llo, &L.lup}) {
+        void *sp[] = {S->row, S->col, S->src, S->rsrc, S->val, S->rdiag};
         for (void *q : sp) dfree(q);
     }
     L = IluPlan();
@@ -668,8 +634,6 @@ static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
         return PYHIP_ERR_INVALID;
     }
     L.lo_ptr = H.lo_ptr;
-    L.lo_solve = Q.big_lo_ptr;
-    L.up_solve = Q.big_up_ptr;
     L.requested = W->ilu_order;
     L.multicolor = H.multicolor;
     L.nsliced = (int)Q.subs.size();
@@ -711,10 +675,23 @@ static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
         if ((rc = side(L.slo, Q.lo)) || (rc = side(L.sup, Q.up))) return rc;
     }
     if (!Q.big_lo.empty()) {
-        LUP(L.big_lo, Q.big_lo);
-        LUP(L.big_up, Q.big_up);
-        if ((rc = kalloc(&L.tmp64, n, W)) || (rc = kalloc(&L.tmp64b, n, W)) || (rc = kalloc(&L.tmp32, n, W)) ||
-            (rc = kalloc(&L.tmp32b, n, W)))
+        auto levels = [&](IluPlan::Levels &D, const std::vector<int32_t> &rows, const std::vector<int64_t> &ptr,
+                          bool lower) -> int {
+            IluLevelSide S;
+            if (ilu_level_host(H, rows, ptr, lower, S, err)) {
+                set_error(err);
+                return PYHIP_ERR_INVALID;
+            }
+            LUP(D.row, S.row);
+            LUP(D.col, S.col);
+            LUP(D.src, S.src);
+            LUP(D.rsrc, S.rsrc);
+            D.entries = (int64_t)S.col.size();
+            D.rows = (int64_t)S.row.size();
+            D.lev = std::move(S.lev);
+            return PYHIP_OK;
+        };
+        if ((rc = levels(L.llo, Q.big_lo, Q.big_lo_ptr, true)) || (rc = levels(L.lup, Q.big_up, Q.big_up_ptr, false)))
             return rc;
     }
 #undef LUP
@@ -734,7 +711,7 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
         L.lu = nullptr;
         L.lu_prec = -1;
         if ((rc = dev_alloc((T **)&L.lu, L.nnz, W->bytes))) return rc;
-        for (void **q : {&L.slo.val, &L.sup.val, &L.sdiag}) {
+        for (void **q : {&L.slo.val, &L.sup.val, &L.sdiag, &L.llo.val, &L.lup.val, &L.llo.rdiag, &L.lup.rdiag, &L.tmp}) {
             dfree(*q);
             *q = nullptr;
         }
@@ -747,6 +724,13 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
             PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ilu_sliced_apply_kernel<T>),
                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
                                                 (int)((L.max_rows + 1) * sizeof(T))));
+        }
+        if (L.llo.rows) {
+            for (IluPlan::Levels *S : {&L.llo, &L.lup})
+                if ((rc = dev_alloc((T **)&S->val, S->entries, W->bytes)) ||
+                    (rc = dev_alloc((T **)&S->rdiag, S->rows, W->bytes)))
+                    return rc;
+            if ((rc = dev_alloc((T **)&L.tmp, L.n, W->bytes))) return rc;
         }
         L.lu_prec = prec;
     }
@@ -769,6 +753,10 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
     fill(L.slo.nval, L.slo.src, L.slo.val, 0);
     fill(L.sup.nval, L.sup.src, L.sup.val, 0);
     fill(L.ndiag, L.sdsrc, L.sdiag, 1);
+    for (IluPlan::Levels *S : {&L.llo, &L.lup}) {
+        fill(S->entries, S->src, S->val, 0);
+        fill(S->rows, S->rsrc, S->rdiag, 1);
+    }
     KCHECK();
     PYHIP_CHECK_HIP(hipMemcpyAsync(W->nactive_h, W->nactive_d, sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
     PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
@@ -795,23 +783,32 @@ static int ilu_apply(pyhip_problem *p, KrylovWork *W, const T *v, T *z, const in
                            dev(L.slo, nullptr), dev(L.sup, (const T *)L.sdiag), v, z, act);
         KCHECK();
     }
-    if (!L.big_lo) return PYHIP_OK;
-    T *a = std::is_same<T, float>::value ? (T *)L.tmp32 : (T *)L.tmp64;
-    T *b = std::is_same<T, float>::value ? (T *)L.tmp32b : (T *)L.tmp64b;
-    hipLaunchKernelGGL((permute_kernel<T>), dim3(nblk(n)), dim3(256), 0, p->st, n, L.perm, v, a);
-    for (size_t l = 0; l + 1 < L.lo_solve.size(); l++) {
-        const int64_t nr = L.lo_solve[l + 1] - L.lo_solve[l];
-        hipLaunchKernelGGL((trsv_level_kernel<T, true>), dim3(nblk(nr, 16)), dim3(256), 0, p->st, nr,
-                           L.big_lo + L.lo_solve[l], L.rs, L.col, L.diag, lu, a, b);
-    }
-    for (size_t l = 0; l + 1 < L.up_solve.size(); l++) {
-        const int64_t nr = L.up_solve[l + 1] - L.up_solve[l];
-        hipLaunchKernelGGL((trsv_level_kernel<T, false>), dim3(nblk(nr, 16)), dim3(256), 0, p->st, nr,
-                           L.big_up + L.up_solve[l], L.rs, L.col, L.diag, lu, b, a);
-    }
-    // back to the problem's order, the rows of the big sub-problems only
-    const int64_t nb = L.up_solve.back();
-    hipLaunchKernelGGL((unpermute_rows_kernel<T>), dim3(nblk(nb)), dim3(256), 0, p->st, nb, L.big_up, L.perm, a, z);
+    if (!L.llo.rows) return PYHIP_OK;
+    T *y = (T *)L.tmp;
+    auto level = [&](const IluPlan::Levels &S, size_t l, bool lower, const T *x, int32_t nfirst) {
+        const IluLevel &V = S.lev[l];
+        const dim3 grid(nblk((int64_t)V.rows * V.lanes) + nblk(nfirst));
+        const T *val = (const T *)S.val, *rd = (const T *)S.rdiag;
+#define PYHIP_ILU_LEVEL(K, LOW)                                                                                 \
+    hipLaunchKernelGGL((ilu_level_kernel<T, K, LOW>), grid, dim3(256), 0, p->st, V, nfirst, S.row, S.col, val, rd, v, x, \
+                       y, z)
+        if (lower) {
+            if (V.lanes == 8) PYHIP_ILU_LEVEL(8, true);
+            else if (V.lanes == 4) PYHIP_ILU_LEVEL(4, true);
+            else PYHIP_ILU_LEVEL(2, true);
+        } else {
+            if (V.lanes == 8) PYHIP_ILU_LEVEL(8, false);
+            else if (V.lanes == 4) PYHIP_ILU_LEVEL(4, false);
+            else PYHIP_ILU_LEVEL(2, false);
+        }
+#undef PYHIP_ILU_LEVEL
+    };
+    // the first lower level with the second's launch (alone: as a level without entries), the
+    // first upper level inside the lower ones
+    if (L.llo.lev.size() == 1) level(L.llo, 0, true, v, 0);
+    for (size_t l = 1; l < L.llo.lev.size(); l++)
+        level(L.llo, l, true, l == 1 ? v : y, l == 1 ? L.llo.lev[0].rows : 0);
+    for (size_t l = 1; l < L.lup.lev.size(); l++) level(L.lup, l, false, z, 0);
     KCHECK();
     return PYHIP_OK;
 }

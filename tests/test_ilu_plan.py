@@ -315,3 +315,75 @@ def test_sliced_solve_emulated_equals_the_triangular_solves(order, cap):
                     x[r] = v
             assert np.all(seen == 1)
             assert np.allclose(x[:m], want[side][r0:r0 + m], rtol=1e-12, atol=1e-13)
+
+
+@pytest.mark.parametrize("cap", [0, 60])
+@pytest.mark.parametrize("order", [AUTO, NATURAL, MULTICOLOR])
+def test_level_solve_emulated_equals_the_triangular_solves(order, cap):
+    """The level layout of the sub-problems above the cap, walked as the level kernels walk it
+    (first lower level with the second, rows without upper entries finished by the lower
+    solve), gives z = (L U)^-1 v in the problem's own numbering."""
+    import scipy.sparse.linalg as sl
+    parts = [oracle_problem("ns", N=6), oracle_problem("bratu", N=9, space="C1", lam=1.0), oracle_problem("poisson", N=11)]
+    A, off, grp = _batch(parts)
+    P = _plan(A.indptr, A.indices, off, is_p=grp, order=order)
+    n = A.shape[0]
+    rng = np.random.default_rng(2)
+    lu = rng.uniform(-0.05, 0.05, len(P["pcol"]))
+    lu[P["pdiag"]] = rng.uniform(1.0, 2.0, n)
+    v = rng.standard_normal(n)
+    F = sp.csr_matrix((lu, P["pcol"], P["prs"]), shape=(n, n))
+    D = sp.diags(lu[P["pdiag"]])
+    want = np.empty(n)
+    w = sl.spsolve_triangular((sp.tril(F, -1) + sp.eye(n)).tocsr(), v[P["perm"]], lower=True)
+    want[P["perm"]] = sl.spsolve_triangular((sp.triu(F, 1) + D).tocsr(), w, lower=False)
+    big = np.concatenate([np.arange(off[s], off[s + 1]) for s in range(len(parts)) if off[s + 1] - off[s] > cap])
+
+    L = _lib_ilu()
+    rs, col = np.ascontiguousarray(A.indptr, np.int32), np.ascontiguousarray(A.indices, np.int32)
+    so, g = np.ascontiguousarray(off, np.int64), np.ascontiguousarray(grp, np.int8)
+    h = L.pyhip_ilu_plan_new(n, rs.ctypes.data_as(_lib.c_i32p), col.ctypes.data_as(_lib.c_i32p), len(so) - 1,
+                             so.ctypes.data_as(_lib.c_i64p), g.ctypes.data_as(ctypes.POINTER(ctypes.c_int8)), order, 64)
+    f = L.pyhip_ilu_level_copy
+    f.argtypes = [ctypes.c_void_p, ctypes.c_int, _lib.c_i64p, ctypes.c_int, ctypes.c_int, _lib.c_i64p] + \
+        [ctypes.c_void_p] * 5
+    sides = []
+    for side in (0, 1):
+        sz = np.zeros(3, np.int64)
+        head = [h, len(so) - 1, so.ctypes.data_as(_lib.c_i64p), cap, side, sz.ctypes.data_as(_lib.c_i64p)]
+        assert f(*head, *[None] * 5) == 0
+        a = (np.zeros((sz[0], 29), np.int64), np.zeros(sz[1], np.int32), np.zeros(sz[2], np.int32),
+             np.zeros(sz[2], np.int32), np.zeros(sz[1], np.int32))
+        assert f(*head, *[q.ctypes.data for q in a]) == 0
+        sides.append(a)
+    L.pyhip_ilu_plan_free(h)
+
+    def row_sums(lv, col, src, x):
+        rows, _, lanes, nseg = (int(q) for q in lv[:4])
+        seg, steps, offs = lv[4:13], lv[13:21], lv[21:29]
+        out, ns = np.zeros(rows), 8 // lanes
+        for k in range(nseg):
+            S = int(seg[k + 1] - seg[k]) * lanes
+            m = S * ns * int(steps[k])
+            c, q = col[offs[k]:offs[k] + m], src[offs[k]:offs[k] + m]
+            e = (np.where(q >= 0, lu[q], 0.0) * x[c]).reshape(-1, seg[k + 1] - seg[k], lanes)
+            out[seg[k]:seg[k + 1]] = e.sum(axis=(0, 2))
+        assert seg[0] == 0 and seg[nseg] == rows
+        return out
+
+    y, z = np.full(n, np.nan), np.full(n, np.nan)
+    levels, row, col, src, rsrc = sides[0]
+    for k, lv in enumerate(levels):
+        r = row[lv[1]:lv[1] + lv[0]]
+        i, last = r & 0x7fffffff, r < 0
+        # the second level reads v itself: its columns all lie in the first
+        s = row_sums(lv, col, src, v if k <= 1 else y)
+        y[i] = v[i] - s
+        z[i[last]] = y[i[last]] / lu[rsrc[lv[1]:lv[1] + lv[0]][last]]
+    levels, row, col, src, rsrc = sides[1]
+    assert np.all(np.isfinite(z[row[:levels[0][0]]]))   # the first upper level is already done
+    for lv in levels[1:]:
+        r = row[lv[1]:lv[1] + lv[0]]
+        z[r] = (y[r] - row_sums(lv, col, src, z)) / lu[rsrc[lv[1]:lv[1] + lv[0]]]
+    assert np.allclose(z[big], want[big], rtol=1e-12, atol=1e-13)
+    assert np.all(np.isnan(np.delete(z, big)))
