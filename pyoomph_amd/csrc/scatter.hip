@@ -22,8 +22,14 @@ constexpr int kRowLanes = 32;
 constexpr int kRowsPerBlock = 256 / kRowLanes;
 constexpr int kGatherBlock = 256;
 
-// CSR values from element matrices: the value blocks own one entry per thread; the
-// blocks after them (when res is given) own one residual row per thread.
+// CSR values from element matrices: a thread of the value blocks owns kGatherPer entries,
+// kGatherBlock apart; the blocks after them (when res is given) own one residual row per
+// thread. An entry is a chain of dependent loads (contribution bounds, index, element value)
+// of which a thread keeps kGatherPer * kGatherAhead going at a time: with one entry per thread
+// the gather waited 93 % of its cycles (192 problems, 1.05 GB read and 0.33 GB written: 483 us,
+// now 430; visiting the entries in the order of the elements did not lower the bytes and took
+// 558). Each sum keeps its list's order.
+constexpr int kGatherPer = 2, kGatherAhead = 3;
 template <typename TE, typename TV>
 __global__ __launch_bounds__(kGatherBlock) void gather_values_kernel(
     int64_t nnz, int64_t nrow, int64_t nb_vals, const int32_t *__restrict__ cptr,
@@ -36,15 +42,43 @@ __global__ __launch_bounds__(kGatherBlock) void gather_values_kernel(
     const int64_t per = (nb_vals + 7) / 8, nb_pad = 8 * per;
     if ((int64_t)blockIdx.x < nb_pad) {
         const int64_t lb = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
-        const int64_t i = lb * kGatherBlock + threadIdx.x;
-        if (lb >= nb_vals || i >= nnz) return;
-        TV acc = TV(0);
-        for (int32_t c = cptr[i]; c < cptr[i + 1]; c++) {
-            const TV v = TV(Ej[cidx[c]]);
-            // oomph skips contributions with !(fabs(v) > 0): zeros and NaN
-            if (v > TV(0) || v < TV(0)) acc = acc + v;
+        if (lb >= nb_vals) return;
+        const int64_t i0 = lb * kGatherBlock * kGatherPer + threadIdx.x;
+        int32_t c[kGatherPer], n[kGatherPer], len = 0;
+        TV acc[kGatherPer];
+#pragma unroll
+        for (int u = 0; u < kGatherPer; u++) {
+            const int64_t i = i0 + u * kGatherBlock;
+            c[u] = i < nnz ? cptr[i] : 0;
+            n[u] = i < nnz ? cptr[i + 1] - c[u] : 0;
+            acc[u] = TV(0);
         }
-        vals[i] = acc;
+#pragma unroll
+        for (int u = 0; u < kGatherPer; u++) len = max(len, n[u]);
+        for (int32_t t = 0; t < len; t += kGatherAhead) {
+            uint32_t k[kGatherPer][kGatherAhead];
+            TV v[kGatherPer][kGatherAhead];
+#pragma unroll
+            for (int u = 0; u < kGatherPer; u++)
+#pragma unroll
+                for (int a = 0; a < kGatherAhead; a++)
+                    if (t + a < n[u]) k[u][a] = cidx[c[u] + t + a];
+#pragma unroll
+            for (int u = 0; u < kGatherPer; u++)
+#pragma unroll
+                for (int a = 0; a < kGatherAhead; a++) v[u][a] = t + a < n[u] ? TV(Ej[k[u][a]]) : TV(0);
+            // oomph skips contributions with !(fabs(v) > 0): zeros and NaN
+#pragma unroll
+            for (int u = 0; u < kGatherPer; u++)
+#pragma unroll
+                for (int a = 0; a < kGatherAhead; a++)
+                    if (v[u][a] > TV(0) || v[u][a] < TV(0)) acc[u] = acc[u] + v[u][a];
+        }
+#pragma unroll
+        for (int u = 0; u < kGatherPer; u++) {
+            const int64_t i = i0 + u * kGatherBlock;
+            if (i < nnz) vals[i] = acc[u];
+        }
     } else {
         const int64_t r = ((int64_t)blockIdx.x - nb_pad) * kGatherBlock + threadIdx.x;
         if (r >= nrow) return;
@@ -208,7 +242,7 @@ static int exclusive_scan_i32(int64_t n, const int32_t *in, int32_t *totals, int
 template <typename T>
 static int launch_gather_values(const GatherMap &m, const T *Ej, const T *Er, T *vals, double *res,
                                 hipStream_t st) {
-    const int64_t nb_vals = (m.nnz + kGatherBlock - 1) / kGatherBlock;
+    const int64_t nb_vals = (m.nnz + kGatherBlock * kGatherPer - 1) / (kGatherBlock * kGatherPer);
     const int64_t nb_pad = 8 * ((nb_vals + 7) / 8);
     const int64_t nb_res = res ? (m.nrow + kGatherBlock - 1) / kGatherBlock : 0;
     if (nb_pad + nb_res == 0) return PYHIP_OK;

@@ -1,0 +1,55 @@
+"""Element kernels and the gather at the edges of their workgroups: one element, a last
+workgroup that is nearly empty, exactly full ones and the next size (128 triangles, 7 and 28
+bricks, 128 (element, node) pairs of Taylor-Hood elements, 512 matrix entries), steady and
+with the time derivative.
+
+Bar: FP64 bitwise against the oracle (1e-12 where the exponential enters, as in the parity
+tests). FP32 against FP64, relative to the largest entry: (27 + 16 N) 2^-24. A sum of at most
+27 points gives 27 * 2^-24; the rounded coordinates (2^-25 in the unit square) enter the
+tangents with shape derivatives whose absolute sum is at most 8, over tangents of length 1 / N,
+8 N * 2^-25 = 4 N * 2^-24, and the entry holds four factors of the metric (two gradients and
+the weight, of degree two)."""
+import numpy as np
+import pytest
+
+from oracle import timestepping as ots
+from tests.test_gpu_parity import build, rel
+
+pytestmark = pytest.mark.gpu
+
+SIZES = ([("bratu", dict(N=N, space=sp, lam=2.0)) for sp in ("C1", "C2") for N in (2, 8, 9, 17)] +
+         [("poisson", dict(N=N)) for N in (2, 8, 9)] +
+         [("rd", dict(N=N)) for N in (1, 2, 3, 4)] +
+         [("ns", dict(N=N)) for N in (2, 4, 15)])
+
+
+@pytest.mark.parametrize("transient", [False, True])
+@pytest.mark.parametrize("kind,kw", SIZES)
+def test_assembly_at_workgroup_edges(gpu, kind, kw, transient):
+    import torch
+    P, op = build(kind, kw)
+    if not P.ndof:
+        pytest.skip("no free value")
+    rng = np.random.default_rng(kw["N"])
+    x, h1, h2 = (rng.uniform(-0.4, 0.4, P.ndof) for _ in range(3))
+    P.set_current_dofs(x)
+    tw = ots.bdf2_weights(0.05, 0.08)
+    if transient:
+        P.set_time_state(tw, *(torch.tensor(h, dtype=torch.float64, device=P.device) for h in (h1, h2)))
+        op.set_time(tw, h1, h2)
+    r, rs, col, val = op.get_jacobian(x)
+    R, J = P.assemble_jacobian()
+    only = P.get_residuals()
+    r32, v32 = P.assemble_device("f32")
+    _, v64 = P.assemble_device("f64")
+    assert np.array_equal(J.indptr, rs) and np.array_equal(J.indices, col)
+    assert rel(J.data, val) <= 1e-12 and rel(R, r) <= 1e-12
+    if kind != "bratu":
+        assert np.array_equal(J.data, val)
+    if kind not in ("bratu", "poisson"):
+        assert np.array_equal(R, r)
+    assert np.array_equal(only, R)
+    scale = float(v64.abs().max())
+    tol = (27 + 16 * kw["N"]) * 2.0**-24
+    assert float((v32.double() - v64).abs().max()) <= tol * scale
+    assert np.max(np.abs(r32.cpu().numpy() - R)) <= tol * max(scale, np.max(np.abs(R)))
