@@ -11,7 +11,10 @@
 // (src/elements.cpp:4564-4575), field interpolation, then the test-function row and its
 // shape-function columns, skipping pinned equations (local_eqn < 0).
 //
-// Mapping (one workgroup = a block of elements, 64-wide waves):
+// Residuals and Jacobians of triangles (a thread per element)
+// have kernels of their own further down; the rest takes the general ones.
+//
+// Mapping of the general ones (one workgroup = a block of elements, 64-wide waves):
 //   thread = (element, slot row i) in phase B and (element, integration point) in
 //   phase A; EPB = 256 / max(NS, points per chunk) elements per workgroup.
 //   Per element the nodal coordinates, slot values, equations and auxiliary field are
@@ -24,6 +27,8 @@
 // Output: element vectors Er[e][i] and matrices Ej[e][i][j] in slot numbering; the
 // deterministic gather (scatter.hip) sums them into the residual and the CSR values.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 #include "element_common.h"
 
@@ -45,6 +50,8 @@ __device__ __constant__ const int8_t kTHNodeSlot[9] = {0, 3, 5, 8, 10, 12, 14, 1
 // q = t, t + NS, ... of the chunk: geometry, dx_shape of all nodes, u, grad u and the
 // source term and its derivative. Phase B: thread = test row i, accumulates its residual
 // and Jacobian row over the chunk's points in increasing point order.
+
+constexpr int kTriThreads = 128;   // elements per workgroup of tri_element_kernel
 
 // TR: the form has a time derivative (a.transient); HV: the matrix output is the
 // Hessian-vector product sum_k dJ_ij/du_k y_k = int d2src (sum_k y_k psi_k) psi_j psi_i
@@ -233,6 +240,124 @@ __global__ __launch_bounds__(256) void scalar_element_kernel(ElemArgs<T> a) {
 #pragma unroll
             for (int j = 0; j < NS; j++) dst[j] = Jacc[j];
         }
+    }
+}
+
+// Scalar forms on triangles, one thread per element: residual (JAC false) or residual and
+// Jacobian, steady or with the time derivative (TR). The element matrix (9 or 36 values), the
+// coordinates and one point's geometry fit a thread's registers, so no value is read twice
+// from LDS: with a thread per (element, row) every matrix entry of every point took its
+// gradients, shape values and equation number from LDS, and the kernel waited 68 % of its
+// time (sweep of 192 problems: P2 part 557 us, now 257, P1 part 61, now 38). Same operations in the same order per
+// output. The matrices leave through LDS (odd stride per element: no bank conflicts), as
+// contiguous 16-byte stores of the block's elements; entries of pinned rows and columns are
+// written too (nothing reads them). Bound: FP64 ALU without contraction, then the stores.
+template <typename T, int KIND, int FORM, bool TR, bool JAC>
+__global__ __launch_bounds__(kTriThreads) void tri_element_kernel(ElemArgs<T> a) {
+    using Tt = ElemTraits<KIND>;
+    constexpr int NN = Tt::NN, DIM = 2, NQ = Tt::NQ, NJ = NN * NN, ST = NJ | 1;
+    __shared__ T out[JAC ? kTriThreads * ST : 1];
+    const int eb = a.e0 + (int)blockIdx.x * kTriThreads, e = eb + (int)threadIdx.x;
+    const int el = e < a.e1 ? e : a.e1 - 1;   // the threads past the end repeat the last element
+    T X[NN][DIM], U[NN], F[FORM == PYHIP_FORM_REACTION_DIFFUSION ? NN : 1], H[TR ? NN : 1];
+#pragma unroll
+    for (int l = 0; l < NN; l++) {
+        const int node = a.conn[(int64_t)l * a.nel + el], eq = a.seqn[(int64_t)l * a.nel + el];
+#pragma unroll
+        for (int d = 0; d < DIM; d++) X[l][d] = T(a.coords[(int64_t)node * 3 + d]);
+        const double pin = a.pinned[(int64_t)node * a.nvalue];
+        U[l] = T(eq >= 0 ? a.dofs[eq] : pin);
+        if constexpr (FORM == PYHIP_FORM_REACTION_DIFFUSION) F[l] = T(a.aux[node]);
+        if constexpr (TR) {
+            const double u1 = eq >= 0 ? a.hist1[eq] : pin, u2 = eq >= 0 ? a.hist2[eq] : pin;
+            H[l] = T(a.tw1 * u1 + a.tw2 * u2);
+        }
+    }
+    const double *par = a.params + (int64_t)a.sub[el] * a.pstride;
+    const T par0 = T(par[0]), tw0 = T(a.tw0);
+    T R[NN], J[JAC ? NJ : 1];
+#pragma unroll
+    for (int i = 0; i < NN; i++) R[i] = T(0);
+#pragma unroll
+    for (int k = 0; k < (JAC ? NJ : 1); k++) J[k] = T(0);
+#pragma unroll 1
+    for (int q = 0; q < NQ; q++) {
+        const T *P = a.tab->psi + q * NN;
+        T dx[NN][DIM];
+        const T W = point_geometry<T, NN, DIM>(X, a.tab->dpsi + q * NN * DIM, a.tab->w[q], dx);
+        T u = T(0);
+#pragma unroll
+        for (int l = 0; l < NN; l++) u = u + U[l] * P[l];
+        T gu[DIM];
+#pragma unroll
+        for (int i = 0; i < DIM; i++) {
+            T sacc = T(0);
+#pragma unroll
+            for (int l = 0; l < NN; l++) sacc = sacc + U[l] * dx[l][i];
+            gu[i] = sacc;
+        }
+        T src = T(0), dsrc = T(0);
+        if constexpr (FORM == PYHIP_FORM_POISSON) {
+            T x = T(0), y = T(0);
+#pragma unroll
+            for (int l = 0; l < NN; l++) x = x + X[l][0] * P[l];
+#pragma unroll
+            for (int l = 0; l < NN; l++) y = y + X[l][1] * P[l];
+            T f = T(0);
+            const int ng = (int)par[0];  // Gaussians follow as (cx, cy, w, a)
+            for (int k = 1; k < 1 + 4 * ng; k += 4) {
+                T ddx = x - T(par[k + 0]), ddy = y - T(par[k + 1]);
+                T r2 = ddx * ddx + ddy * ddy;
+                T wk = T(par[k + 2]);
+                f = f + T(par[k + 3]) * texp(-r2 / (wk * wk));
+            }
+            src = -f;
+        } else if constexpr (FORM == PYHIP_FORM_BRATU) {
+            T ev = texp(u);
+            src = -par0 * ev;
+            dsrc = -par0 * ev;
+        } else {
+            T f = T(0);
+#pragma unroll
+            for (int l = 0; l < NN; l++) f = f + F[l] * P[l];
+            src = u * u * u - f;
+            dsrc = T(3) * (u * u);
+        }
+        T ut = T(0);
+        if constexpr (TR) {
+            T hq = T(0);
+#pragma unroll
+            for (int l = 0; l < NN; l++) hq = hq + H[l] * P[l];
+            ut = tw0 * u + hq;
+        }
+#pragma unroll
+        for (int i = 0; i < NN; i++) {
+            if constexpr (TR) R[i] = R[i] + W * ((dotv<T, DIM>(gu, dx[i]) + src * P[i]) + ut * P[i]);
+            else R[i] = R[i] + W * (dotv<T, DIM>(gu, dx[i]) + src * P[i]);
+            if constexpr (JAC) {
+#pragma unroll
+                for (int j = 0; j < NN; j++) {
+                    T inner;
+                    if constexpr (FORM == PYHIP_FORM_POISSON) inner = dotv<T, DIM>(dx[j], dx[i]);
+                    else inner = dotv<T, DIM>(dx[j], dx[i]) + (dsrc * P[j]) * P[i];
+                    const T v = TR ? W * (inner + (tw0 * P[j]) * P[i]) : W * inner;
+                    J[i * NN + j] = J[i * NN + j] + v;
+                }
+            }
+        }
+    }
+    if (e < a.e1) {
+#pragma unroll
+        for (int i = 0; i < NN; i++) a.Er[(int64_t)e * NN + i] = R[i];
+    }
+    if constexpr (JAC) {
+#pragma unroll
+        for (int k = 0; k < NJ; k++) out[threadIdx.x * ST + k] = J[k];
+        __syncthreads();
+        const int n = min(kTriThreads, a.e1 - eb) * NJ;
+        T *dst = a.Ej + (int64_t)eb * NJ;
+#pragma unroll 4
+        for (int k = threadIdx.x; k < n; k += kTriThreads) dst[k] = out[(k / NJ) * ST + k % NJ];
     }
 }
 
