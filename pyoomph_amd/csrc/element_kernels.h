@@ -11,7 +11,7 @@
 // (src/elements.cpp:4564-4575), field interpolation, then the test-function row and its
 // shape-function columns, skipping pinned equations (local_eqn < 0).
 //
-// Residuals and Jacobians of triangles (a thread per element)
+// Residuals and Jacobians of triangles (a thread per element) and bricks (nine lanes)
 // have kernels of their own further down; the rest takes the general ones.
 //
 // Mapping of the general ones (one workgroup = a block of elements, 64-wide waves):
@@ -359,6 +359,235 @@ __global__ __launch_bounds__(kTriThreads) void tri_element_kernel(ElemArgs<T> a)
 #pragma unroll 4
         for (int k = threadIdx.x; k < n; k += kTriThreads) dst[k] = out[(k / NJ) * ST + k % NJ];
     }
+}
+
+// Scalar forms on Q2 bricks: residual (JAC false) or residual and Jacobian, steady or with the
+// time derivative (TR). A wave owns seven elements and needs no workgroup barrier after the
+// reference tables are in LDS.
+// Phase A: a thread per (element, point), three rounds of 63: tangents, metric, interpolated
+// fields and source in its registers; only the dual vectors, the weight and the fields stay
+// (15 or 16 values per point in LDS), not the 81 gradients.
+// Phase B: nine lanes per element walk the points; each forms the gradients of three nodes
+// from the dual vectors (15 operations a node) and shares them through LDS, adds its three
+// residual rows and its 9 x 9 block of the matrix (rows 9 (t / 3) .., columns 9 (t % 3) ..),
+// which stays in registers: 18 nodes' gradients read per point serve 81 entries. A thread per
+// row read the gradients, shape value and equation number of every entry from LDS (four reads
+// for nine operations). FP64 takes 256 registers and so one wave per SIMD; 18 lanes with 9 x 5
+// blocks and twice the waves gave the same for the matrix and more for the residual. Same
+// operations in the same order per output. Bound: FP64 ALU without contraction (9 operations
+// per entry and point) with the LDS reads beside it. Before and now: 13824 elements FP32 with
+// the matrix 316 and 90 us; 32000 FP64 858 and 580 us, residual only 234 (shared records of an
+// even number of doubles, whose lanes meet on few banks) and 151 us.
+constexpr int kHexPerWave = 7, kHexWaves = 4, kHexPerBlock = kHexPerWave * kHexWaves;
+template <typename T, int FORM, bool TR>
+struct HexWave {   // one wave's LDS
+    // odd in FP64: an even number of doubles puts the lanes of a column on few banks
+    static constexpr int kRec = 15 + (TR ? 2 : 0), kG = sizeof(T) == 8 ? 5 : 4;
+    T rec[kHexPerWave][27][kRec];   // dual vectors [3][3], weight, src, dsrc, grad u, du/dt
+    union {
+        struct {
+            T X[kHexPerWave][27][3], U[kHexPerWave][27];
+            T F[FORM == PYHIP_FORM_REACTION_DIFFUSION ? kHexPerWave : 1][27], H[TR ? kHexPerWave : 1][27];
+        } in;
+        T g[kHexPerWave][27][kG];    // gradient of each node, and (source derivative) * shape
+    } u;
+};
+template <typename T, int FORM, bool TR>
+constexpr size_t hex_lds() {
+    return 27 * 27 * 4 * sizeof(T) + kHexWaves * sizeof(HexWave<T, FORM, TR>);
+}
+template <typename T, int FORM, bool TR, bool JAC>
+__global__ __launch_bounds__(64 * kHexWaves) void hex_element_kernel(ElemArgs<T> a) {
+    constexpr int NN = 27, DIM = 3, NQ = 27, B = 9;
+    extern __shared__ __align__(16) unsigned char hex_mem[];
+    T *tD = (T *)hex_mem, *tP = tD + NQ * NN * DIM;
+    using Wave = HexWave<T, FORM, TR>;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    Wave &M = ((Wave *)(tP + NQ * NN))[wave];
+    for (int k = threadIdx.x; k < NQ * NN * DIM; k += 64 * kHexWaves) tD[k] = a.tab->dpsi[k];
+    for (int k = threadIdx.x; k < NQ * NN; k += 64 * kHexWaves) tP[k] = a.tab->psi[k];
+    const int ew = a.e0 + (int)blockIdx.x * kHexPerBlock + wave * kHexPerWave;   // the wave's first element
+    const int ne = min(kHexPerWave, a.e1 - ew);                                     // (<= 0: none)
+    for (int k = lane; k < ne * NN; k += 64) {
+        const int le = k / NN, l = k % NN, e = ew + le;
+        const int node = a.conn[(int64_t)l * a.nel + e], eq = a.seqn[(int64_t)l * a.nel + e];
+#pragma unroll
+        for (int d = 0; d < DIM; d++) M.u.in.X[le][l][d] = T(a.coords[(int64_t)node * 3 + d]);
+        const double pin = a.pinned[(int64_t)node * a.nvalue];
+        M.u.in.U[le][l] = T(eq >= 0 ? a.dofs[eq] : pin);
+        if constexpr (FORM == PYHIP_FORM_REACTION_DIFFUSION) M.u.in.F[le][l] = T(a.aux[node]);
+        if constexpr (TR) {
+            const double u1 = eq >= 0 ? a.hist1[eq] : pin, u2 = eq >= 0 ? a.hist2[eq] : pin;
+            M.u.in.H[le][l] = T(a.tw1 * u1 + a.tw2 * u2);
+        }
+    }
+    __syncthreads();
+    auto sync = []() {   // the wave's LDS writes before its later reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    const T tw0 = T(a.tw0);
+    // ---- phase A
+#pragma unroll 1
+    for (int k = lane; k < ne * NQ; k += 63) {
+        if (lane == 63) break;
+        const int le = k / NQ, q = k % NQ;
+        const T *D = tD + q * NN * DIM, *P = tP + q * NN;
+        const T(*X)[DIM] = M.u.in.X[le];
+        T t[DIM][DIM], g[DIM][DIM];
+#pragma unroll
+        for (int i = 0; i < DIM; i++)
+#pragma unroll
+            for (int j = 0; j < DIM; j++) t[i][j] = T(0);
+#pragma unroll 3
+        for (int l = 0; l < NN; l++)
+#pragma unroll
+            for (int i = 0; i < DIM; i++)
+#pragma unroll
+                for (int j = 0; j < DIM; j++) t[j][i] = t[j][i] + X[l][i] * D[l * DIM + j];
+        T *r = M.rec[le][q];
+        const T W = metric<T, DIM>(t, a.tab->w[q], g);
+        T u = T(0), f = T(0), hq = T(0), gu[DIM] = {T(0), T(0), T(0)}, x = T(0), y = T(0);
+#pragma unroll 3
+        for (int l = 0; l < NN; l++) {
+            const T ul = M.u.in.U[le][l];
+            u = u + ul * P[l];
+#pragma unroll
+            for (int i = 0; i < DIM; i++) {
+                T s = T(0);
+#pragma unroll
+                for (int b = 0; b < DIM; b++) s = s + g[b][i] * D[l * DIM + b];
+                gu[i] = gu[i] + ul * s;
+            }
+            if constexpr (FORM == PYHIP_FORM_REACTION_DIFFUSION) f = f + M.u.in.F[le][l] * P[l];
+            if constexpr (FORM == PYHIP_FORM_POISSON) {
+                x = x + X[l][0] * P[l];
+                y = y + X[l][1] * P[l];
+            }
+            if constexpr (TR) hq = hq + M.u.in.H[le][l] * P[l];
+        }
+        const double *par = a.params + (int64_t)a.sub[ew + le] * a.pstride;
+        T src = T(0), dsrc = T(0);
+        if constexpr (FORM == PYHIP_FORM_POISSON) {
+            const int ng = (int)par[0];  // Gaussians follow as (cx, cy, w, a)
+            for (int c = 1; c < 1 + 4 * ng; c += 4) {
+                T ddx = x - T(par[c + 0]), ddy = y - T(par[c + 1]);
+                T r2 = ddx * ddx + ddy * ddy;
+                T wk = T(par[c + 2]);
+                f = f + T(par[c + 3]) * texp(-r2 / (wk * wk));
+            }
+            src = -f;
+        } else if constexpr (FORM == PYHIP_FORM_BRATU) {
+            const T par0 = T(par[0]), ev = texp(u);
+            src = -par0 * ev;
+            dsrc = -par0 * ev;
+        } else {
+            src = u * u * u - f;
+            dsrc = T(3) * (u * u);
+        }
+#pragma unroll
+        for (int b = 0; b < DIM; b++)
+#pragma unroll
+            for (int i = 0; i < DIM; i++) r[b * DIM + i] = g[b][i];
+        r[9] = W;
+        r[10] = src;
+        r[11] = dsrc;
+#pragma unroll
+        for (int i = 0; i < DIM; i++) r[12 + i] = gu[i];
+        if constexpr (TR) r[15] = tw0 * u + hq;
+    }
+    sync();
+    // ---- phase B
+    const int le = lane / B, t = lane % B, e = ew + le;
+    const bool active = le < ne && lane < B * kHexPerWave;
+    const int r0 = (t / 3) * B, c0 = (t % 3) * B;
+    T J[JAC ? B : 1][B], R[3];   // lane t's residual rows: t, t + 9, t + 18
+#pragma unroll
+    for (int i = 0; i < (JAC ? B : 1); i++)
+#pragma unroll
+        for (int j = 0; j < B; j++) J[i][j] = T(0);
+#pragma unroll
+    for (int i = 0; i < 3; i++) R[i] = T(0);
+#pragma unroll 1
+    for (int q = 0; q < NQ; q++) {
+        const T *D = tD + q * NN * DIM, *P = tP + q * NN;
+        const T *r = M.rec[active ? le : 0][q];
+        const T W = r[9];
+        if (active) {
+            T g[DIM][DIM];
+#pragma unroll
+            for (int b = 0; b < DIM; b++)
+#pragma unroll
+                for (int i = 0; i < DIM; i++) g[b][i] = r[b * DIM + i];
+            const T src = r[10], dsrc = r[11], gu[DIM] = {r[12], r[13], r[14]};
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const int l = t + k * B;
+                T dx[DIM];
+#pragma unroll
+                for (int i = 0; i < DIM; i++) {
+                    T s = T(0);
+#pragma unroll
+                    for (int b = 0; b < DIM; b++) s = s + g[b][i] * D[l * DIM + b];
+                    dx[i] = s;
+                }
+                const T p = P[l];
+                if constexpr (TR) R[k] = R[k] + W * ((dotv<T, DIM>(gu, dx) + src * p) + r[15] * p);
+                else R[k] = R[k] + W * (dotv<T, DIM>(gu, dx) + src * p);
+                if constexpr (JAC) {
+#pragma unroll
+                    for (int i = 0; i < DIM; i++) M.u.g[le][l][i] = dx[i];
+                    M.u.g[le][l][3] = dsrc * p;
+                }
+            }
+        }
+        if constexpr (JAC) {
+            sync();
+            if (active) {
+                // columns in two groups held in registers, the rows read for each
+                auto block = [&](auto first, auto count) {
+                    constexpr int J0 = decltype(first)::value, NJ = decltype(count)::value;
+                    T gj[NJ][4], tp[TR ? NJ : 1];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) {
+#pragma unroll
+                        for (int k = 0; k < 4; k++) gj[j][k] = M.u.g[le][c0 + J0 + j][k];
+                        if constexpr (TR) tp[j] = tw0 * P[c0 + J0 + j];
+                    }
+#pragma unroll
+                    for (int i = 0; i < B; i++) {
+                        const T *gi = M.u.g[le][r0 + i];
+                        const T dxi[DIM] = {gi[0], gi[1], gi[2]};
+                        const T pi = P[r0 + i];
+#pragma unroll
+                        for (int j = 0; j < NJ; j++) {
+                            T inner;
+                            if constexpr (FORM == PYHIP_FORM_POISSON) inner = dotv<T, DIM>(gj[j], dxi);
+                            else inner = dotv<T, DIM>(gj[j], dxi) + gj[j][3] * pi;
+                            T v;
+                            if constexpr (TR) v = W * (inner + tp[j] * pi);
+                            else v = W * inner;
+                            J[i][J0 + j] = J[i][J0 + j] + v;
+                        }
+                    }
+                };
+                block(std::integral_constant<int, 0>{}, std::integral_constant<int, 5>{});
+                block(std::integral_constant<int, 5>{}, std::integral_constant<int, 4>{});
+            }
+            sync();   // the next point overwrites the gradients
+        }
+    }
+    if (!active) return;
+#pragma unroll
+    for (int k = 0; k < 3; k++) a.Er[(int64_t)e * NN + t + k * B] = R[k];
+    if constexpr (JAC)
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            T *dst = a.Ej + ((int64_t)e * NN + r0 + i) * NN + c0;
+#pragma unroll
+            for (int j = 0; j < B; j++) dst[j] = J[i][j];
+        }
 }
 
 // Taylor-Hood Q2/Q1 steady Navier-Stokes (22 slots, 9 geometric nodes). Phase A: thread

@@ -25,6 +25,27 @@ static int launch_scalar(const ElemArgs<T> &a, hipStream_t s) {
             return PYHIP_OK;
         }
     }
+    if constexpr (KIND == ELEM_HEX_Q2) {
+        if (!a.hvec && !a.deriv && a.flag < 2) {
+            const dim3 g((a.e1 - a.e0 + kHexPerBlock - 1) / kHexPerBlock), t(64 * kHexWaves);
+            // most of a CU's LDS
+            auto run = [&](auto *kernel, size_t lds) -> int {
+                PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                hipLaunchKernelGGL(kernel, g, t, lds, s, a);
+                PYHIP_CHECK_HIP(hipGetLastError());
+                return PYHIP_OK;
+            };
+            if (a.transient) {
+                constexpr size_t lds = hex_lds<T, FORM, true>();
+                return a.flag ? run(&hex_element_kernel<T, FORM, true, true>, lds)
+                              : run(&hex_element_kernel<T, FORM, true, false>, lds);
+            }
+            constexpr size_t lds = hex_lds<T, FORM, false>();
+            return a.flag ? run(&hex_element_kernel<T, FORM, false, true>, lds)
+                          : run(&hex_element_kernel<T, FORM, false, false>, lds);
+        }
+    }
     if (a.hvec)
         hipLaunchKernelGGL((scalar_element_kernel<T, KIND, FORM, false, true>), dim3(blocks), dim3(256), 0, s, a);
     else if (a.transient)
