@@ -11,8 +11,9 @@
 // (src/elements.cpp:4564-4575), field interpolation, then the test-function row and its
 // shape-function columns, skipping pinned equations (local_eqn < 0).
 //
-// Residuals and Jacobians of triangles (a thread per element) and bricks (nine lanes)
-// have kernels of their own further down; the rest takes the general ones.
+// Residuals and Jacobians of triangles, bricks and Taylor-Hood elements have kernels of their
+// own further down (a thread, nine lanes, a thread per node); quadrilaterals, parameter
+// derivatives, mass matrices and Hessian products take the general ones.
 //
 // Mapping of the general ones (one workgroup = a block of elements, 64-wide waves):
 //   thread = (element, slot row i) in phase B and (element, integration point) in
@@ -588,6 +589,180 @@ __global__ __launch_bounds__(64 * kHexWaves) void hex_element_kernel(ElemArgs<T>
 #pragma unroll
             for (int j = 0; j < B; j++) dst[j] = J[i][j];
         }
+}
+
+// Taylor-Hood Navier-Stokes: residual (JAC false) or residual and Jacobian, steady or with the
+// time derivative (TR). Phase A as th_element_kernel: a thread per (element, integration
+// point). Phase B: a thread per (element, node) holds the node's two velocity rows (44 values)
+// in registers and walks the points and the nine column nodes; the four pressure rows follow.
+// A thread per slot row put the three kinds of rows side by side in a wave, which then ran
+// every kind's code for every entry, with an equation-number read and branch for each
+// (16384 elements: 176 us, now 45). Same operations in the same order per output; the entries of
+// pinned rows and columns are written too (nothing reads them). Bound: FP64 ALU without
+// contraction.
+constexpr int kThPer = 14, kThThreads = 128;   // elements and threads per workgroup (9 threads per element)
+template <typename T, bool TR, bool JAC>
+__global__ __launch_bounds__(kThThreads) void th_node_kernel(ElemArgs<T> a) {
+    constexpr int NN = 9, DIM = 2, NQ = 9, NS = 22, QV = TR ? 9 : 7;
+    constexpr int kSlot[9] = {0, 3, 5, 8, 10, 12, 14, 17, 19};   // velocity-x slot of each node
+    constexpr int kPress[4] = {2, 7, 16, 21};
+    struct El {
+        T X[NN][DIM], V[NS], H[TR ? NS : 1], W[NQ], g[NQ][NN][DIM], Q[NQ][QV];
+    };
+    __shared__ El els[kThPer];
+    __shared__ T sP[NQ][NN];
+    const int le = threadIdx.x / NN, t = threadIdx.x % NN;
+    const int e = a.e0 + (int)blockIdx.x * kThPer + le;
+    const bool active = le < kThPer && e < a.e1;
+    El &E = els[le < kThPer ? le : 0];
+    for (int k = threadIdx.x; k < NQ * NN; k += kThThreads) sP[k / NN][k % NN] = a.tab->psi[k];
+    T mu = T(0), rho = T(0);
+    if (active) {
+        const double *par = a.params + (int64_t)a.sub[e] * a.pstride;
+        mu = T(par[0]);
+        rho = T(par[1]);
+        const int node = a.conn[(int64_t)t * a.nel + e];
+        E.X[t][0] = T(a.coords[(int64_t)node * 3 + 0]);
+        E.X[t][1] = T(a.coords[(int64_t)node * 3 + 1]);
+        // corners (nodes 0, 2, 6, 8) carry the pressure after their velocities
+        const int s0 = kTHNodeSlot[t], nk = (t & 1) == 0 && t != 4 ? 3 : 2;
+        for (int k = 0; k < nk; k++) {
+            const int eq = a.seqn[(int64_t)(s0 + k) * a.nel + e];
+            const double pin = a.pinned[(int64_t)node * a.nvalue + k];
+            E.V[s0 + k] = T(eq >= 0 ? a.dofs[eq] : pin);
+            if constexpr (TR) {
+                const double u1 = eq >= 0 ? a.hist1[eq] : pin, u2 = eq >= 0 ? a.hist2[eq] : pin;
+                E.H[s0 + k] = T(a.tw1 * u1 + a.tw2 * u2);
+            }
+        }
+    }
+    __syncthreads();
+    if (active) {
+        const int q = t;
+        const T *D = a.tab->dpsi + q * NN * DIM;
+        const T *P = sP[q];
+        const T *C = a.tab->psi1 + q * 4;
+        E.W[q] = point_geometry<T, NN, DIM>(E.X, D, a.tab->w[q], E.g[q]);
+        T u0 = T(0), u1 = T(0), p = T(0);
+#pragma unroll
+        for (int l = 0; l < NN; l++) u0 = u0 + E.V[kSlot[l]] * P[l];
+#pragma unroll
+        for (int l = 0; l < NN; l++) u1 = u1 + E.V[kSlot[l] + 1] * P[l];
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            T s0 = T(0), s1 = T(0);
+#pragma unroll
+            for (int l = 0; l < NN; l++) s0 = s0 + E.V[kSlot[l]] * E.g[q][l][b];
+#pragma unroll
+            for (int l = 0; l < NN; l++) s1 = s1 + E.V[kSlot[l] + 1] * E.g[q][l][b];
+            E.Q[q][2 + b] = s0;       // du[0][b]
+            E.Q[q][4 + b] = s1;       // du[1][b]
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) p = p + E.V[kPress[k]] * C[k];
+        E.Q[q][0] = u0;
+        E.Q[q][1] = u1;
+        E.Q[q][6] = p;
+        if constexpr (TR) {
+            T h0 = T(0), h1 = T(0);
+#pragma unroll
+            for (int l = 0; l < NN; l++) h0 = h0 + E.H[kSlot[l]] * P[l];
+#pragma unroll
+            for (int l = 0; l < NN; l++) h1 = h1 + E.H[kSlot[l] + 1] * P[l];
+            E.Q[q][7] = T(a.tw0) * u0 + h0;
+            E.Q[q][8] = T(a.tw0) * u1 + h1;
+        }
+    }
+    __syncthreads();
+    if (active) {
+        T R0 = T(0), R1 = T(0), J0[JAC ? NS : 1], J1[JAC ? NS : 1];
+#pragma unroll
+        for (int j = 0; j < (JAC ? NS : 1); j++) J0[j] = J1[j] = T(0);
+#pragma unroll 1
+        for (int q = 0; q < NQ; q++) {
+            const T *P = a.tab->psi + q * NN, *C = a.tab->psi1 + q * 4;
+            const T W = E.W[q], pl = sP[q][t];
+            const T u0 = E.Q[q][0], u1 = E.Q[q][1], p = E.Q[q][6];
+            const T d00 = E.Q[q][2], d01 = E.Q[q][3], d10 = E.Q[q][4], d11 = E.Q[q][5];
+            const T l0 = E.g[q][t][0], l1 = E.g[q][t][1];
+            const T s00 = mu * (d00 + d00) - p, s01 = mu * (d01 + d10), s10 = mu * (d10 + d01), s11 = mu * (d11 + d11) - p;
+            const T c0 = rho * (u0 * d00 + u1 * d01), c1 = rho * (u0 * d10 + u1 * d11);
+            if constexpr (TR) {
+                R0 = R0 + W * (((s00 * l0 + s01 * l1) + c0 * pl) + (rho * E.Q[q][7]) * pl);
+                R1 = R1 + W * (((s10 * l0 + s11 * l1) + c1 * pl) + (rho * E.Q[q][8]) * pl);
+            } else {
+                R0 = R0 + W * ((s00 * l0 + s01 * l1) + c0 * pl);
+                R1 = R1 + W * ((s10 * l0 + s11 * l1) + c1 * pl);
+            }
+            if constexpr (JAC) {
+#pragma unroll
+                for (int n = 0; n < NN; n++) {
+                    const T x0 = E.g[q][n][0], x1 = E.g[q][n][1], ps = P[n];
+                    const T lap = x0 * l0 + x1 * l1, adv = u0 * x0 + u1 * x1;
+                    const T a00 = mu * (lap + x0 * l0) + (rho * (ps * d00 + adv)) * pl;
+                    const T a01 = mu * (x0 * l1) + (rho * (ps * d01)) * pl;
+                    const T a10 = mu * (x1 * l0) + (rho * (ps * d10)) * pl;
+                    const T a11 = mu * (lap + x1 * l1) + (rho * (ps * d11 + adv)) * pl;
+                    const int c = kSlot[n];
+                    if constexpr (TR) {
+                        const T m = ((rho * T(a.tw0)) * ps) * pl;
+                        J0[c] = J0[c] + W * (a00 + m);
+                        J1[c + 1] = J1[c + 1] + W * (a11 + m);
+                    } else {
+                        J0[c] = J0[c] + W * a00;
+                        J1[c + 1] = J1[c + 1] + W * a11;
+                    }
+                    J0[c + 1] = J0[c + 1] + W * a01;
+                    J1[c] = J1[c] + W * a10;
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    J0[kPress[k]] = J0[kPress[k]] + W * (-(C[k] * l0));
+                    J1[kPress[k]] = J1[kPress[k]] + W * (-(C[k] * l1));
+                }
+            }
+        }
+        const int64_t row = (int64_t)e * NS + kTHNodeSlot[t];
+        a.Er[row] = R0;
+        a.Er[row + 1] = R1;
+        if constexpr (JAC) {
+            T *dst = a.Ej + row * NS;
+#pragma unroll
+            for (int j = 0; j < NS; j++) dst[j] = J0[j];
+#pragma unroll
+            for (int j = 0; j < NS; j++) dst[NS + j] = J1[j];
+        }
+    }
+    // pressure rows: a thread per (element, corner)
+    const int lp = threadIdx.x / 4, k = threadIdx.x % 4, ep = a.e0 + (int)blockIdx.x * kThPer + lp;
+    if (lp >= kThPer || ep >= a.e1) return;
+    const El &F = els[lp];
+    T R = T(0), J[JAC ? NN : 1][DIM];
+#pragma unroll
+    for (int n = 0; n < (JAC ? NN : 1); n++) J[n][0] = J[n][1] = T(0);
+#pragma unroll 1
+    for (int q = 0; q < NQ; q++) {
+        const T W = F.W[q], c = a.tab->psi1[q * 4 + k];
+        R = R + W * ((F.Q[q][2] + F.Q[q][5]) * c);
+        if constexpr (JAC)
+#pragma unroll
+            for (int n = 0; n < NN; n++) {
+                J[n][0] = J[n][0] + W * (F.g[q][n][0] * c);
+                J[n][1] = J[n][1] + W * (F.g[q][n][1] * c);
+            }
+    }
+    const int64_t row = (int64_t)ep * NS + (k == 0 ? kPress[0] : k == 1 ? kPress[1] : k == 2 ? kPress[2] : kPress[3]);
+    a.Er[row] = R;
+    if constexpr (JAC) {
+        T *dst = a.Ej + row * NS;
+#pragma unroll
+        for (int n = 0; n < NN; n++) {
+            dst[kSlot[n]] = J[n][0];
+            dst[kSlot[n] + 1] = J[n][1];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) dst[kPress[j]] = T(0);
+    }
 }
 
 // Taylor-Hood Q2/Q1 steady Navier-Stokes (22 slots, 9 geometric nodes). Phase A: thread

@@ -78,6 +78,19 @@ static int launch_elements_impl(int kind, int form, const ElemArgs<T> &a, hipStr
         constexpr int EPB = 256 / 22;
         const int blocks = (a.e1 - a.e0 + EPB - 1) / EPB;
         if (blocks == 0) return PYHIP_OK;
+        if (!a.hvec && a.flag < 2) {
+            // mass matrices and Hessian products: a thread per slot row
+            const dim3 g((a.e1 - a.e0 + kThPer - 1) / kThPer), t(kThThreads);
+            if (a.transient) {
+                if (a.flag) hipLaunchKernelGGL((th_node_kernel<T, true, true>), g, t, 0, s, a);
+                else hipLaunchKernelGGL((th_node_kernel<T, true, false>), g, t, 0, s, a);
+            } else {
+                if (a.flag) hipLaunchKernelGGL((th_node_kernel<T, false, true>), g, t, 0, s, a);
+                else hipLaunchKernelGGL((th_node_kernel<T, false, false>), g, t, 0, s, a);
+            }
+            PYHIP_CHECK_HIP(hipGetLastError());
+            return PYHIP_OK;
+        }
         if (a.hvec) {
             // the product of the steady Jacobian (the time term is linear)
             hipLaunchKernelGGL((th_element_kernel<T, false, true>), dim3(blocks), dim3(256), 0, s, a);
