@@ -221,12 +221,16 @@ static inline bool spmv_variant_ok(int v) {
 
 // Matrices of up to kSpmvOneRows rows take one row per lane group, untimed: 256-row blocks
 // would leave most CUs without one and run a block's rows one after another (Taylor-Hood
-// 26^2, 5930 rows of 40 entries: 14.0 us against 4.7 us; the variants' times there differ by
-// less than the timing of two launches does). Lanes by the mean row length. 0: time them.
-constexpr int64_t kSpmvOneRows = 16384;
+// 26^2, 5930 rows of 40 entries: 14.0 us against 4.7 us; 46 000 velocity rows of 15 entries:
+// 12.8 against 5.5; FP32 aggregation level of 71 000 rows: 12.3 against 5.9), and two timed
+// launches of a few microseconds tell the variants apart so badly that the timing chose the
+// slow one of these pairs. From 131072 rows on (some 10 us and more) it finds the best within
+// a few percent. Lanes by the mean row length (51 000 rows of 45 entries: 9.3 us with 8
+// lanes, 10.7 with 4; 71 000 of 17: 7.0 and 5.9). 0: time them.
+constexpr int64_t kSpmvOneRows = 131072;
 static inline int spmv_small_variant(int64_t n, int64_t nnz) {
     if (n > kSpmvOneRows) return 0;
-    return nnz <= 4 * n ? kSpmvOne2 : nnz <= 14 * n ? kSpmvOne4 : kSpmvOne8;
+    return nnz <= 4 * n ? kSpmvOne2 : nnz <= 20 * n ? kSpmvOne4 : kSpmvOne8;
 }
 
 static inline unsigned spmv_grid(int64_t n, int rows) {
