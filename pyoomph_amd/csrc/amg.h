@@ -23,6 +23,9 @@ struct AmgDevLevel {
     int32_t *cont = nullptr;           // [nsub] 1: the sub-problem continues below this level
     int32_t *ends = nullptr;           // sub-problems solved on this level (coarsest solve)
     int nends = 0;
+    // chunks of the power iteration's norms: each one's sub-problem, each sub-problem's first
+    int32_t *csub = nullptr, *nch = nullptr;
+    int nchunks = 0;
     const double *vals = nullptr;      // A_l values (level 0: the problem's)
     double *own_vals = nullptr;        // A_l values computed here (levels > 0)
     double *d = nullptr, *w = nullptr, *pv = nullptr, *qv = nullptr, *ptv = nullptr;
@@ -50,7 +53,7 @@ struct AmgDev {
     int max_bot_rows = 0;
     std::vector<AmgDevLevel> lv;       // levels with a coarser level
     AmgDevLevel bot;                   // coarsest level
-    double *nrm = nullptr;             // [2*nsub] power-iteration norms
+    double *nrm = nullptr;             // [2 * most chunks of a level] power-iteration norms
     double *chol = nullptr;            // [nsub][kBottomMaxRows^2] coarsest-level Cholesky factors
     int32_t *chol_fail = nullptr;      // [nsub] 1 if a pivot was not positive
     float *chol32 = nullptr;           // FP32 copy of the coarsest inverses

@@ -50,59 +50,112 @@ __global__ __launch_bounds__(256) void amg_power_start_kernel(int64_t n, const i
     v[i] = ((h & 1u) ? 1.0 : -1.0) * (1.0 + (double)((h >> 8) & 7u) * 0.125);
 }
 
-// per sub-problem, with y = A v: out[2s] = (D^-1 y, D^-1 y), out[2s+1] = (v, v); one
-// block per sub-problem, strided rows then a fixed tree
+// Norms per sub-problem, with y = A v: (D^-1 y, D^-1 y), and (v, v) of the last step (VV).
+// Workgroup b takes the kNormRows rows of one chunk (nch: a sub-problem's first chunk, csub: a
+// chunk's sub-problem), a thread kNormPer of them with all its loads in flight, and writes one partial sum (a fixed tree); the readers add a
+// sub-problem's partials in order. A sub-problem's sums are thus the same alone and in a batch.
+// With one workgroup per sub-problem, one row per thread at a time, the loads' latency bound it
+// (16 us a launch for one cavity of 76^2, 30 for 192 problems, now 3 and 6).
+constexpr int kNormPer = 8, kNormRows = 256 * kNormPer;
+template <bool VV>
 __global__ __launch_bounds__(256) void amg_sub_norms_kernel(const int64_t *__restrict__ sub_off,
+                                                            const int32_t *__restrict__ nch,
+                                                            const int32_t *__restrict__ csub,
                                                             const double *__restrict__ d,
                                                             const double *__restrict__ y,
                                                             const double *__restrict__ v,
-                                                            double *__restrict__ out) {
-    __shared__ double sy[256], sv[256];
-    const int s = blockIdx.x, t = threadIdx.x;
+                                                            double *__restrict__ part) {
+    __shared__ double sy[256], sv[VV ? 256 : 1];
+    const int s = csub[blockIdx.x], t = threadIdx.x;
+    const int64_t r0 = sub_off[s] + (int64_t)((int)blockIdx.x - nch[s]) * kNormRows,
+                  r1 = min(sub_off[s + 1], r0 + kNormRows);
+    double yy[kNormPer], dd[kNormPer], vv[VV ? kNormPer : 1];
+#pragma unroll
+    for (int k = 0; k < kNormPer; k++) {
+        const int64_t i = r0 + k * 256 + t;
+        yy[k] = i < r1 ? y[i] : 0.0;
+        dd[k] = i < r1 ? d[i] : 1.0;
+        if constexpr (VV) vv[k] = i < r1 ? v[i] : 0.0;
+    }
     double ay = 0.0, av = 0.0;
-    for (int64_t i = sub_off[s] + t; i < sub_off[s + 1]; i += 256) {
-        const double yi = y[i] / d[i];
-        ay += yi * yi;
-        av += v[i] * v[i];
+#pragma unroll
+    for (int k = 0; k < kNormPer; k++) {
+        const double q = yy[k] / dd[k];
+        ay += q * q;
+        if constexpr (VV) av += vv[k] * vv[k];
     }
     sy[t] = ay;
-    sv[t] = av;
+    if constexpr (VV) sv[t] = av;
     __syncthreads();
     for (int off = 128; off > 0; off >>= 1) {
         if (t < off) {
             sy[t] += sy[t + off];
-            sv[t] += sv[t + off];
+            if constexpr (VV) sv[t] += sv[t + off];
         }
         __syncthreads();
     }
     if (t == 0) {
-        out[2 * s] = sy[0];
-        out[2 * s + 1] = sv[0];
+        double *o = part + 2 * (int64_t)blockIdx.x;
+        o[0] = sy[0];
+        if constexpr (VV) o[1] = sv[0];
     }
 }
 
-// v = D^-1 y / |D^-1 y|_s
-__global__ __launch_bounds__(256) void amg_power_scale_kernel(int64_t n, const int32_t *__restrict__ row_sub,
-                                                              const double *__restrict__ nrm,
+// sum over a sub-problem's m partials of part[2 c + which]: thread t adds c = t, t + 256, ..,
+// then a fixed tree; every thread of the workgroup gets it
+__device__ __forceinline__ double amg_sum_partials(const double *part, int m, int which, double *sh) {
+    const int t = threadIdx.x;
+    if (m <= 1) return part[which];
+    double a = 0.0;
+    for (int c = t; c < m; c += 256) a += part[2 * c + which];
+    sh[t] = a;
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1) {
+        if (t < off) sh[t] += sh[t + off];
+        __syncthreads();
+    }
+    const double r = sh[0];
+    __syncthreads();
+    return r;
+}
+
+// v = D^-1 y / |D^-1 y|_s, on the workgroups of the norms
+__global__ __launch_bounds__(256) void amg_power_scale_kernel(const int64_t *__restrict__ sub_off,
+                                                              const int32_t *__restrict__ nch,
+                                                              const int32_t *__restrict__ csub,
+                                                              const double *__restrict__ part,
                                                               const double *__restrict__ d,
                                                               const double *__restrict__ y, double *__restrict__ v) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const double yy = nrm[2 * row_sub[i]];
-    v[i] = yy > 0.0 ? (y[i] / d[i]) / sqrt(yy) : 0.0;
+    __shared__ double sh[256];
+    const int s = csub[blockIdx.x], c0 = nch[s], m = nch[s + 1] - c0;
+    const int64_t r0 = sub_off[s] + (int64_t)((int)blockIdx.x - c0) * kNormRows, r1 = min(sub_off[s + 1], r0 + kNormRows);
+    const double yy = amg_sum_partials(part + 2 * (int64_t)c0, m, 0, sh);
+    const double nr = sqrt(yy);
+#pragma unroll
+    for (int k = 0; k < kNormPer; k++) {
+        const int64_t i = r0 + k * 256 + threadIdx.x;
+        if (i < r1) v[i] = yy > 0.0 ? (y[i] / d[i]) / nr : 0.0;
+    }
 }
 
 // w_i = 4 / (3 * safety * lambda_s) / d_i, lambda_s = sqrt((y,y) / (v,v)) of the last step
-__global__ __launch_bounds__(256) void amg_weights_kernel(int64_t n, const int32_t *__restrict__ row_sub,
-                                                          const double *__restrict__ nrm,
+__global__ __launch_bounds__(256) void amg_weights_kernel(const int64_t *__restrict__ sub_off,
+                                                          const int32_t *__restrict__ nch,
+                                                          const int32_t *__restrict__ csub,
+                                                          const double *__restrict__ part,
                                                           const double *__restrict__ d, double *__restrict__ w) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int s = row_sub[i];
-    const double vv = nrm[2 * s + 1];
-    const double lam = vv > 0.0 ? sqrt(nrm[2 * s] / vv) : 1.0;
+    __shared__ double sh[256];
+    const int s = csub[blockIdx.x], c0 = nch[s], m = nch[s + 1] - c0;
+    const int64_t r0 = sub_off[s] + (int64_t)((int)blockIdx.x - c0) * kNormRows, r1 = min(sub_off[s + 1], r0 + kNormRows);
+    const double *p = part + 2 * (int64_t)c0;
+    const double yy = amg_sum_partials(p, m, 0, sh), vv = amg_sum_partials(p, m, 1, sh);
+    const double lam = vv > 0.0 ? sqrt(yy / vv) : 1.0;
     const double om = (lam > 0.0 && isfinite(lam)) ? 4.0 / (3.0 * kLambdaSafety * lam) : 0.0;
-    w[i] = (d[i] != 0.0 && isfinite(d[i])) ? om / d[i] : 0.0;
+#pragma unroll
+    for (int k = 0; k < kNormPer; k++) {
+        const int64_t i = r0 + k * 256 + threadIdx.x;
+        if (i < r1) w[i] = (d[i] != 0.0 && isfinite(d[i])) ? om / d[i] : 0.0;
+    }
 }
 
 // P[q] = [pcol(q) == agg(i)] - w_i * (sum of the A entries listed for q), i = prow(q): one
@@ -262,12 +315,18 @@ __global__ __launch_bounds__(256) void amg_wb_kernel(int64_t n, const T *__restr
 }
 
 // Dense Cholesky factor of the listed sub-problems' matrices (<= kBottomMaxRows rows),
-// one workgroup per sub-problem, right-looking, fixed order. A non-positive pivot is
-// replaced by 1 and flagged. The workgroup then writes the explicit inverse
-// X = L^-T L^-1 (thread c solves L y = e_c, L^T x = y for column c, 32 columns per pass)
-// as a symmetric matrix (entry (i, j) from the column max(i, j)), so the coarsest solve is
-// one dense symmetric product and the V-cycle stays a symmetric operator.
+// one wave per sub-problem, right-looking, fixed order. A non-positive pivot is replaced by 1
+// and flagged. The wave then writes the explicit inverse X = L^-T L^-1 (thread c solves
+// L y = e_c, L^T x = y for column c) as a symmetric matrix (entry (i, j) from the column
+// max(i, j)), so the coarsest solve is one dense symmetric product and the V-cycle stays a
+// symmetric operator.
+// A serial chain bounds it, so the loops keep independent operations going: rows are updated
+// eight columns at a time, and the solves take four rows at a time (four sums run over the
+// rows already solved, then the 4 x 4 triangle), all 64 columns at once (110 us with a
+// row at a time and 32 columns per pass, now 37).
 static_assert(kCholThreads == kBottomMaxRows, "one thread per coarsest row");
+constexpr int kCholLd = kBottomMaxRows + 1;
+constexpr size_t kCholLds = 2 * (size_t)kBottomMaxRows * kCholLd * sizeof(double);
 __global__ __launch_bounds__(kCholThreads) void amg_chol_factor_kernel(const int32_t *__restrict__ subs,
                                                                        const int64_t *__restrict__ sub_off,
                                                                        const int32_t *__restrict__ rs,
@@ -275,65 +334,94 @@ __global__ __launch_bounds__(kCholThreads) void amg_chol_factor_kernel(const int
                                                                        const double *__restrict__ vals,
                                                                        double *__restrict__ cinv,
                                                                        int32_t *__restrict__ fail) {
-    __shared__ double a[kBottomMaxRows][kBottomMaxRows + 1];
-    __shared__ double w[kBottomMaxRows][kCholThreads / 2 + 1];
+    constexpr int M = kBottomMaxRows;
+    extern __shared__ double chol_mem[];
+    double(*a)[kCholLd] = (double(*)[kCholLd])chol_mem, (*w)[kCholLd] = a + M;
     const int s = subs[blockIdx.x], t = threadIdx.x;
     const int64_t r0 = sub_off[s];
     const int m = (int)(sub_off[s + 1] - r0);
-    for (int i = t; i < kBottomMaxRows; i += kCholThreads)
-        for (int j = 0; j < kBottomMaxRows; j++) a[i][j] = 0.0;
+    // rows and columns from m on: the identity, so that whole groups can be taken
+    for (int j = 0; j < M; j++) a[j][t] = j == t && t >= m ? 1.0 : 0.0;
     __syncthreads();
-    for (int i = t; i < m; i += kCholThreads)
-        for (int32_t e = rs[r0 + i]; e < rs[r0 + i + 1]; e++) a[i][col[e] - r0] = vals[e];
+    if (t < m)
+        for (int32_t e = rs[r0 + t]; e < rs[r0 + t + 1]; e++) a[t][col[e] - r0] = vals[e];
     __syncthreads();
     for (int k = 0; k < m; k++) {
+        double pv = a[k][k];
+        const bool bad = !(pv > 0.0) || !isfinite(pv);
+        if (bad) pv = 1.0;
+        const double l = sqrt(pv);
+        __syncthreads();   // every thread has read the pivot
         if (t == 0) {
-            double pv = a[k][k];
-            if (!(pv > 0.0) || !isfinite(pv)) {
-                fail[s] = 1;
-                pv = 1.0;
-            }
-            a[k][k] = sqrt(pv);
+            if (bad) fail[s] = 1;
+            a[k][k] = l;
+        }
+        double f = 0.0;   // L(t, k)
+        if (t > k) {
+            f = a[t][k] / l;
+            a[t][k] = f;
         }
         __syncthreads();
-        for (int i = k + 1 + t; i < m; i += kCholThreads) a[i][k] = a[i][k] / a[k][k];
-        __syncthreads();
-        for (int i = k + 1 + t; i < m; i += kCholThreads)
-            for (int j = k + 1; j <= i; j++) a[i][j] = a[i][j] - a[i][k] * a[j][k];
-        __syncthreads();
-    }
-    double *X = cinv + (int64_t)s * kBottomMaxRows * kBottomMaxRows;
-    constexpr int H = kCholThreads / 2;
-    for (int c0 = 0; c0 < m; c0 += H) {
-        const int c = c0 + t;
-        if (t < H && c < m) {
-            for (int i = 0; i < m; i++) {          // L y = e_c (y_i = 0 for i < c)
-                if (i < c) {
-                    w[i][t] = 0.0;
-                    continue;
+        if (t > k) {   // columns right of the diagonal are updated too; nothing reads them
+            int j = k + 1;
+            for (; j + 8 <= m; j += 8) {
+                double u[8], v[8];
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    u[c] = a[j + c][k];
+                    v[c] = a[t][j + c];
                 }
-                double v = i == c ? 1.0 : 0.0;
-                for (int k = c; k < i; k++) v = v - a[i][k] * w[k][t];
-                w[i][t] = v / a[i][i];
+#pragma unroll
+                for (int c = 0; c < 8; c++) a[t][j + c] = v[c] - f * u[c];
             }
-            for (int i = m - 1; i >= 0; i--) {     // L^T x = y
-                double v = w[i][t];
-                for (int k = i + 1; k < m; k++) v = v - a[k][i] * w[k][t];
-                w[i][t] = v / a[i][i];
-            }
-        }
-        __syncthreads();
-        // columns c0 .. c0+H-1: entries (i, c) with i <= c, mirrored
-        for (int q = t; q < H * m; q += kCholThreads) {
-            const int cc = q / m, i = q % m, c = c0 + cc;
-            if (c < m && i <= c) {
-                const double v = w[i][cc];
-                X[i * kBottomMaxRows + c] = v;
-                X[c * kBottomMaxRows + i] = v;
-            }
+            for (; j < m; j++) a[t][j] = a[t][j] - f * a[j][k];
         }
         __syncthreads();
     }
+    // L y = e_t (y_i = 0 for i < t), rows i .. i + 3 at a time; m4: m rounded up to fours
+    const int m4 = (m + 3) & ~3;
+    for (int i = 0; i < m4; i += 4) {
+        double v[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = i + r == t ? 1.0 : 0.0;
+#pragma unroll 4
+        for (int k = 0; k < i; k++) {
+            const double wk = w[k][t];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = v[r] - a[i + r][k] * wk;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+#pragma unroll
+            for (int q = 0; q < r; q++) v[r] = v[r] - a[i + r][i + q] * v[q];
+            v[r] = v[r] / a[i + r][i + r];
+            w[i + r][t] = v[r];
+        }
+    }
+    // L^T x = y
+    for (int i = m4 - 4; i >= 0; i -= 4) {
+        double v[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = w[i + r][t];
+#pragma unroll 4
+        for (int k = i + 4; k < m4; k++) {
+            const double wk = w[k][t];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = v[r] - a[k][i + r] * wk;
+        }
+#pragma unroll
+        for (int r = 3; r >= 0; r--) {
+#pragma unroll
+            for (int q = r + 1; q < 4; q++) v[r] = v[r] - a[i + q][i + r] * v[q];
+            v[r] = v[r] / a[i + r][i + r];
+            w[i + r][t] = v[r];
+        }
+    }
+    __syncthreads();
+    // entries (i, c) with i <= c, mirrored
+    double *X = cinv + (int64_t)s * M * M;
+    if (t < m)
+        for (int i = 0; i < m; i++) X[i * M + t] = i <= t ? w[i][t] : w[t][i];
 }
 
 // Non-symmetric coarsest matrices: in-place Gauss-Jordan inverse without pivoting (the
@@ -435,7 +523,7 @@ void amg_free(AmgDev &A) {
         void *ptrs[] = {L.rs, L.col, L.diag, L.agg, L.pfix, L.prs, L.pcol, L.pcptr, L.pcidx, L.trs, L.trow, L.tsrc,
                         L.qrs, L.qcol, L.row_sub, L.sub_off, L.own_vals, L.d, L.w, L.pv, L.qv, L.b, L.x,
                         L.x2, L.r, L.pw, L.py, L.cont, L.ends, L.ptv, L.prow, L.tinv, L.own_vals32, L.w32,
-                        L.pv32, L.ptv32, L.b32, L.x32, L.x2_32, L.r32};
+                        L.pv32, L.ptv32, L.b32, L.x32, L.x2_32, L.r32, L.csub, L.nch};
         for (void *q : ptrs) dfree(q);
         L = AmgDevLevel();
     };
@@ -465,6 +553,13 @@ static int upload_level(AmgDevLevel &D, const std::vector<int32_t> &rs, const st
         D.h_rows[s] = sub_off[s + 1] - sub_off[s];
         D.h_nnz[s] = (int64_t)rs[sub_off[s + 1]] - rs[sub_off[s]];
     }
+    std::vector<int32_t> csub, nch(ns + 1, 0);
+    for (size_t s = 0; s < ns; s++) {
+        for (int64_t r = 0; r < D.h_rows[s]; r += kNormRows) csub.push_back((int32_t)s);
+        nch[s + 1] = (int32_t)csub.size();
+    }
+    D.nchunks = (int)csub.size();
+    if ((rc = aup(&D.csub, csub, B)) || (rc = aup(&D.nch, nch, B))) return rc;
     if (own_vals && (rc = dev_alloc(&D.own_vals, D.nnz, B))) return rc;
     if ((rc = dev_alloc(&D.d, D.n, B)) || (rc = dev_alloc(&D.w, D.n, B)) || (rc = dev_alloc(&D.b, D.n, B)) ||
         (rc = dev_alloc(&D.x, D.n, B)) || (rc = dev_alloc(&D.x2, D.n, B)) || (rc = dev_alloc(&D.r, D.n, B)) ||
@@ -519,7 +614,9 @@ int amg_build(AmgDev &A, int64_t n, const int32_t *rs_h, const int32_t *col_h, c
         return rc;
     A.bot.nends = (int)plan.bot_subs.size();
     if ((rc = aup(&A.bot.ends, plan.bot_subs, B))) return rc;
-    if ((rc = dev_alloc(&A.nrm, 2 * std::max(1, A.nsub), B)) ||
+    int nch = 1;
+    for (const AmgDevLevel &L : A.lv) nch = std::max(nch, L.nchunks);
+    if ((rc = dev_alloc(&A.nrm, 2 * (size_t)nch, B)) ||
         (rc = dev_alloc(&A.chol, (size_t)std::max(1, A.nsub) * kBottomMaxRows * kBottomMaxRows, B)) ||
         (rc = dev_alloc(&A.chol_fail, std::max(1, A.nsub), B)))
         return rc;
@@ -631,20 +728,39 @@ static int tune_levels(AmgDev &A, hipStream_t st) {
     return PYHIP_OK;
 }
 
-static int level_weights(hipStream_t st, AmgDevLevel &L, const double *vals, double *nrm, int nsub,
+static int level_weights(hipStream_t st, AmgDevLevel &L, const double *vals, double *nrm,
                          KernelTimer *tm) {
     const int64_t n = L.n;
+    if (n == 0) return PYHIP_OK;
     const int lpr = L.lpr_a ? L.lpr_a : lanes_for(L.nnz, n);
     hipLaunchKernelGGL(amg_diag_kernel, dim3(ablk(n)), dim3(256), 0, st, n, L.diag, vals, L.d);
     hipLaunchKernelGGL(amg_power_start_kernel, dim3(ablk(n)), dim3(256), 0, st, n, L.row_sub, L.sub_off, L.pw);
+    const dim3 g((unsigned)L.nchunks), t(256);
     for (int it = 0; it < kPowerIters; it++) {
         level_spmv<double>(tm, kSpmvPlain, lpr, st, n, L.nnz, n, n, L.rs, L.col, vals, L.pw, L.py, nullptr);
-        hipLaunchKernelGGL(amg_sub_norms_kernel, dim3(nsub), dim3(256), 0, st, L.sub_off, L.d, L.py, L.pw, nrm);
-        if (it + 1 < kPowerIters)
-            hipLaunchKernelGGL(amg_power_scale_kernel, dim3(ablk(n)), dim3(256), 0, st, n, L.row_sub, nrm, L.d, L.py,
-                               L.pw);
+        if (it + 1 < kPowerIters) {
+            hipLaunchKernelGGL((amg_sub_norms_kernel<false>), g, t, 0, st, L.sub_off, L.nch, L.csub, L.d, L.py, L.pw, nrm);
+            hipLaunchKernelGGL(amg_power_scale_kernel, g, t, 0, st, L.sub_off, L.nch, L.csub, nrm, L.d, L.py, L.pw);
+        } else {
+            hipLaunchKernelGGL((amg_sub_norms_kernel<true>), g, t, 0, st, L.sub_off, L.nch, L.csub, L.d, L.py, L.pw, nrm);
+        }
     }
-    hipLaunchKernelGGL(amg_weights_kernel, dim3(ablk(n)), dim3(256), 0, st, n, L.row_sub, nrm, L.d, L.w);
+    hipLaunchKernelGGL(amg_weights_kernel, g, t, 0, st, L.sub_off, L.nch, L.csub, nrm, L.d, L.w);
+    ACHECK();
+    return PYHIP_OK;
+}
+
+// inverses of the sub-problems whose coarsest level L is
+static int launch_inverse(AmgDev &A, hipStream_t st, const AmgDevLevel &L, const double *vals) {
+    if (A.nonsym) {
+        hipLaunchKernelGGL(amg_gj_inverse_kernel, dim3(L.nends), dim3(kCholThreads), 0, st, L.ends, L.sub_off, L.rs,
+                           L.col, vals, A.chol, A.chol_fail);
+    } else {
+        PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(amg_chol_factor_kernel),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCholLds));
+        hipLaunchKernelGGL(amg_chol_factor_kernel, dim3(L.nends), dim3(kCholThreads), kCholLds, st, L.ends, L.sub_off,
+                           L.rs, L.col, vals, A.chol, A.chol_fail);
+    }
     ACHECK();
     return PYHIP_OK;
 }
@@ -661,10 +777,9 @@ int amg_setup(AmgDev &A, hipStream_t st, const double *vals0, KernelTimer *tm, c
         AmgDevLevel &L = A.lv[l];
         if (l > 0) vals = L.own_vals;
         L.vals = vals;
-        if ((rc = level_weights(st, L, vals, A.nrm, A.nsub, tm))) return rc;
+        if ((rc = level_weights(st, L, vals, A.nrm, tm))) return rc;
         if (L.nends)
-            hipLaunchKernelGGL(A.nonsym ? amg_gj_inverse_kernel : amg_chol_factor_kernel, dim3(L.nends),
-                               dim3(kCholThreads), 0, st, L.ends, L.sub_off, L.rs, L.col, vals, A.chol, A.chol_fail);
+            if ((rc = launch_inverse(A, st, L, vals))) return rc;
         if (L.nnzp > 0)
             hipLaunchKernelGGL(amg_pvals_kernel, dim3(ablk(L.nnzp)), dim3(256), 0, st, L.nnzp, L.prow,
                                L.pcptr, L.pcidx, L.pfix, vals, L.w, L.tinv, L.pv, L.ptv);
@@ -680,9 +795,7 @@ int amg_setup(AmgDev &A, hipStream_t st, const double *vals0, KernelTimer *tm, c
     }
     A.bot.vals = A.lv.empty() ? vals0 : A.bot.own_vals;
     if (A.bot.nends)
-        hipLaunchKernelGGL(A.nonsym ? amg_gj_inverse_kernel : amg_chol_factor_kernel, dim3(A.bot.nends),
-                           dim3(kCholThreads), 0, st, A.bot.ends, A.bot.sub_off, A.bot.rs, A.bot.col, A.bot.vals,
-                           A.chol, A.chol_fail);
+        if ((rc = launch_inverse(A, st, A.bot, A.bot.vals))) return rc;
     ACHECK();
     // A coarsest matrix that is not positive definite (an indefinite Jacobian, e.g. past a
     // fold) makes the V-cycle an invalid preconditioner: report it instead of iterating on.
