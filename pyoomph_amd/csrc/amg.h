@@ -53,6 +53,8 @@ struct AmgDev {
     int max_bot_rows = 0;
     std::vector<AmgDevLevel> lv;       // levels with a coarser level
     AmgDevLevel bot;                   // coarsest level
+    int tail = 0;                      // first level of the cycle's one-workgroup part (lv.size(): none)
+    size_t tail_len = 0;               // its LDS, in vector entries
     double *nrm = nullptr;             // [2 * most chunks of a level] power-iteration norms
     double *chol = nullptr;            // [nsub][kBottomMaxRows^2] coarsest-level Cholesky factors
     int32_t *chol_fail = nullptr;      // [nsub] 1 if a pivot was not positive

@@ -302,6 +302,8 @@ static void launch_rowprod(double mean_src, hipStream_t st, int64_t nout, const 
 
 // ---- V-cycle kernels -----------------------------------------------------------------------
 
+#include "amg_tail.h"
+
 // x = W b
 // (rows of sub-problems with act[row_sub] == 0 are skipped when act is given)
 template <typename T>
@@ -568,6 +570,7 @@ static int upload_level(AmgDevLevel &D, const std::vector<int32_t> &rs, const st
     return PYHIP_OK;
 }
 
+static void amg_tail_level(AmgDev &A);
 int amg_build(AmgDev &A, int64_t n, const int32_t *rs_h, const int32_t *col_h, const std::vector<int64_t> &sub_off,
               int64_t &B, const AmgFixedInterp *fix) {
     if (A.built) return PYHIP_OK;
@@ -621,6 +624,7 @@ int amg_build(AmgDev &A, int64_t n, const int32_t *rs_h, const int32_t *col_h, c
         (rc = dev_alloc(&A.chol_fail, std::max(1, A.nsub), B)))
         return rc;
     A.max_bot_rows = plan.max_bot_rows;
+    amg_tail_level(A);
     A.built = true;
     return PYHIP_OK;
 }
@@ -713,7 +717,7 @@ static int tune_levels(AmgDev &A, hipStream_t st) {
         L.lpr_a = pick(L.n, L.nnz, [&](int lpr) {
             launch_spmv<double, double, double>(lpr, st, L.n, L.rs, L.col, L.vals, L.b, L.r, nullptr);
         });
-        if (L.nc) {
+        if (L.nc && (int)l < A.tail) {
             L.lpr_t = pick(L.nc, L.nnzp, [&](int lpr) {
                 launch_spmv<double, double, double>(lpr, st, L.nc, L.trs, L.trow, L.ptv, L.r, C.b, nullptr);
             });
@@ -851,6 +855,32 @@ template <> struct AmgView<float> {
     static const float *chol(const AmgDev &A) { return A.chol32; }
 };
 
+// First level of the part that one workgroup per sub-problem runs (lv.size(): none): the first
+// one on which no sub-problem has more than kTailNnz entries, its vectors fit 64 KB of LDS in
+// FP64 and at most kTailLevels levels follow. A workgroup reads some 75 GB/s here, so a pass
+// over 16384 entries of 12 bytes takes the 3 to 4 us that its launch would; limits of 8192 and
+// 32768 chose the same levels for sub-problems of 2000 to 60 000 rows (a level has five to ten
+// times the entries of the next).
+constexpr int64_t kTailNnz = 16384;
+static void amg_tail_level(AmgDev &A) {
+    const int nl = (int)A.lv.size();
+    A.tail = nl;
+    std::vector<int64_t> len(A.nsub, 0);   // per sub-problem: entries of b and x of the levels from l on
+    for (int s = 0; s < A.nsub; s++) len[s] = 2 * A.bot.h_rows[s];
+    for (int l = nl - 1; l >= 0 && nl - l <= kTailLevels; l--) {
+        const AmgDevLevel &L = A.lv[l];
+        int64_t most = 0, nnz = 0;
+        for (int s = 0; s < A.nsub; s++) {
+            len[s] += 2 * L.h_rows[s];
+            most = std::max(most, len[s] + L.h_rows[s]);
+            nnz = std::max(nnz, L.h_nnz[s]);
+        }
+        if (nnz > kTailNnz || most * (int64_t)sizeof(double) > 65536) return;
+        A.tail = l;
+        A.tail_len = (size_t)most;
+    }
+}
+
 // z = M^-1 b (both [n0]) in precision T
 template <typename T>
 static int amg_apply_t(AmgDev &A, hipStream_t st, const T *b, T *z, KernelTimer *tm, const int32_t *act,
@@ -867,7 +897,7 @@ static int amg_apply_t(AmgDev &A, hipStream_t st, const T *b, T *z, KernelTimer 
     }
     // visited rows, entries and P entries per level (all sub-problems without a filter)
     std::vector<int64_t> rows(nl + 1), nnz(nl), nnzp(nl);
-    for (int l = 0; l < nl; l++) {
+    for (int l = 0; l < nl && l <= A.tail; l++) {
         rows[l] = act ? active_sum(A.lv[l].h_rows, act_h) : A.lv[l].n;
         nnz[l] = act ? active_sum(A.lv[l].h_nnz, act_h) : A.lv[l].nnz;
         nnzp[l] = act ? active_sum(A.lv[l].h_nnzp, act_h) : A.lv[l].nnzp;
@@ -876,7 +906,7 @@ static int amg_apply_t(AmgDev &A, hipStream_t st, const T *b, T *z, KernelTimer 
     // down: level l works on right-hand side bl (level 0: b). The rows of sub-problems that
     // end on level l are computed too (their couplings stay in their sub-problem) and are
     // then overwritten by their coarsest solve.
-    for (int l = 0; l < nl; l++) {
+    for (int l = 0; l < A.tail; l++) {
         AmgDevLevel &L = A.lv[l];
         const T *bl = l == 0 ? b : V::b(L);
         AmgDevLevel &C = (l + 1 < nl) ? A.lv[l + 1] : A.bot;
@@ -887,20 +917,33 @@ static int amg_apply_t(AmgDev &A, hipStream_t st, const T *b, T *z, KernelTimer 
         const int la = L.lpr_a ? L.lpr_a : lanes_for(L.nnz, L.n);
         level_spmv<T>(tm, kSpmvSub, la, st, L.n, nnz[l], rows[l], rows[l], L.rs, L.col, V::vals(L), V::x(L),
                       V::r(L), bl, L.row_sub, act);
-        // b_c = P^T r, and x_c = W_c b_c where the coarse level is not the coarsest
-        if (L.nc && l + 1 < nl)
+        // b_c = P^T r, and x_c = W_c b_c where launches smooth the coarse level
+        if (L.nc && l + 1 < A.tail)
             level_spmv<T>(tm, kSpmvScale, L.lpr_t ? L.lpr_t : 8, st, L.nc, nnzp[l], rows[l + 1], rows[l], L.trs,
                           L.trow, V::ptv(L), V::r(L), V::b(C), nullptr, C.row_sub, act, V::w(C), V::x(C));
         else if (L.nc)
             level_spmv<T>(tm, kSpmvPlain, L.lpr_t ? L.lpr_t : 8, st, L.nc, nnzp[l], rows[l + 1], rows[l], L.trs,
                           L.trow, V::ptv(L), V::r(L), V::b(C), nullptr, C.row_sub, act);
     }
-    if (Bt.nends)
+    if (A.tail < nl) {
+        AmgTail<T> R = {};
+        R.nl = nl - A.tail;
+        for (int l = A.tail; l < nl; l++) {
+            AmgDevLevel &L = A.lv[l];
+            R.lv[l - A.tail] = {L.rs,   L.col,      L.trs,   L.trow,    L.prs,    L.pcol,
+                                L.cont, V::vals(L), V::w(L), V::ptv(L), V::pv(L), L.sub_off};
+        }
+        R.lv[R.nl].sub_off = Bt.sub_off;
+        AmgDevLevel &F = A.lv[A.tail];
+        hipLaunchKernelGGL((amg_tail_kernel<T>), dim3(A.nsub), dim3(kTailThreads), A.tail_len * sizeof(T), st, R,
+                           V::chol(A), A.tail == 0 ? b : V::b(F), A.tail == 0 ? z : V::x(F), act);
+    } else if (Bt.nends) {
         hipLaunchKernelGGL((amg_chol_solve_kernel<T>), dim3(Bt.nends), dim3(kCholThreads), 0, st, Bt.ends,
                            Bt.sub_off, V::chol(A), V::b(Bt), V::x(Bt), act);
+    }
     // up: coarse correction and post-sweep; sub-problems ending on a level get their
     // coarsest solve there
-    for (int l = nl - 1; l >= 0; l--) {
+    for (int l = A.tail - 1; l >= 0; l--) {
         AmgDevLevel &L = A.lv[l];
         const T *bl = l == 0 ? b : V::b(L);
         AmgDevLevel &C = (l + 1 < nl) ? A.lv[l + 1] : A.bot;
@@ -921,19 +964,19 @@ static int amg_apply_t(AmgDev &A, hipStream_t st, const T *b, T *z, KernelTimer 
 }
 
 // Row-dependent spmv-family bytes one V-cycle moves for each sub-problem (the terms
-// level_spmv counts, less the 4 bytes per launch), element size esize.
+// level_spmv counts, less the 4 bytes per launch), element size esize; the one-workgroup part
+// is no spmv launch.
 std::vector<int64_t> amg_vcycle_bytes(const AmgDev &A, int esize) {
     std::vector<int64_t> out(std::max(0, A.nsub), 0);
-    const int nl = (int)A.lv.size();
     const int64_t E = esize;
     for (int s = 0; s < A.nsub; s++) {
         int64_t b = 0;
-        for (int l = 0; l < nl; l++) {
+        for (int l = 0; l < A.tail; l++) {
             const AmgDevLevel &L = A.lv[l];
-            const AmgDevLevel &C = (l + 1 < nl) ? A.lv[l + 1] : A.bot;
+            const AmgDevLevel &C = (l + 1 < (int)A.lv.size()) ? A.lv[l + 1] : A.bot;
             const int64_t r = L.h_rows[s], z = L.h_nnz[s], zp = L.h_nnzp[s], rc = C.h_rows[s];
             b += (E + 4) * z + 4 * r + E * r + 2 * E * r;             // r = b - A x
-            if (L.nc) b += (E + 4) * zp + 4 * rc + E * r + (l + 1 < nl ? 3 : 1) * E * rc;   // restriction
+            if (L.nc) b += (E + 4) * zp + 4 * rc + E * r + (l + 1 < A.tail ? 3 : 1) * E * rc;   // restriction
             if (L.nc) b += (E + 4) * zp + 4 * r + E * rc + 2 * E * r; // prolongation x += P x_c
             b += (E + 4) * z + 4 * r + E * r + 4 * E * r;             // post-sweep
         }
