@@ -202,8 +202,12 @@ __device__ __forceinline__ int32_t find_col(const int32_t *__restrict__ cols, in
 // order, the lanes spreading over the source row's entries, each finding its column in
 // the output row by binary search in LDS and adding its product with a fused multiply-add
 // (a source row has distinct columns, so no two lanes touch one sum in a step). A sum thus
-// receives its terms in increasing t whatever G, alone or in a batch. Output rows longer
-// than CAPR take the same sums entry by entry (binary search in the source rows).
+// receives its terms in increasing t whatever G, alone or in a batch. The loads and searches of
+// kProdAhead terms go together; one at a time, a term's two dependent loads and its search
+// were the time (192 P2 problems: A P 509 us, now 419, P^T Q 214, now 161; eight terms: 608 and
+// 153). Bound: the searches' LDS reads. Output rows longer than CAPR take the same sums
+// entry by entry (binary search in the source rows).
+constexpr int kProdAhead = 4;
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -247,6 +251,7 @@ __global__ __launch_bounds__(256) void amg_rowprod_kernel(int64_t nout, const in
         ma[k] = 0.0;
     }
     wave_lds_sync();
+    const int32_t top = R > 0 ? 1 << (31 - __builtin_clz(R)) : 0;   // largest power of two <= R
     for (int32_t tb = t0; tb < t1; tb += G) {
         const int32_t t = tb + lane;
         int32_t sb = 0, se = 0;
@@ -258,20 +263,38 @@ __global__ __launch_bounds__(256) void amg_rowprod_kernel(int64_t nout, const in
             se = srs[r + 1];
         }
         const int nt = min(G, t1 - tb);
-        for (int u = 0; u < nt; u++) {
-            const double p = __shfl(tv, u, G);
-            const int32_t b = __shfl(sb, u, G), e = __shfl(se, u, G);
-            for (int32_t x = b + lane; x < e; x += G) {
-                const int32_t J = scol[x];
-                int32_t lo = 0, hi = R;
-                while (lo < hi) {
-                    const int32_t m = (lo + hi) >> 1;
-                    if (mc[m] < J) lo = m + 1;
-                    else hi = m;
-                }
-                if (lo < R && mc[lo] == J) ma[lo] = __builtin_fma(p, sval[x], ma[lo]);
+        for (int u0 = 0; u0 < nt; u0 += kProdAhead) {
+            double p[kProdAhead], sv[kProdAhead];
+            int32_t x[kProdAhead], e[kProdAhead], J[kProdAhead], at[kProdAhead];
+#pragma unroll
+            for (int a = 0; a < kProdAhead; a++) {
+                const int u = min(u0 + a, G - 1);
+                p[a] = __shfl(tv, u, G);
+                x[a] = __shfl(sb, u, G) + lane;
+                e[a] = __shfl(se, u, G);
+                if (u0 + a >= nt) e[a] = 0;
+                const bool in = x[a] < e[a];
+                J[a] = in ? scol[x[a]] : -1;
+                sv[a] = in ? sval[x[a]] : 0.0;
+                at[a] = 0;
             }
-            wave_lds_sync();
+            // first place not below J (J = -1: 0, which it does not match)
+            for (int32_t h = top; h > 0; h >>= 1)
+#pragma unroll
+                for (int a = 0; a < kProdAhead; a++)
+                    if (at[a] + h <= R && mc[at[a] + h - 1] < J[a]) at[a] += h;
+#pragma unroll
+            for (int a = 0; a < kProdAhead; a++) {
+                if (at[a] < R && mc[at[a]] == J[a]) ma[at[a]] = __builtin_fma(p[a], sv[a], ma[at[a]]);
+                for (int32_t y = x[a] + G; y < e[a]; y += G) {   // source rows of more than G entries
+                    const int32_t K = scol[y];
+                    int32_t lo = 0;
+                    for (int32_t h = top; h > 0; h >>= 1)
+                        if (lo + h <= R && mc[lo + h - 1] < K) lo += h;
+                    if (lo < R && mc[lo] == K) ma[lo] = __builtin_fma(p[a], sval[y], ma[lo]);
+                }
+                wave_lds_sync();
+            }
         }
     }
     for (int32_t k = lane; k < R; k += G) oval[o0 + k] = ma[k];
@@ -280,7 +303,9 @@ constexpr int kQCap = 64, kCCap = 128;
 
 // One row-product launch with G lanes per output row, G chosen from the mean source-row
 // length (the lanes spread over a source row's entries: the element level's prolongator
-// rows hold 1-8 entries, an aggregation level's 10-40). Every G gives the same sums.
+// rows hold 1-8 entries, an aggregation level's 10-40; a wave per output row from 24 on, where
+// half a wave takes a second round of loads and searches per term: P^T Q of 4 x 20^3 bricks
+// 590 us, now 284). Every G gives the same sums.
 template <int CAPR>
 static void launch_rowprod(double mean_src, hipStream_t st, int64_t nout, const int32_t *ors, const int32_t *ocol,
                            double *oval, const int32_t *trs, const int32_t *trow, const double *tval,
@@ -296,7 +321,8 @@ static void launch_rowprod(double mean_src, hipStream_t st, int64_t nout, const 
     }
     if (mean_src <= 6.0) PYHIP_ROWPROD(8);
     else if (mean_src <= 12.0) PYHIP_ROWPROD(16);
-    else PYHIP_ROWPROD(32);
+    else if (mean_src <= 24.0) PYHIP_ROWPROD(32);
+    else PYHIP_ROWPROD(64);
 #undef PYHIP_ROWPROD
 }
 

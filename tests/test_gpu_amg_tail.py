@@ -1,6 +1,7 @@
 """The V-cycle's coarse levels in one workgroup per sub-problem against the same levels in
 launches of their own: a small sub-problem runs the whole cycle in its workgroup when it is
-alone, and only the last levels beside a large one; the bits have to be the same. Sizes: below
+alone, and only the last levels beside a large one; the bits have to be the same. The row products of the set-up take other lane counts
+alone than in the batch (by the mean row length), with the same sums. Sizes: below
 the coarsest level's 48 rows, just above, one pass of 256 rows and the next, several levels,
 and sub-problems of one batch that end on different levels."""
 import numpy as np
