@@ -81,16 +81,27 @@ int amg_set_fine(AmgDev &A, const double *vals);
 // into amg_fine_x (see amg_fine_w), e.g. fused into the update that produced b.
 int amg_apply(AmgDev &A, hipStream_t st, const double *b, double *z, KernelTimer *tm = nullptr,
               const int32_t *act = nullptr, const int32_t *act_h = nullptr, bool x0_ready = false);
-// the finest level's smoothing weights W and first-sweep vector (nullptr without levels)
-inline const double *amg_fine_w(const AmgDev &A) { return A.lv.empty() ? nullptr : A.lv[0].w; }
-inline double *amg_fine_x(const AmgDev &A) { return A.lv.empty() ? nullptr : A.lv[0].x; }
+// the finest level's smoothing weights W and first-sweep vector in precision T (nullptr where
+// the cycle reads none: without levels, or all of them in one workgroup)
+template <typename T>
+inline const T *amg_fine_w(const AmgDev &A) {
+    if (A.tail == 0) return nullptr;
+    if constexpr (sizeof(T) == 8) return A.lv[0].w;
+    else return A.lv[0].w32;
+}
+template <typename T>
+inline T *amg_fine_x(const AmgDev &A) {
+    if (A.tail == 0) return nullptr;
+    if constexpr (sizeof(T) == 8) return A.lv[0].x;
+    else return A.lv[0].x32;
+}
 // FP32 V-cycle: after amg_setup (FP64), FP32 copies of every level's values, weights, P,
 // P^T and the coarsest inverses; then the finest FP32 matrix and z = M^-1 b in FP32 (the
 // same cycle as amg_apply, each operation rounded to FP32).
 int amg_make_f32(AmgDev &A, hipStream_t st, int64_t &bytes);
 int amg_set_fine32(AmgDev &A, const float *vals);
 int amg_apply32(AmgDev &A, hipStream_t st, const float *b, float *z, KernelTimer *tm = nullptr,
-                const int32_t *act = nullptr, const int32_t *act_h = nullptr);
+                const int32_t *act = nullptr, const int32_t *act_h = nullptr, bool x0_ready = false);
 void amg_free(AmgDev &A);
 // row-dependent spmv-family bytes of one V-cycle per sub-problem (element size esize)
 std::vector<int64_t> amg_vcycle_bytes(const AmgDev &A, int esize);

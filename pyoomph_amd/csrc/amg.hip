@@ -1064,8 +1064,8 @@ int amg_set_fine32(AmgDev &A, const float *vals) {
 }
 
 int amg_apply32(AmgDev &A, hipStream_t st, const float *b, float *z, KernelTimer *tm, const int32_t *act,
-                const int32_t *act_h) {
-    return amg_apply_t<float>(A, st, b, z, tm, act, act_h, false);
+                const int32_t *act_h, bool x0_ready) {
+    return amg_apply_t<float>(A, st, b, z, tm, act, act_h, x0_ready);
 }
 
 }  // namespace pyhip

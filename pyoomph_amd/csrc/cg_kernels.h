@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_step_kernel(int nsub, const T *
                                                              const double *__restrict__ part,
                                                              const double *__restrict__ sums, int32_t *active,
                                                              int32_t *__restrict__ fail, int32_t *__restrict__ nspmv,
-                                                             const double *__restrict__ w0, double *__restrict__ x0) {
+                                                             const T *__restrict__ w0, T *__restrict__ x0) {
     __shared__ double sh;
     __shared__ int run;
     const int s = C.sub[blockIdx.x];
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_step_kernel(int nsub, const T *
         const T rn = T(double(r[i]) - a * double(q[i]));
         r[i] = rn;
         // the multigrid V-cycle's first smoothing x0 = W r of the new residual
-        if (x0) x0[i] = w0[i] * double(rn);
+        if (x0) x0[i] = w0[i] * rn;
     }
 }
 

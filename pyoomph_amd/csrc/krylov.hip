@@ -13,9 +13,10 @@
 // device (one thread per sub-problem). The host reads one counter per iteration (the
 // number of sub-problems still iterating).
 //
-// Preconditioners: Jacobi, and ILU(0) on the structural pattern, level-scheduled
-// (rows of one level are independent; a level is one launch; levels of all
-// sub-problems are merged by level index). Taylor-Hood sub-problems are factorised with
+// Preconditioners: Jacobi, and ILU(0) on the structural pattern, level-scheduled (rows of
+// one level are independent). Its solves run in one workgroup per small sub-problem
+// (ilu_sliced.h) and otherwise, as the factorisation, in a launch per level with the levels
+// of all sub-problems merged by level index (ilu_levels.h). Taylor-Hood sub-problems are factorised with
 // the velocity unknowns ordered before the pressure unknowns (natural order within
 // each), which keeps ILU(0) pivots non-zero for the zero pressure-pressure block.
 #include <algorithm>
@@ -944,14 +945,18 @@ __global__ void blk_pressure_kernel(int64_t np, const int32_t *__restrict__ prow
     z[row] = v;
 }
 
-// tv = r_u - (G z_p)_u (t = J pz; without pressure rows t is not read)
+// tv = r_u - (G z_p)_u (t = J pz; without pressure rows t is not read), and the V-cycle's
+// first smoothing x0 = W tv where it reads one
 __global__ void blk_vgather_kernel(int64_t nv, const int32_t *__restrict__ vrows, const int32_t *__restrict__ vsub,
                                    const double *__restrict__ r, const double *__restrict__ t,
-                                   double *__restrict__ tv, const int32_t *__restrict__ act) {
+                                   double *__restrict__ tv, const double *__restrict__ w0,
+                                   double *__restrict__ x0, const int32_t *__restrict__ act) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= nv || (act && !act[vsub[i]])) return;
     const int32_t row = vrows[i];
-    tv[i] = t ? r[row] - t[row] : r[row];
+    const double v = t ? r[row] - t[row] : r[row];
+    tv[i] = v;
+    if (x0) x0[i] = w0[i] * v;
 }
 
 __global__ void blk_vscatter_kernel(int64_t nv, const int32_t *__restrict__ vrows, const int32_t *__restrict__ vsub,
@@ -1085,9 +1090,11 @@ static int blk_apply(pyhip_problem *p, KrylovWork *W, const double *r, double *z
     }
     if (B.nv) {
         hipLaunchKernelGGL(blk_vgather_kernel, dim3(nblk(B.nv)), dim3(256), 0, p->st, B.nv, B.vrows, B.vsub, r,
-                           B.np ? (const double *)B.t : nullptr, B.tv, act);
+                           B.np ? (const double *)B.t : nullptr, B.tv, amg_fine_w<double>(B.amg),
+                           amg_fine_x<double>(B.amg), act);
         KCHECK();
-        if ((rc = amg_apply(B.amg, p->st, B.tv, B.zv, &p->timer, act, act_h))) return rc;
+        if ((rc = amg_apply(B.amg, p->st, B.tv, B.zv, &p->timer, act, act_h, amg_fine_x<double>(B.amg) != nullptr)))
+            return rc;
         hipLaunchKernelGGL(blk_vscatter_kernel, dim3(nblk(B.nv)), dim3(256), 0, p->st, B.nv, B.vrows, B.vsub, B.zv, z,
                            act);
         KCHECK();
@@ -1112,7 +1119,7 @@ static int precond_apply(pyhip_problem *p, KrylovWork *W, int pc, const T *v, T 
         if constexpr (std::is_same<T, double>::value)
             return amg_apply(W->amg, p->st, v, z, &p->timer, act, act_h, x0_ready);
         else
-            return amg_apply32(W->amg, p->st, v, z, &p->timer, act, act_h);
+            return amg_apply32(W->amg, p->st, v, z, &p->timer, act, act_h, x0_ready);
     }
     const T *jd = std::is_same<T, float>::value ? (const T *)W->jdiag32 : (const T *)W->jdiag64;
     hipLaunchKernelGGL((jacobi_apply_kernel<T>), dim3(nblk(p->ndof)), dim3(256), 0, p->st, p->ndof, jd, v, z);
@@ -1433,11 +1440,11 @@ static int cg_generic(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *
     if ((rc = read_active(p, W, &nact))) return rc;
     // with the multigrid preconditioner the x/r update also writes the V-cycle's first
     // smoothing W r of the finest level
-    const double *w0 = nullptr;
-    double *x0 = nullptr;
-    if (std::is_same<T, double>::value && o.precond == PYHIP_PRECOND_AMG) {
-        w0 = amg_fine_w(W->amg);
-        x0 = amg_fine_x(W->amg);
+    const T *w0 = nullptr;
+    T *x0 = nullptr;
+    if (o.precond == PYHIP_PRECOND_AMG) {
+        w0 = amg_fine_w<T>(W->amg);
+        x0 = amg_fine_x<T>(W->amg);
     }
     // The host reads the running count every kPcgRead iterations: in between, a converged
     // sub-problem's flag is cleared on the device and every kernel skips its rows, so the
