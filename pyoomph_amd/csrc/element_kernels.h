@@ -251,7 +251,7 @@ __global__ __launch_bounds__(256) void scalar_element_kernel(ElemArgs<T> a) {
 // gradients, shape values and equation number from LDS, and the kernel waited 68 % of its
 // time (sweep of 192 problems: P2 part 557 us, now 257, P1 part 61, now 38). Same operations in the same order per
 // output. The matrices leave through LDS (odd stride per element: no bank conflicts), as
-// contiguous 16-byte stores of the block's elements; entries of pinned rows and columns are
+// coalesced stores over the block's elements; entries of pinned rows and columns are
 // written too (nothing reads them). Bound: FP64 ALU without contraction, then the stores.
 template <typename T, int KIND, int FORM, bool TR, bool JAC>
 __global__ __launch_bounds__(kTriThreads) void tri_element_kernel(ElemArgs<T> a) {
