@@ -454,7 +454,8 @@ int pyhip_arclength_step(pyhip_problem *p, double *dofs_dev, int param, const py
  * stream around every launch of the named kernel families, "element" (element
  * residual / Jacobian kernels), "gather_values", "gather_residual", "spmv" (every sparse
  * matrix-vector launch: the Krylov solver's and, inside the multigrid V-cycle, those of
- * each level's matrix, restriction and prolongation), "precond" (whole preconditioner
+ * the matrix, restriction and prolongation of each level that runs in launches; the coarse
+ * levels in one workgroup are none), "precond" (whole preconditioner
  * applies and factorisations, including the spmv launches they make), "vector" (dots,
  * updates).
  * pyhip_timing_read returns the launches and summed device milliseconds so far;
