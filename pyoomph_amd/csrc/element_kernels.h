@@ -54,6 +54,23 @@ __device__ __constant__ const int8_t kTHNodeSlot[9] = {0, 3, 5, 8, 10, 12, 14, 1
 
 constexpr int kTriThreads = 128;   // elements per workgroup of tri_element_kernel
 
+// Triangles take a thread per element from this many elements on (-1: never). Below, a thread
+// per row fills the chip better. FP64, row and element: P2 matrices 10.4 and 12.2 us on 512
+// elements, 12.2 and 14.0 on 8192, 21.6 both ways on 32768, 36.8 and 24.3 on 80000; P2
+// residuals 6.4 and 9.6 on 3200, 10.1 and 10.6 on 32768, 20.1 and 17.1 on 80000; P1 residuals 4.1
+// and 4.4 on 18432, 8.1 and 7.5 on 80000; P1 matrices never slower; Poisson with its
+// exponentials per point: matrices 31.6 and 32.8 on 52000, 41.9 and 32.8 on 81000, residuals
+// 20.2 and 25.5, 28.1 and 27.9. Both kernels give the same FP64 bits. In FP32 contraction is the
+// compiler's choice, so one kernel serves every size and a sub-problem has the same bits alone and
+// in a batch: an element per thread (8.8 us both ways on 512 elements, 23.3 and 19.3 on 80000),
+// for Poisson a row per thread (9.4 and 12.2 us, 27.1 and 26.7).
+template <typename T, int KIND, int FORM>
+constexpr int tri_min_elements(bool jac) {
+    if (sizeof(T) == 4) return FORM == PYHIP_FORM_POISSON ? -1 : 0;
+    if (FORM == PYHIP_FORM_POISSON) return jac ? 65536 : 81920;
+    return jac ? (KIND == ELEM_TRI_P1 ? 0 : 32768) : 65536;
+}
+
 // TR: the form has a time derivative (a.transient); HV: the matrix output is the
 // Hessian-vector product sum_k dJ_ij/du_k y_k = int d2src (sum_k y_k psi_k) psi_j psi_i
 // (d2src: Bratu -lambda e^u, reaction-diffusion 6u, Poisson 0), symmetric in i, j and k,
@@ -256,8 +273,9 @@ __global__ __launch_bounds__(256) void scalar_element_kernel(ElemArgs<T> a) {
 template <typename T, int KIND, int FORM, bool TR, bool JAC>
 __global__ __launch_bounds__(kTriThreads) void tri_element_kernel(ElemArgs<T> a) {
     using Tt = ElemTraits<KIND>;
-    constexpr int NN = Tt::NN, DIM = 2, NQ = Tt::NQ, NJ = NN * NN, ST = NJ | 1;
-    __shared__ T out[JAC ? kTriThreads * ST : 1];
+    constexpr int NN = Tt::NN, DIM = 2, NQ = Tt::NQ, NJ = NN * NN, ST = (JAC ? NJ : NQ) | 1;
+    constexpr bool GAUSS = FORM == PYHIP_FORM_POISSON;
+    __shared__ T out[JAC || GAUSS ? kTriThreads * ST : 1];   // the matrices; before, the sources
     const int eb = a.e0 + (int)blockIdx.x * kTriThreads, e = eb + (int)threadIdx.x;
     const int el = e < a.e1 ? e : a.e1 - 1;   // the threads past the end repeat the last element
     T X[NN][DIM], U[NN], F[FORM == PYHIP_FORM_REACTION_DIFFUSION ? NN : 1], H[TR ? NN : 1];
@@ -281,6 +299,33 @@ __global__ __launch_bounds__(kTriThreads) void tri_element_kernel(ElemArgs<T> a)
     for (int i = 0; i < NN; i++) R[i] = T(0);
 #pragma unroll
     for (int k = 0; k < (JAC ? NJ : 1); k++) J[k] = T(0);
+    if constexpr (GAUSS) {
+        // the sources of all points together, a Gaussian read once and NQ exponentials of it
+        // independent of each other (point by point: 36 us for 81000 elements, now 33)
+        T x[NQ], y[NQ], f[NQ];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const T *P = a.tab->psi + q * NN;
+            x[q] = y[q] = f[q] = T(0);
+#pragma unroll
+            for (int l = 0; l < NN; l++) x[q] = x[q] + X[l][0] * P[l];
+#pragma unroll
+            for (int l = 0; l < NN; l++) y[q] = y[q] + X[l][1] * P[l];
+        }
+        const int ng = (int)par[0];  // Gaussians follow as (cx, cy, w, a)
+#pragma unroll 1
+        for (int k = 1; k < 1 + 4 * ng; k += 4) {
+            const T cx = T(par[k + 0]), cy = T(par[k + 1]), wk = T(par[k + 2]), ak = T(par[k + 3]);
+#pragma unroll
+            for (int q = 0; q < NQ; q++) {
+                T ddx = x[q] - cx, ddy = y[q] - cy;
+                T r2 = ddx * ddx + ddy * ddy;
+                f[q] = f[q] + ak * texp(-r2 / (wk * wk));
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; q++) out[threadIdx.x * ST + q] = f[q];
+    }
 #pragma unroll 1
     for (int q = 0; q < NQ; q++) {
         const T *P = a.tab->psi + q * NN;
@@ -299,20 +344,7 @@ __global__ __launch_bounds__(kTriThreads) void tri_element_kernel(ElemArgs<T> a)
         }
         T src = T(0), dsrc = T(0);
         if constexpr (FORM == PYHIP_FORM_POISSON) {
-            T x = T(0), y = T(0);
-#pragma unroll
-            for (int l = 0; l < NN; l++) x = x + X[l][0] * P[l];
-#pragma unroll
-            for (int l = 0; l < NN; l++) y = y + X[l][1] * P[l];
-            T f = T(0);
-            const int ng = (int)par[0];  // Gaussians follow as (cx, cy, w, a)
-            for (int k = 1; k < 1 + 4 * ng; k += 4) {
-                T ddx = x - T(par[k + 0]), ddy = y - T(par[k + 1]);
-                T r2 = ddx * ddx + ddy * ddy;
-                T wk = T(par[k + 2]);
-                f = f + T(par[k + 3]) * texp(-r2 / (wk * wk));
-            }
-            src = -f;
+            src = -out[threadIdx.x * ST + q];
         } else if constexpr (FORM == PYHIP_FORM_BRATU) {
             T ev = texp(u);
             src = -par0 * ev;

@@ -10,19 +10,21 @@ static int launch_scalar(const ElemArgs<T> &a, hipStream_t s) {
     const int blocks = (a.e1 - a.e0 + EPB - 1) / EPB;
     if (blocks == 0) return PYHIP_OK;
     if constexpr (KIND == ELEM_TRI_P1 || KIND == ELEM_TRI_P2) {
-        // residuals and Jacobians: a thread per element; parameter derivatives, mass matrices
-        // and Hessian products: a thread per row
-        if (!a.hvec && !a.deriv && a.flag < 2) {
-            const dim3 g((a.e1 - a.e0 + kTriThreads - 1) / kTriThreads), t(kTriThreads);
-            if (a.transient) {
-                if (a.flag) hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, true, true>), g, t, 0, s, a);
-                else hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, true, false>), g, t, 0, s, a);
-            } else {
-                if (a.flag) hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, false, true>), g, t, 0, s, a);
-                else hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, false, false>), g, t, 0, s, a);
+        // residuals and Jacobians of many elements: a thread per element; few, parameter
+        // derivatives, mass matrices and Hessian products: a thread per row
+        if constexpr (tri_min_elements<T, KIND, FORM>(true) >= 0) {
+            if (!a.hvec && !a.deriv && a.flag < 2 && a.e1 - a.e0 >= tri_min_elements<T, KIND, FORM>(a.flag)) {
+                const dim3 g((a.e1 - a.e0 + kTriThreads - 1) / kTriThreads), t(kTriThreads);
+                if (a.transient) {
+                    if (a.flag) hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, true, true>), g, t, 0, s, a);
+                    else hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, true, false>), g, t, 0, s, a);
+                } else {
+                    if (a.flag) hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, false, true>), g, t, 0, s, a);
+                    else hipLaunchKernelGGL((tri_element_kernel<T, KIND, FORM, false, false>), g, t, 0, s, a);
+                }
+                PYHIP_CHECK_HIP(hipGetLastError());
+                return PYHIP_OK;
             }
-            PYHIP_CHECK_HIP(hipGetLastError());
-            return PYHIP_OK;
         }
     }
     if constexpr (KIND == ELEM_HEX_Q2) {

@@ -1,7 +1,7 @@
 """Element kernels and the gather at the edges of their workgroups: one element, a last
-workgroup that is nearly empty, exactly full ones and the next size (128 triangles, 7 and 28
-bricks, 128 (element, node) pairs of Taylor-Hood elements, 512 matrix entries), steady and
-with the time derivative.
+workgroup that is nearly empty, exactly full ones and the next size (128 triangles; 32768, 65536
+and 81920 triangles, where FP64 changes the kernel; 7 and 28 bricks, 128 (element, node)
+pairs of Taylor-Hood elements, 512 matrix entries), steady and with the time derivative.
 
 Bar: FP64 bitwise against the oracle (1e-12 where the exponential enters, as in the parity
 tests). FP32 against FP64, relative to the largest entry: (27 + 16 N) 2^-24. A sum of at most
@@ -18,7 +18,9 @@ from tests.test_gpu_parity import build, rel
 pytestmark = pytest.mark.gpu
 
 SIZES = ([("bratu", dict(N=N, space=sp, lam=2.0)) for sp in ("C1", "C2") for N in (2, 8, 9, 17)] +
-         [("poisson", dict(N=N)) for N in (2, 8, 9)] +
+         [("bratu", dict(N=N, space=sp, lam=2.0)) for sp, N in (("C1", 181), ("C1", 182), ("C2", 127), ("C2", 128),
+                                                                ("C2", 182))] +
+         [("poisson", dict(N=N)) for N in (2, 8, 9, 181, 182, 203)] +
          [("rd", dict(N=N)) for N in (1, 2, 3, 4)] +
          [("ns", dict(N=N)) for N in (2, 4, 15)])
 
