@@ -21,6 +21,10 @@ namespace pyhip {
 constexpr int kIluSlicedThreads = 64 * kIluSliceWaves;
 // rows whose FP64 vector (and the zero behind it) fits the CU's LDS
 constexpr int kIluSlicedRows = 20000;
+template <typename T>
+constexpr size_t ilu_sliced_lds(int rows) {
+    return (size_t)(rows + 1) * sizeof(T);
+}
 
 template <typename T>
 struct IluSlicedDev {

@@ -676,6 +676,15 @@ static void ilu_free(KrylovWork *W) {
     L = IluPlan();
 }
 
+// rows of the largest sub-problem that one workgroup of this device solves
+static int ilu_sliced_cap(int *cap) {
+    int lds = 0, dev = 0;
+    PYHIP_CHECK_HIP(hipGetDevice(&dev));
+    PYHIP_CHECK_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    *cap = std::max(0, std::min<int>(kIluSlicedRows, lds / (int)sizeof(double) - 1));
+    return PYHIP_OK;
+}
+
 static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
     IluPlan &L = W->ilu;
     if (L.built && L.requested == W->ilu_order) return PYHIP_OK;
@@ -718,12 +727,10 @@ static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
         return PYHIP_ERR_BREAKDOWN;
     }
     // sub-problems whose vector fits one CU's LDS are solved in one workgroup each
-    int lds = 0, dev = 0;
-    PYHIP_CHECK_HIP(hipGetDevice(&dev));
-    PYHIP_CHECK_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    int cap = 0, rc;
+    if ((rc = ilu_sliced_cap(&cap))) return rc;
     IluSlicedPlan Q;
-    if (ilu_sliced_host(H, p->dof_off_h, std::max(0, std::min<int>(kIluSlicedRows, lds / (int)sizeof(double) - 1)), Q,
-                        err)) {
+    if (ilu_sliced_host(H, p->dof_off_h, cap, Q, err)) {
         set_error(err);
         return PYHIP_ERR_INVALID;
     }
@@ -732,7 +739,6 @@ static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
     L.multicolor = H.multicolor;
     L.nsliced = (int)Q.subs.size();
     L.max_rows = Q.max_rows;
-    int rc;
 #define LUP(dst, v)                                                                        \
     if ((rc = kalloc(&(dst), (v).size(), W))) return rc;                                   \
     if (!(v).empty())                                                                      \
@@ -814,10 +820,13 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
                 (rc = dev_alloc((T **)&L.sup.val, L.sup.nval, W->bytes)) ||
                 (rc = dev_alloc((T **)&L.sdiag, L.ndiag, W->bytes)))
                 return rc;
-            // the solve's vector takes most of a CU's LDS
+            // The limit belongs to the function, not to this problem: always the largest one, so that
+            // other problems' applies, older ones and those of other threads, stay within it.
+            int cap = 0;
+            if ((rc = ilu_sliced_cap(&cap))) return rc;
             PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ilu_sliced_apply_kernel<T>),
                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                (int)((L.max_rows + 1) * sizeof(T))));
+                                                (int)ilu_sliced_lds<T>(cap)));
         }
         if (L.llo.rows) {
             for (IluPlan::Levels *S : {&L.llo, &L.lup})
@@ -873,7 +882,7 @@ static int ilu_apply(pyhip_problem *p, KrylovWork *W, const T *v, T *z, const in
             return IluSlicedDev<T>{S.nlev, S.chunk0, S.idx, (const T *)S.val, rdiag};
         };
         hipLaunchKernelGGL((ilu_sliced_apply_kernel<T>), dim3(L.nsliced), dim3(kIluSlicedThreads),
-                           (size_t)(L.max_rows + 1) * sizeof(T), p->st, L.ssubs, L.srow0, L.srows, L.perm,
+                           ilu_sliced_lds<T>(L.max_rows), p->st, L.ssubs, L.srow0, L.srows, L.perm,
                            dev(L.slo, nullptr), dev(L.sup, (const T *)L.sdiag), v, z, act);
         KCHECK();
     }
@@ -1246,7 +1255,8 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     const GsChunks C = W->gs_chunks();
     const bool reduced = W->gs_max > kGsFusedChunks;
     PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gs_backsolve_kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)gs_backsolve_lds(m, mr)));
+                                        hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)gs_backsolve_lds(kMaxRestart, kMaxRestart)));   // as any solve sets it
     int total = 0, nact = 0;
     const int max_cycles = std::max(1, (o.max_iters + mr - 1) / mr);
     for (int cyc = 0; cyc < max_cycles; cyc++) {

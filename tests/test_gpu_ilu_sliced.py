@@ -49,3 +49,25 @@ def test_plugin_solves_matrices_at_the_edges_of_the_rule(gpu, n, band):
     S.solve_serial(2, n, A.nnz, 1, None, None, None, x, n, 1)
     want = sl.spsolve(A.tocsc(), b)
     assert np.linalg.norm(x - want) <= 1e-9 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_large_problem_solves_again_after_a_small_one(gpu, precision):
+    """The LDS limit of the kernel is one of the function, whatever problem was set up last:
+    9801 rows (78 KB in FP64), then 49, both alive, then the large one without a new set-up."""
+    import torch
+    from pyoomph_amd import workloads as wl
+    from pyoomph_amd.problem import Problem
+
+    def solve(P):
+        with torch.cuda.stream(P._stream):
+            P.dofs.zero_()
+        assert all(s["converged"] and s["linear_failures"] == 0 for s in P.solve())
+        return P.get_current_dofs()
+
+    large, small = (Problem([wl.bratu(N, "C1", 1.0)]) for N in (100, 8))
+    for P in (large, small):
+        P.preconditioner, P.linear_precision = "ilu0", precision
+    x = solve(large)
+    solve(small)
+    assert np.array_equal(x, solve(large))
