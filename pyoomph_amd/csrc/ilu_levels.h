@@ -98,4 +98,29 @@ __global__ __launch_bounds__(256) void ilu_level_kernel(IluLevel L, int32_t nfir
     }
 }
 
+// The rows, columns and factor places of one level, once per plan; a thread per (row, stripe)
+__global__ __launch_bounds__(256) void ilu_level_layout_kernel(IluLevel L, const int32_t *__restrict__ order,
+                                                               const int32_t *__restrict__ prs,
+                                                               const int32_t *__restrict__ pcol,
+                                                               const int32_t *__restrict__ pdiag,
+                                                               const int32_t *__restrict__ perm, bool lower,
+                                                               int32_t *__restrict__ row, int32_t *__restrict__ col,
+                                                               int32_t *__restrict__ src, int32_t *__restrict__ rsrc) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= 8 * (int64_t)L.rows) return;
+    ilu_level_stripe(L, (int32_t)(k / 8), (int)(k % 8), order, prs, pcol, pdiag, perm, lower, row, col, src, rsrc);
+}
+
+// val[k] = lu[src[k]] (0 at padding), or, for the pivots, its reciprocal
+template <typename T>
+__global__ __launch_bounds__(256) void ilu_level_fill_kernel(int64_t n, const int32_t *__restrict__ src,
+                                                             const T *__restrict__ lu, T *__restrict__ val,
+                                                             int reciprocal) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= n) return;
+    const int32_t s = src[k];
+    const T v = s >= 0 ? lu[s] : T(0);
+    val[k] = reciprocal ? (s >= 0 ? T(1) / v : T(0)) : v;
+}
+
 }  // namespace pyhip

@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <thread>
 #include <utility>
 
 namespace pyhip {
@@ -144,14 +145,50 @@ int ilu_plan_host(int64_t n, const int32_t *rs, const int32_t *col, const std::v
     return 0;
 }
 
+// Stable sort of rows [b, e) by decreasing key(row) >= 0; tmp, cnt: scratch
+template <typename K>
+static void sort_decreasing(int32_t *b, int32_t *e, K key, std::vector<int32_t> &tmp, std::vector<int32_t> &cnt) {
+    const int64_t n = e - b;
+    int32_t top = 0;
+    for (int32_t *r = b; r < e; r++) top = std::max(top, key(*r));
+    if (n < 16 || top > 4 * n) {   // few rows, or more counters than rows
+        std::stable_sort(b, e, [&](int32_t x, int32_t y) { return key(x) > key(y); });
+        return;
+    }
+    cnt.assign(top + 2, 0);
+    for (int32_t *r = b; r < e; r++) cnt[top - key(*r) + 1]++;
+    for (int32_t k = 0; k <= top; k++) cnt[k + 1] += cnt[k];
+    tmp.assign(b, e);
+    for (int32_t r : tmp) b[cnt[top - key(r)]++] = r;
+}
+
+template <typename F>
+static void parallel_subs(int n, F &&fn) {
+    unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+    if (n < 64) nt = 1;
+    const int per = (n + (int)nt - 1) / (int)nt;
+    std::vector<std::thread> th;
+    for (int b = 0; b < n; b += per) {
+        const int e = std::min(n, b + per);
+        if (nt == 1) fn(b, e);
+        else th.emplace_back([&fn, b, e]() { fn(b, e); });
+    }
+    for (auto &x : th) x.join();
+}
+
 // One side (lower or upper) of the sliced plan for the handled sub-problems: level lists
 // from the merged level lists `rows` / `ptr` of the whole batch.
 static int sliced_side(const IluHostPlan &H, const std::vector<int32_t> &rows, const std::vector<int64_t> &ptr,
                        bool lower, const std::vector<int32_t> &slot_of, const IluSlicedPlan &P, const std::vector<int32_t> &row_sub, IluSlicedSide &S,
                        std::vector<int32_t> &big, std::vector<int64_t> &big_ptr, std::string &err) {
     const int nh = (int)P.subs.size(), nl = (int)ptr.size() - 1;
-    // per handled sub-problem: (level, rows) lists in level order
-    std::vector<std::vector<std::pair<int32_t, std::vector<int32_t>>>> lists(nh);
+    auto len = [&](int32_t r) { return lower ? H.pdiag[r] - H.prs[r] : H.prs[r + 1] - H.pdiag[r] - 1; };
+    // rows of each handled sub-problem in level order, and each one's level
+    std::vector<int64_t> start(nh + 1, 0);
+    for (int t = 0; t < nh; t++) start[t + 1] = start[t] + P.rows[t];
+    std::vector<int64_t> pos(start.begin(), start.end() - 1);
+    std::vector<int32_t> level(start[nh]);
+    S.order.resize(start[nh]);
     big_ptr.assign(1, 0);
     for (int l = 0; l < nl; l++) {
         for (int64_t w = ptr[l]; w < ptr[l + 1]; w++) {
@@ -160,87 +197,98 @@ static int sliced_side(const IluHostPlan &H, const std::vector<int32_t> &rows, c
                 big.push_back(r);
                 continue;
             }
-            if (lists[t].empty() || lists[t].back().first != l) lists[t].push_back({l, {}});
-            lists[t].back().second.push_back(r);
+            level[pos[t]] = l;
+            S.order[pos[t]++] = r;
         }
         if ((int64_t)big.size() > big_ptr.back()) big_ptr.push_back((int64_t)big.size());
     }
-    auto len = [&](int32_t r) { return lower ? H.pdiag[r] - H.prs[r] : H.prs[r + 1] - H.pdiag[r] - 1; };
-    S.chunk0.assign(1, 0);
-    struct Slice {
-        int level, lanes;
-        size_t b, n;
-        const std::vector<int32_t> *rows;
-    };
-    for (int t = 0; t < nh; t++) {
-        const int32_t r0 = P.row0[t], dummy = P.rows[t];
-        std::vector<std::vector<Slice>> waves(kIluSliceWaves);
-        for (size_t l = 0; l < lists[t].size(); l++) {
-            auto &R = lists[t][l].second;
-            std::stable_sort(R.begin(), R.end(), [&](int32_t a, int32_t b) { return len(a) > len(b); });
+    // the slices of sub-problem t, whose levels are sorted: f(wave, level, lanes, first row, rows, chunks)
+    auto cut = [&](int t, auto f) {
+        for (int64_t a = start[t]; a < start[t + 1];) {
+            int64_t e = a;
+            while (e < start[t + 1] && level[e] == level[a]) e++;
+            const int64_t R = e - a;
+            const int32_t longest = len(S.order[a]);
             // lanes that still leave the level at most one slice per wave
             int fill = 1;
-            while (fill < 16 && 2 * fill * (int64_t)R.size() <= kIluSliceLanes * kIluSliceWaves && fill < len(R[0]))
-                fill *= 2;
+            while (fill < 16 && 2 * fill * R <= kIluSliceLanes * kIluSliceWaves && fill < longest) fill *= 2;
             int k = 0;
-            for (size_t b = 0; b < R.size(); k++) {
+            for (int64_t b = a; b < e; k++) {
                 int lanes = fill;
-                while (lanes < 16 && (len(R[b]) + lanes - 1) / lanes > kIluChunk) lanes *= 2;
-                const size_t m = std::min<size_t>(kIluSliceLanes / lanes, R.size() - b);
-                waves[k % kIluSliceWaves].push_back({(int)l, lanes, b, m, &R});
+                const int32_t n = len(S.order[b]);
+                while (lanes < 16 && (n + lanes - 1) / lanes > kIluChunk) lanes *= 2;
+                const int m = (int)std::min<int64_t>(kIluSliceLanes / lanes, e - b);
+                const int steps = (n + lanes - 1) / lanes;
+                f(k % kIluSliceWaves, (int)level[a], lanes, b, m, std::max(1, (steps + kIluChunk - 1) / kIluChunk));
                 b += m;
             }
+            a = e;
         }
-        S.nlev.push_back((int32_t)lists[t].size());
-        for (const auto &tasks : waves) {
-            const size_t first = S.chunk0.back();
-            uint16_t mark = 0;
-            // appends an empty chunk
-            auto chunk = [&]() -> size_t {
-                const size_t c = S.idx.size() / kIluChunkIdx;
-                S.idx.resize((c + 1) * kIluChunkIdx, (uint16_t)dummy);
-                S.src.resize((c + 1) * kIluChunkVal, -1);
-                for (int lane = 0; lane < kIluSliceLanes; lane++) {
-                    S.idx[c * kIluChunkIdx + lane * 8 + kIluChunk] = kIluNoRow;
-                    S.idx[c * kIluChunkIdx + lane * 8 + kIluChunk + 1] = mark;
-                }
-                return c;
-            };
-            for (const Slice &sl : tasks) {
-                const std::vector<int32_t> &R = *sl.rows;
-                const int lanes = sl.lanes, w = (len(R[sl.b]) + lanes - 1) / lanes;
-                const int nch = std::max(1, (w + kIluChunk - 1) / kIluChunk);
-                const uint16_t base = (uint16_t)(sl.level | __builtin_ctz(lanes) << 12);
-                size_t c0 = 0;
-                for (int c = 0; c < nch; c++) {
-                    mark = (uint16_t)(base | (c + 1 < nch ? 1 << 15 : 0));
-                    const size_t at = chunk();
-                    if (c == 0) c0 = at;
-                    for (int lane = 0; lane < kIluSliceLanes; lane++)
-                        if ((size_t)(lane / lanes) < sl.n)
-                            S.idx[at * kIluChunkIdx + lane * 8 + kIluChunk] =
-                                (uint16_t)(R[sl.b + lane / lanes] - r0);
-                }
-                for (size_t q = 0; q < sl.n; q++) {
-                    const int32_t r = R[sl.b + q], k0 = lower ? H.prs[r] : H.pdiag[r] + 1;
-                    for (int e = 0; e < len(r); e++) {
-                        const int step = e / lanes, j = step % kIluChunk;
-                        const size_t lane = q * lanes + e % lanes, c = c0 + step / kIluChunk;
-                        S.idx[c * kIluChunkIdx + lane * 8 + j] = (uint16_t)(H.pcol[k0 + e] - r0);
-                        S.src[c * kIluChunkVal + (j / 2) * 2 * kIluSliceLanes + 2 * lane + j % 2] = k0 + e;
-                    }
-                }
+    };
+    S.nlev.resize(nh);
+    std::vector<int64_t> c0((size_t)nh * kIluSliceWaves + 1, 0);
+    parallel_subs(nh, [&](int t0, int t1) {
+        std::vector<int32_t> tmp, cnt;
+        for (int t = t0; t < t1; t++) {
+            int32_t *o = S.order.data();
+            for (int64_t a = start[t], e; a < start[t + 1]; a = e) {
+                for (e = a; e < start[t + 1] && level[e] == level[a];) e++;
+                sort_decreasing(o + a, o + e, len, tmp, cnt);
             }
-            mark &= 0xfff;   // padding stays on the wave's last level
-            while ((S.idx.size() / kIluChunkIdx - first) % kIluDepth) chunk();
-            if (S.src.size() >= (size_t)INT32_MAX) {
-                err = "ILU(0) sliced plan: too many entries";
-                return -1;
+            S.nlev[t] = start[t + 1] > start[t] ? level[start[t + 1] - 1] + 1 : 0;
+            int64_t *c = c0.data() + (size_t)t * kIluSliceWaves + 1;
+            cut(t, [&](int w, int, int, int64_t, int, int nch) { c[w] += nch; });
+            for (int w = 0; w < kIluSliceWaves; w++) c[w] = (c[w] + kIluDepth - 1) / kIluDepth * kIluDepth;
+        }
+    });
+    for (size_t w = 1; w < c0.size(); w++) c0[w] += c0[w - 1];
+    if (c0.back() > INT32_MAX || start[nh] > INT32_MAX) {
+        err = "ILU(0) sliced plan: too many chunks";
+        return -1;
+    }
+    S.chunk0.assign(c0.begin(), c0.end());
+    S.chunk.resize(c0.back());
+    parallel_subs(nh, [&](int t0, int t1) {
+        for (int t = t0; t < t1; t++) {
+            const int64_t *c = c0.data() + (size_t)t * kIluSliceWaves;
+            int64_t at[kIluSliceWaves];
+            uint16_t last[kIluSliceWaves] = {0};
+            std::copy(c, c + kIluSliceWaves, at);
+            cut(t, [&](int w, int lev, int lanes, int64_t b, int m, int nch) {
+                const uint16_t base = (uint16_t)(lev | __builtin_ctz(lanes) << 12);
+                for (int q = 0; q < nch; q++)
+                    S.chunk[at[w]++] = IluChunk{(int32_t)b, q * kIluChunk, t,
+                                                (uint16_t)(base | (q + 1 < nch ? 1 << 15 : 0)), (uint16_t)m};
+                last[w] = (uint16_t)lev;
+            });
+            // padding stays on the wave's last level
+            for (int w = 0; w < kIluSliceWaves; w++)
+                while (at[w] < c[w + 1]) S.chunk[at[w]++] = IluChunk{0, 0, t, last[w], 0};
+        }
+    });
+    return 0;
+}
+
+void ilu_sliced_expand(const IluHostPlan &H, const IluSlicedPlan &P, bool lower, std::vector<uint16_t> &idx,
+                       std::vector<int32_t> &src) {
+    const IluSlicedSide &S = lower ? P.lo : P.up;
+    idx.resize(S.chunk.size() * kIluChunkIdx);
+    src.assign(S.chunk.size() * kIluChunkVal, -1);
+    for (size_t c = 0; c < S.chunk.size(); c++) {
+        const IluChunk &C = S.chunk[c];
+        const int32_t r0 = P.row0[C.slot];
+        for (int lane = 0; lane < kIluSliceLanes; lane++) {
+            const IluLane L = ilu_chunk_lane(C, lane, S.order.data(), H.prs.data(), H.pdiag.data(), lower);
+            uint16_t *ix = idx.data() + c * kIluChunkIdx + lane * 8;
+            for (int j = 0; j < kIluChunk; j++) {
+                const bool in = L.e(j) < L.len;
+                ix[j] = (uint16_t)(in ? H.pcol[L.k0 + L.e(j)] - r0 : P.rows[C.slot]);
+                if (in) src[c * kIluChunkVal + (j / 2) * 2 * kIluSliceLanes + 2 * lane + j % 2] = L.k0 + L.e(j);
             }
-            S.chunk0.push_back((int32_t)(S.idx.size() / kIluChunkIdx));
+            ix[kIluChunk] = L.row >= 0 ? (uint16_t)(L.row - r0) : kIluNoRow;
+            ix[kIluChunk + 1] = C.mark;
         }
     }
-    return 0;
 }
 
 int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, int cap, IluSlicedPlan &out,
@@ -292,21 +340,23 @@ int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, i
     return rc;
 }
 
-int ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
-                   bool lower, IluLevelSide &out, std::string &err) {
+void ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
+                    bool lower, IluLevelSide &out) {
     out = IluLevelSide();
-    auto len = [&](int32_t r) { return lower ? H.pdiag[r] - H.prs[r] : H.prs[r + 1] - H.pdiag[r] - 1; };
-    std::vector<int32_t> R;
+    auto steps_of = [&](int32_t r) {
+        const int32_t n = lower ? H.pdiag[r] - H.prs[r] : H.prs[r + 1] - H.pdiag[r] - 1;
+        return (n + 7) / 8;
+    };
+    out.order = big_rows;
+    std::vector<int32_t> tmp, cnt;
     for (size_t l = 0; l + 1 < big_ptr.size(); l++) {
-        R.assign(big_rows.begin() + big_ptr[l], big_rows.begin() + big_ptr[l + 1]);
-        auto steps_of = [&](int32_t r) { return (len(r) + 7) / 8; };
-        std::stable_sort(R.begin(), R.end(), [&](int32_t a, int32_t b) { return steps_of(a) > steps_of(b); });
+        int32_t *R = out.order.data() + big_ptr[l];
+        sort_decreasing(R, out.order.data() + big_ptr[l + 1], steps_of, tmp, cnt);
         IluLevel L;
-        L.rows = (int32_t)R.size();
-        L.row0 = (int32_t)out.row.size();
+        L.rows = (int32_t)(big_ptr[l + 1] - big_ptr[l]);
+        L.row0 = (int32_t)big_ptr[l];
         // narrow levels: more lanes per row, for more loads in flight
         L.lanes = L.rows <= 16384 ? 8 : L.rows <= 65536 ? 4 : 2;
-        const int ns = 8 / L.lanes;
         for (int32_t b = 0; b < L.rows;) {
             const int g = L.nseg++, steps = steps_of(R[b]);
             int32_t e = b;
@@ -315,34 +365,25 @@ int ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, c
             L.seg_row[g] = b;
             L.seg_row[g + 1] = e;
             L.steps[g] = steps;
-            L.off[g] = (int64_t)out.col.size();
-            const int64_t S = (int64_t)(e - b) * L.lanes;
-            out.col.resize(out.col.size() + S * ns * steps);
-            out.src.resize(out.col.size(), -1);
-            for (int32_t q = b; q < e; q++) {
-                const int32_t r = R[q], k0 = lower ? H.prs[r] : H.pdiag[r] + 1, n = len(r);
-                const int32_t pad = n ? H.perm[H.pcol[k0]] : H.perm[r];
-                for (int k = 0; k < 8 * steps; k++) {
-                    const int st = k % 8, u = st % L.lanes, j = st / L.lanes;
-                    const int64_t at = L.off[g] + ((int64_t)(k / 8) * ns + j) * S + (int64_t)(q - b) * L.lanes + u;
-                    out.col[at] = k < n ? H.perm[H.pcol[k0 + k]] : pad;
-                    out.src[at] = k < n ? k0 + k : -1;
-                }
-            }
+            L.off[g] = out.entries;
+            out.entries += (int64_t)(e - b) * 8 * steps;
             b = e;
-        }
-        for (const int32_t r : R) {
-            const bool last = lower && H.prs[r + 1] - H.pdiag[r] == 1;
-            out.row.push_back(last ? (H.perm[r] | kIluLast) : H.perm[r]);
-            out.rsrc.push_back(H.pdiag[r]);
         }
         out.lev.push_back(L);
     }
-    if (out.col.size() >= (size_t)INT64_C(1) << 40) {
-        err = "ILU(0) level plan: too many entries";
-        return -1;
-    }
-    return 0;
+}
+
+void ilu_level_expand(const IluHostPlan &H, const IluLevelSide &S, bool lower, std::vector<int32_t> &row,
+                      std::vector<int32_t> &col, std::vector<int32_t> &src, std::vector<int32_t> &rsrc) {
+    row.resize(S.order.size());
+    rsrc.resize(S.order.size());
+    col.resize(S.entries);
+    src.resize(S.entries);
+    for (const IluLevel &L : S.lev)
+        for (int32_t i = 0; i < L.rows; i++)
+            for (int st = 0; st < 8; st++)
+                ilu_level_stripe(L, i, st, S.order.data(), H.prs.data(), H.pcol.data(), H.pdiag.data(), H.perm.data(),
+                                 lower, row.data(), col.data(), src.data(), rsrc.data());
 }
 
 }  // namespace pyhip

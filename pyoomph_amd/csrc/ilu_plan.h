@@ -6,6 +6,13 @@
 #include <string>
 #include <vector>
 
+#if defined(__HIPCC__)
+#include <hip/hip_runtime.h>
+#define PYHIP_HD __host__ __device__
+#else
+#define PYHIP_HD
+#endif
+
 namespace pyhip {
 
 struct IluHostPlan {
@@ -39,6 +46,10 @@ int ilu_plan_host(int64_t n, const int32_t *rs, const int32_t *col, const std::v
 // in level order, padded with empty ones to a multiple of kIluDepth, so that a wave reads one
 // stream. Columns and rows are local to the sub-problem (16 bits); steps past a row's end
 // point at the local row `rows` (one past the last), where the solve keeps a zero.
+// The host cuts the levels (IluChunk: 16 bytes a chunk); the chunks' columns and the place of
+// their factor entries are written out where they are used, by kernels (ilu_sliced.h) or for
+// tests (ilu_sliced_expand): written out by the host and copied, the padded arrays took up to ten
+// times the rest of a first solve (4096 P1 meshes of 8 x 8: 17 ms without them, 173 with).
 constexpr int kIluSliceLanes = 64;
 constexpr int kIluSliceWaves = 16;
 constexpr int kIluChunk = 6;
@@ -46,11 +57,17 @@ constexpr int kIluDepth = 3;                // chunks a wave loads ahead
 constexpr int kIluChunkIdx = kIluSliceLanes * 8, kIluChunkVal = kIluSliceLanes * kIluChunk;
 constexpr uint16_t kIluNoRow = 0xffff;
 constexpr int kIluMaxLevels = 4096;
+struct IluChunk {
+    int32_t at;        // its rows: [at, at + n) of the side's row list
+    int32_t first;     // their first step in this chunk
+    int32_t slot;      // handled sub-problem
+    uint16_t mark, n;  // n 0: padding
+};
 struct IluSlicedSide {
     std::vector<int32_t> nlev;               // [handled] levels of each sub-problem
     std::vector<int32_t> chunk0;             // [handled * waves + 1] first chunk of each wave
-    std::vector<uint16_t> idx;               // [chunks * kIluChunkIdx]
-    std::vector<int32_t> src;                // [chunks * kIluChunkVal] index in the permuted pattern (-1: none)
+    std::vector<int32_t> order;              // permuted rows by (sub-problem, level, decreasing length)
+    std::vector<IluChunk> chunk;
 };
 struct IluSlicedPlan {
     std::vector<int32_t> subs, row0, rows;   // handled sub-problems (longest first), first permuted row, row count
@@ -59,6 +76,24 @@ struct IluSlicedPlan {
     std::vector<int64_t> big_lo_ptr, big_up_ptr;
     int max_rows = 0;                        // largest handled sub-problem
 };
+
+// Lane `lane` of a chunk: its permuted row (-1: none), the row's entries on this side
+// [k0, k0 + len) of the permuted pattern and the lane's entry of step j, e(j) (< len: taken)
+struct IluLane {
+    int32_t row, k0, len, lanes, e0;
+    PYHIP_HD int32_t e(int j) const { return e0 + j * lanes; }
+};
+PYHIP_HD inline IluLane ilu_chunk_lane(const IluChunk &C, int lane, const int32_t *order, const int32_t *prs,
+                                       const int32_t *pdiag, bool lower) {
+    const int sh = (C.mark >> 12) & 7;
+    IluLane L = {-1, 0, 0, 1 << sh, 0};
+    if ((lane >> sh) >= C.n) return L;
+    L.row = order[C.at + (lane >> sh)];
+    L.k0 = lower ? prs[L.row] : pdiag[L.row] + 1;
+    L.len = (lower ? pdiag[L.row] : prs[L.row + 1]) - L.k0;
+    L.e0 = C.first * L.lanes + (lane & (L.lanes - 1));
+    return L;
+}
 
 // The sliced plan of H (ilu_plan_host); cap < 65535. A sub-problem is handled if it has at
 // most cap rows and kIluMaxLevels levels on each side, and at most kIluEntriesPerLevel
@@ -70,7 +105,9 @@ struct IluSlicedPlan {
 constexpr int64_t kIluEntriesPerLevel = 10000;
 int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, int cap, IluSlicedPlan &out,
                     std::string &err);
-
+// idx and, as indices in the permuted pattern (-1: none), val of a side
+void ilu_sliced_expand(const IluHostPlan &H, const IluSlicedPlan &P, bool lower, std::vector<uint16_t> &idx,
+                       std::vector<int32_t> &src);
 
 // Level-by-level solves of the other sub-problems, a launch per level, in the problem's own
 // row numbering. A level's rows are sorted by decreasing entry count and cut into segments of
@@ -87,14 +124,43 @@ struct IluLevel {
     int64_t off[kIluSegments] = {0};           // first entry of each segment
 };
 constexpr int32_t kIluLast = INT32_MIN;        // row mark (sign bit): no upper entries
+// Place of entry k (0 .. 8 steps - 1) of the level's row i, in segment g
+PYHIP_HD inline int64_t ilu_level_place(const IluLevel &L, int g, int32_t i, int k) {
+    const int ns = 8 / L.lanes, st = k % 8;
+    const int64_t S = (int64_t)(L.seg_row[g + 1] - L.seg_row[g]) * L.lanes;
+    return L.off[g] + ((int64_t)(k / 8) * ns + st / L.lanes) * S + (int64_t)(i - L.seg_row[g]) * L.lanes + st % L.lanes;
+}
 struct IluLevelSide {
     std::vector<IluLevel> lev;
-    std::vector<int32_t> row, col, src, rsrc;  // problem rows (lower: | kIluLast where it applies), problem
-                                               // columns, permuted-pattern index of each entry (-1: padding)
-                                               // and of each row's pivot
+    std::vector<int32_t> order;              // permuted rows by (level, decreasing steps)
+    int64_t entries = 0;
 };
-// big_rows / big_ptr: the permuted rows by level (IluSlicedPlan). Returns 0 or -1 (err).
-int ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
-                   bool lower, IluLevelSide &out, std::string &err);
+// Written out, by a kernel (ilu_levels.h) or ilu_level_expand: problem rows (lower: | kIluLast
+// where it applies), problem columns, permuted-pattern index of each entry (-1: padding) and
+// of each row's pivot.
+// big_rows / big_ptr: the permuted rows by level (IluSlicedPlan).
+void ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
+                    bool lower, IluLevelSide &out);
+void ilu_level_expand(const IluHostPlan &H, const IluLevelSide &S, bool lower, std::vector<int32_t> &row,
+                      std::vector<int32_t> &col, std::vector<int32_t> &src, std::vector<int32_t> &rsrc);
+// one stripe (entries st, st + 8, ...) of the level's row i
+PYHIP_HD inline void ilu_level_stripe(const IluLevel &L, int32_t i, int st, const int32_t *order, const int32_t *prs,
+                                      const int32_t *pcol, const int32_t *pdiag, const int32_t *perm, bool lower,
+                                      int32_t *row, int32_t *col, int32_t *src, int32_t *rsrc) {
+    const int32_t r = order[L.row0 + i], k0 = lower ? prs[r] : pdiag[r] + 1,
+                  n = (lower ? pdiag[r] : prs[r + 1]) - k0;
+    if (st == 0) {
+        const bool last = lower && prs[r + 1] - pdiag[r] == 1;
+        row[L.row0 + i] = last ? (perm[r] | kIluLast) : perm[r];
+        rsrc[L.row0 + i] = pdiag[r];
+    }
+    int g = 0;
+    while (i >= L.seg_row[g + 1]) g++;
+    for (int k = st; k < 8 * L.steps[g]; k += 8) {
+        const int64_t at = ilu_level_place(L, g, i, k);
+        col[at] = k < n ? perm[pcol[k0 + k]] : n ? perm[pcol[k0]] : perm[r];
+        src[at] = k < n ? k0 + k : -1;
+    }
+}
 
 }  // namespace pyhip

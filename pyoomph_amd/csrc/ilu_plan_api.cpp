@@ -76,10 +76,13 @@ int pyhip_ilu_sliced_copy(const void *h, int nsub, const int64_t *sub_off, int c
     IluSlicedPlan Q;
     if (ilu_sliced_host(*P, std::vector<int64_t>(sub_off, sub_off + nsub + 1), cap, Q, g_ilu_err)) return -1;
     const IluSlicedSide &S = side ? Q.up : Q.lo;
+    std::vector<uint16_t> x;
+    std::vector<int32_t> sr;
+    if (idx || src) ilu_sliced_expand(*P, Q, side == 0, x, sr);
     const auto &bg = side ? Q.big_up : Q.big_lo;
     const auto &bp = side ? Q.big_up_ptr : Q.big_lo_ptr;
     sizes[0] = (int64_t)Q.subs.size();
-    sizes[1] = (int64_t)S.idx.size() / kIluChunkIdx;
+    sizes[1] = (int64_t)S.chunk.size();
     sizes[2] = (int64_t)bg.size();
     sizes[3] = (int64_t)bp.size() - 1;
     auto cp = [](auto *dst, const auto &v) {
@@ -88,8 +91,8 @@ int pyhip_ilu_sliced_copy(const void *h, int nsub, const int64_t *sub_off, int c
     cp(subs, Q.subs);
     cp(nlev, S.nlev);
     cp(chunk0, S.chunk0);
-    cp(idx, S.idx);
-    cp(src, S.src);
+    cp(idx, x);
+    cp(src, sr);
     cp(big, bg);
     cp(big_ptr, bp);
     return 0;
@@ -104,12 +107,13 @@ int pyhip_ilu_level_copy(const void *h, int nsub, const int64_t *sub_off, int ca
     if (!P || !sizes || !sub_off || nsub < 1) return -1;
     IluSlicedPlan Q;
     IluLevelSide S;
-    if (ilu_sliced_host(*P, std::vector<int64_t>(sub_off, sub_off + nsub + 1), cap, Q, g_ilu_err) ||
-        ilu_level_host(*P, side ? Q.big_up : Q.big_lo, side ? Q.big_up_ptr : Q.big_lo_ptr, side == 0, S, g_ilu_err))
-        return -1;
+    if (ilu_sliced_host(*P, std::vector<int64_t>(sub_off, sub_off + nsub + 1), cap, Q, g_ilu_err)) return -1;
+    ilu_level_host(*P, side ? Q.big_up : Q.big_lo, side ? Q.big_up_ptr : Q.big_lo_ptr, side == 0, S);
+    std::vector<int32_t> r, c, sr, rsr;
+    if (row || col || src || rsrc) ilu_level_expand(*P, S, side == 0, r, c, sr, rsr);
     sizes[0] = (int64_t)S.lev.size();
-    sizes[1] = (int64_t)S.row.size();
-    sizes[2] = (int64_t)S.col.size();
+    sizes[1] = (int64_t)S.order.size();
+    sizes[2] = S.entries;
     if (levels)
         for (const IluLevel &L : S.lev) {
             for (int64_t v : {(int64_t)L.rows, (int64_t)L.row0, (int64_t)L.lanes, (int64_t)L.nseg}) *levels++ = v;
@@ -120,10 +124,10 @@ int pyhip_ilu_level_copy(const void *h, int nsub, const int64_t *sub_off, int ca
     auto cp = [](auto *dst, const auto &v) {
         if (dst && !v.empty()) std::memcpy(dst, v.data(), v.size() * sizeof(v[0]));
     };
-    cp(row, S.row);
-    cp(col, S.col);
-    cp(src, S.src);
-    cp(rsrc, S.rsrc);
+    cp(row, r);
+    cp(col, c);
+    cp(src, sr);
+    cp(rsrc, rsr);
     return 0;
 }
 

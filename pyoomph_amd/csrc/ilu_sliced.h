@@ -147,17 +147,50 @@ __global__ __launch_bounds__(kIluSlicedThreads) void ilu_sliced_apply_kernel(
     }
 }
 
-// the factor in slice order: val[k] = lu[src[k]] (0 at padding)
-// (or, for the pivots, its reciprocal)
-template <typename T>
-__global__ __launch_bounds__(256) void ilu_sliced_fill_kernel(int64_t n, const int32_t *__restrict__ src,
-                                                              const T *__restrict__ lu, T *__restrict__ val,
-                                                              int reciprocal) {
+// The chunks' columns, rows and marks, once per plan; a thread per (chunk, lane)
+__global__ __launch_bounds__(256) void ilu_sliced_index_kernel(int64_t lanes, const IluChunk *__restrict__ chunk,
+                                                               const int32_t *__restrict__ order,
+                                                               const int32_t *__restrict__ prs,
+                                                               const int32_t *__restrict__ pcol,
+                                                               const int32_t *__restrict__ pdiag,
+                                                               const int32_t *__restrict__ row0,
+                                                               const int32_t *__restrict__ rows, bool lower,
+                                                               ilu_u32x4 *__restrict__ idx) {
     const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    const int32_t s = src[k];
-    const T v = s >= 0 ? lu[s] : T(0);
-    val[k] = reciprocal ? (s >= 0 ? T(1) / v : T(0)) : v;
+    if (k >= lanes) return;
+    const IluChunk C = chunk[k / kIluSliceLanes];
+    const IluLane L = ilu_chunk_lane(C, (int)(k % kIluSliceLanes), order, prs, pdiag, lower);
+    const int32_t r0 = row0[C.slot], dummy = rows[C.slot];
+    uint32_t c[kIluChunk];
+#pragma unroll
+    for (int j = 0; j < kIluChunk; j++) c[j] = (uint32_t)(L.e(j) < L.len ? pcol[L.k0 + L.e(j)] - r0 : dummy);
+    const uint32_t row = L.row >= 0 ? (uint32_t)(L.row - r0) : (uint32_t)kIluNoRow;
+    idx[k] = ilu_u32x4{c[0] | c[1] << 16, c[2] | c[3] << 16, c[4] | c[5] << 16, row | (uint32_t)C.mark << 16};
+}
+
+// The factor in chunk order (0 at padding) and, with rdiag, each lane's reciprocal pivot
+template <typename T>
+__global__ __launch_bounds__(256) void ilu_sliced_fill_kernel(int64_t lanes, const IluChunk *__restrict__ chunk,
+                                                              const int32_t *__restrict__ order,
+                                                              const int32_t *__restrict__ prs,
+                                                              const int32_t *__restrict__ pdiag, bool lower,
+                                                              const T *__restrict__ lu, T *__restrict__ val,
+                                                              T *__restrict__ rdiag) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= lanes) return;
+    const int64_t c = k / kIluSliceLanes;
+    const int lane = (int)(k % kIluSliceLanes);
+    const IluLane L = ilu_chunk_lane(chunk[c], lane, order, prs, pdiag, lower);
+    using P = typename IluPair<T>::type;
+    P *v = (P *)val + c * (kIluChunkVal / 2) + lane;
+#pragma unroll
+    for (int j = 0; j < kIluChunk; j += 2) {
+        P q;
+        q.x = L.e(j) < L.len ? lu[L.k0 + L.e(j)] : T(0);
+        q.y = L.e(j + 1) < L.len ? lu[L.k0 + L.e(j + 1)] : T(0);
+        v[j / 2 * kIluSliceLanes] = q;
+    }
+    if (rdiag) rdiag[k] = L.row >= 0 ? T(1) / lu[pdiag[L.row]] : T(0);
 }
 
 }  // namespace pyhip

@@ -33,16 +33,15 @@ struct IluPlan {
     // sub-problems solved in one workgroup each (ilu_sliced.h); the others level by
     // level (ilu_levels.h)
     struct Side {
-        int32_t *nlev = nullptr, *chunk0 = nullptr, *src = nullptr;
+        int32_t *nlev = nullptr, *chunk0 = nullptr, *order = nullptr;
+        IluChunk *chunk = nullptr;
         uint16_t *idx = nullptr;
-        void *val = nullptr;      // [nval] (T)
-        int64_t nval = 0;
+        void *val = nullptr;      // [chunks * kIluChunkVal] (T)
+        int64_t chunks = 0;
     } slo, sup;
     int nsliced = 0, max_rows = 0;
     int32_t *ssubs = nullptr, *srow0 = nullptr, *srows = nullptr;   // [nsliced]
-    int32_t *sdsrc = nullptr;     // [chunks * 64] pivot of each lane's row in lu (upper side)
-    void *sdiag = nullptr;        // [chunks * 64] reciprocal pivots (T)
-    int64_t ndiag = 0;
+    void *sdiag = nullptr;        // [chunks * 64] reciprocal pivot of each lane's row (upper side, T)
     struct Levels {
         std::vector<IluLevel> lev;
         int32_t *row = nullptr, *col = nullptr, *src = nullptr, *rsrc = nullptr;

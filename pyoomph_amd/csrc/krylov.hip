@@ -663,10 +663,10 @@ constexpr int kGmresCheck = 8;   // GMRES iterations between host reads of the a
 static void ilu_free(KrylovWork *W) {
     IluPlan &L = W->ilu;
     void *ptrs[] = {L.perm, L.rs, L.col, L.src, L.diag, L.lo_rows, L.lu, L.tmp, L.ssubs, L.srow0,
-                    L.srows, L.sdsrc, L.sdiag};
+                    L.srows, L.sdiag};
     for (void *q : ptrs) dfree(q);
     for (IluPlan::Side *S : {&L.slo, &L.sup}) {
-        void *sp[] = {S->nlev, S->chunk0, S->src, S->idx, S->val};
+        void *sp[] = {S->nlev, S->chunk0, S->order, S->chunk, S->idx, S->val};
         for (void *q : sp) dfree(q);
     }
     for (IluPlan::Levels *S : {&L.llo, &L.lup}) {
@@ -753,41 +753,42 @@ static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
         LUP(L.ssubs, Q.subs);
         LUP(L.srow0, Q.row0);
         LUP(L.srows, Q.rows);
-        // the pivot of each lane's row on the upper side
-        std::vector<int32_t> dsrc(Q.up.idx.size() / 8, -1);
-        for (size_t t = 0; t < Q.subs.size(); t++) {
-            const int64_t c0 = Q.up.chunk0[t * kIluSliceWaves], c1 = Q.up.chunk0[(t + 1) * kIluSliceWaves];
-            for (int64_t k = c0 * kIluSliceLanes; k < c1 * kIluSliceLanes; k++) {
-                const uint16_t r = Q.up.idx[k * 8 + kIluChunk];
-                if (r != kIluNoRow) dsrc[k] = H.pdiag[Q.row0[t] + r];
-            }
-        }
-        LUP(L.sdsrc, dsrc);
-        L.ndiag = (int64_t)dsrc.size();
-        auto side = [&](IluPlan::Side &D, const IluSlicedSide &S) -> int {
+        auto side = [&](IluPlan::Side &D, const IluSlicedSide &S, bool lower) -> int {
             LUP(D.nlev, S.nlev);
             LUP(D.chunk0, S.chunk0);
-            LUP(D.src, S.src);
-            LUP(D.idx, S.idx);
-            D.nval = (int64_t)S.src.size();
+            LUP(D.order, S.order);
+            LUP(D.chunk, S.chunk);
+            D.chunks = (int64_t)S.chunk.size();
+            if ((rc = kalloc(&D.idx, (size_t)D.chunks * kIluChunkIdx, W))) return rc;
+            const int64_t lanes = D.chunks * kIluSliceLanes;
+            hipLaunchKernelGGL(ilu_sliced_index_kernel, dim3(nblk(lanes)), dim3(256), 0, p->st, lanes, D.chunk, D.order,
+                               L.rs, L.col, L.diag, L.srow0, L.srows, lower, (ilu_u32x4 *)D.idx);
+            KCHECK();
             return PYHIP_OK;
         };
-        if ((rc = side(L.slo, Q.lo)) || (rc = side(L.sup, Q.up))) return rc;
+        if ((rc = side(L.slo, Q.lo, true)) || (rc = side(L.sup, Q.up, false))) return rc;
     }
     if (!Q.big_lo.empty()) {
+        int64_t once = 0;
         auto levels = [&](IluPlan::Levels &D, const std::vector<int32_t> &rows, const std::vector<int64_t> &ptr,
                           bool lower) -> int {
             IluLevelSide S;
-            if (ilu_level_host(H, rows, ptr, lower, S, err)) {
-                set_error(err);
-                return PYHIP_ERR_INVALID;
-            }
-            LUP(D.row, S.row);
-            LUP(D.col, S.col);
-            LUP(D.src, S.src);
-            LUP(D.rsrc, S.rsrc);
-            D.entries = (int64_t)S.col.size();
-            D.rows = (int64_t)S.row.size();
+            ilu_level_host(H, rows, ptr, lower, S);
+            D.entries = S.entries;
+            D.rows = (int64_t)S.order.size();
+            if ((rc = kalloc(&D.row, D.rows, W)) || (rc = kalloc(&D.rsrc, D.rows, W)) ||
+                (rc = kalloc(&D.col, D.entries, W)) || (rc = kalloc(&D.src, D.entries, W)))
+                return rc;
+            int32_t *order = nullptr;   // read by the layout only
+            if ((rc = dev_alloc(&order, D.rows, once))) return rc;
+            hipError_t e = hipMemcpyAsync(order, S.order.data(), D.rows * sizeof(int32_t), hipMemcpyHostToDevice, p->st);
+            for (const IluLevel &V : S.lev)
+                hipLaunchKernelGGL(ilu_level_layout_kernel, dim3(nblk(8 * (int64_t)V.rows)), dim3(256), 0, p->st, V, order,
+                                   L.rs, L.col, L.diag, L.perm, lower, D.row, D.col, D.src, D.rsrc);
+            if (e == hipSuccess) e = hipGetLastError();
+            if (e == hipSuccess) e = hipStreamSynchronize(p->st);
+            dfree(order);
+            PYHIP_CHECK_HIP(e);
             D.lev = std::move(S.lev);
             return PYHIP_OK;
         };
@@ -816,9 +817,9 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
             *q = nullptr;
         }
         if (L.nsliced) {
-            if ((rc = dev_alloc((T **)&L.slo.val, L.slo.nval, W->bytes)) ||
-                (rc = dev_alloc((T **)&L.sup.val, L.sup.nval, W->bytes)) ||
-                (rc = dev_alloc((T **)&L.sdiag, L.ndiag, W->bytes)))
+            if ((rc = dev_alloc((T **)&L.slo.val, (size_t)L.slo.chunks * kIluChunkVal, W->bytes)) ||
+                (rc = dev_alloc((T **)&L.sup.val, (size_t)L.sup.chunks * kIluChunkVal, W->bytes)) ||
+                (rc = dev_alloc((T **)&L.sdiag, (size_t)L.sup.chunks * kIluSliceLanes, W->bytes)))
                 return rc;
             // The limit belongs to the function, not to this problem: always the largest one, so that
             // other problems' applies, older ones and those of other threads, stay within it.
@@ -848,14 +849,19 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
                            L.lo_rows + L.lo_ptr[l], L.rs, L.col, L.diag, lu, W->nactive_d, L.perm, p->dof_sub,
                            need);
     }
+    auto fill_side = [&](const IluPlan::Side &S, bool lower, T *rdiag) {
+        const int64_t lanes = S.chunks * kIluSliceLanes;
+        if (lanes)
+            hipLaunchKernelGGL((ilu_sliced_fill_kernel<T>), dim3(nblk(lanes)), dim3(256), 0, p->st, lanes, S.chunk,
+                               S.order, L.rs, L.diag, lower, lu, (T *)S.val, rdiag);
+    };
+    fill_side(L.slo, true, nullptr);
+    fill_side(L.sup, false, (T *)L.sdiag);
     auto fill = [&](int64_t m, const int32_t *src, void *val, int reciprocal) {
         if (m)
-            hipLaunchKernelGGL((ilu_sliced_fill_kernel<T>), dim3(nblk(m)), dim3(256), 0, p->st, m, src, lu, (T *)val,
+            hipLaunchKernelGGL((ilu_level_fill_kernel<T>), dim3(nblk(m)), dim3(256), 0, p->st, m, src, lu, (T *)val,
                                reciprocal);
     };
-    fill(L.slo.nval, L.slo.src, L.slo.val, 0);
-    fill(L.sup.nval, L.sup.src, L.sup.val, 0);
-    fill(L.ndiag, L.sdsrc, L.sdiag, 1);
     for (IluPlan::Levels *S : {&L.llo, &L.lup}) {
         fill(S->entries, S->src, S->val, 0);
         fill(S->rows, S->rsrc, S->rdiag, 1);
