@@ -98,29 +98,51 @@ __global__ __launch_bounds__(256) void ilu_level_kernel(IluLevel L, int32_t nfir
     }
 }
 
-// The rows, columns and factor places of one level, once per plan; a thread per (row, stripe)
-__global__ __launch_bounds__(256) void ilu_level_layout_kernel(IluLevel L, const int32_t *__restrict__ order,
-                                                               const int32_t *__restrict__ prs,
-                                                               const int32_t *__restrict__ pcol,
-                                                               const int32_t *__restrict__ pdiag,
-                                                               const int32_t *__restrict__ perm, bool lower,
-                                                               int32_t *__restrict__ row, int32_t *__restrict__ col,
-                                                               int32_t *__restrict__ src, int32_t *__restrict__ rsrc) {
-    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k >= 8 * (int64_t)L.rows) return;
-    ilu_level_stripe(L, (int32_t)(k / 8), (int)(k % 8), order, prs, pcol, pdiag, perm, lower, row, col, src, rsrc);
+// Level of place q in a side's row list (nlev levels, consecutive rows)
+__device__ __forceinline__ const IluLevel &ilu_level_of(const IluLevel *lev, int nlev, int32_t q) {
+    int lo = 0, hi = nlev;   // lev[lo].row0 <= q < lev[hi].row0
+    while (hi - lo > 1) {
+        const int m = (lo + hi) >> 1;
+        if (lev[m].row0 <= q) lo = m;
+        else hi = m;
+    }
+    return lev[lo];
 }
 
-// val[k] = lu[src[k]] (0 at padding), or, for the pivots, its reciprocal
+// The rows and columns of a side, once per plan; a thread per (row, stripe)
+__global__ __launch_bounds__(256) void ilu_level_index_kernel(int64_t stripes, const IluLevel *__restrict__ lev, int nlev,
+                                                              const int32_t *__restrict__ order,
+                                                              const int32_t *__restrict__ prs,
+                                                              const int32_t *__restrict__ pcol,
+                                                              const int32_t *__restrict__ pdiag,
+                                                              const int32_t *__restrict__ perm, bool lower,
+                                                              int32_t *__restrict__ row, int32_t *__restrict__ col) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= stripes) return;
+    const int32_t q = (int32_t)(t / 8), r = order[q];
+    const IluLevel &L = ilu_level_of(lev, nlev, q);
+    const int32_t k0 = lower ? prs[r] : pdiag[r] + 1, n = (lower ? pdiag[r] : prs[r + 1]) - k0;
+    if (t % 8 == 0) row[q] = ilu_level_row(r, prs, pdiag, perm, lower);
+    ilu_level_stripe(L, q - L.row0, (int)(t % 8),
+                     [&](int64_t at, int k) { col[at] = ilu_level_col(r, k0, n, k, pcol, perm); });
+}
+
+// The factor of a side (0 at padding) and each row's reciprocal pivot
 template <typename T>
-__global__ __launch_bounds__(256) void ilu_level_fill_kernel(int64_t n, const int32_t *__restrict__ src,
+__global__ __launch_bounds__(256) void ilu_level_fill_kernel(int64_t stripes, const IluLevel *__restrict__ lev, int nlev,
+                                                             const int32_t *__restrict__ order,
+                                                             const int32_t *__restrict__ prs,
+                                                             const int32_t *__restrict__ pdiag, bool lower,
                                                              const T *__restrict__ lu, T *__restrict__ val,
-                                                             int reciprocal) {
-    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    const int32_t s = src[k];
-    const T v = s >= 0 ? lu[s] : T(0);
-    val[k] = reciprocal ? (s >= 0 ? T(1) / v : T(0)) : v;
+                                                             T *__restrict__ rdiag) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= stripes) return;
+    const int32_t q = (int32_t)(t / 8), r = order[q];
+    const IluLevel &L = ilu_level_of(lev, nlev, q);
+    const int32_t k0 = lower ? prs[r] : pdiag[r] + 1, n = (lower ? pdiag[r] : prs[r + 1]) - k0;
+    if (t % 8 == 0) rdiag[q] = T(1) / lu[pdiag[r]];
+    ilu_level_stripe(L, q - L.row0, (int)(t % 8),
+                     [&](int64_t at, int k) { val[at] = k < n ? lu[k0 + k] : T(0); });
 }
 
 }  // namespace pyhip

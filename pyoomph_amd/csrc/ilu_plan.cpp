@@ -149,6 +149,7 @@ int ilu_plan_host(int64_t n, const int32_t *rs, const int32_t *col, const std::v
 template <typename K>
 static void sort_decreasing(int32_t *b, int32_t *e, K key, std::vector<int32_t> &tmp, std::vector<int32_t> &cnt) {
     const int64_t n = e - b;
+    if (std::is_sorted(b, e, [&](int32_t x, int32_t y) { return key(x) > key(y); })) return;
     int32_t top = 0;
     for (int32_t *r = b; r < e; r++) top = std::max(top, key(*r));
     if (n < 16 || top > 4 * n) {   // few rows, or more counters than rows
@@ -332,6 +333,14 @@ int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, i
         out.rows.push_back((int32_t)(sub_off[s + 1] - sub_off[s]));
         out.max_rows = std::max(out.max_rows, out.rows.back());
     }
+    if (out.subs.empty()) {
+        out.lo.chunk0 = out.up.chunk0 = {0};
+        out.big_lo = H.lo_rows;
+        out.big_up = H.up_rows;
+        out.big_lo_ptr = H.lo_ptr;
+        out.big_up_ptr = H.up_ptr;
+        return 0;
+    }
     int rc = sliced_side(H, H.lo_rows, H.lo_ptr, true, slot_of, out, row_sub, out.lo, out.big_lo,
                          out.big_lo_ptr, err);
     if (!rc)
@@ -340,21 +349,21 @@ int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, i
     return rc;
 }
 
-void ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
-                    bool lower, IluLevelSide &out) {
+void ilu_level_host(const IluHostPlan &H, std::vector<int32_t> rows, const std::vector<int64_t> &ptr, bool lower,
+                    IluLevelSide &out) {
     out = IluLevelSide();
     auto steps_of = [&](int32_t r) {
         const int32_t n = lower ? H.pdiag[r] - H.prs[r] : H.prs[r + 1] - H.pdiag[r] - 1;
         return (n + 7) / 8;
     };
-    out.order = big_rows;
+    out.order = std::move(rows);
     std::vector<int32_t> tmp, cnt;
-    for (size_t l = 0; l + 1 < big_ptr.size(); l++) {
-        int32_t *R = out.order.data() + big_ptr[l];
-        sort_decreasing(R, out.order.data() + big_ptr[l + 1], steps_of, tmp, cnt);
+    for (size_t l = 0; l + 1 < ptr.size(); l++) {
+        int32_t *R = out.order.data() + ptr[l];
+        sort_decreasing(R, out.order.data() + ptr[l + 1], steps_of, tmp, cnt);
         IluLevel L;
-        L.rows = (int32_t)(big_ptr[l + 1] - big_ptr[l]);
-        L.row0 = (int32_t)big_ptr[l];
+        L.rows = (int32_t)(ptr[l + 1] - ptr[l]);
+        L.row0 = (int32_t)ptr[l];
         // narrow levels: more lanes per row, for more loads in flight
         L.lanes = L.rows <= 16384 ? 8 : L.rows <= 65536 ? 4 : 2;
         for (int32_t b = 0; b < L.rows;) {
@@ -380,10 +389,17 @@ void ilu_level_expand(const IluHostPlan &H, const IluLevelSide &S, bool lower, s
     col.resize(S.entries);
     src.resize(S.entries);
     for (const IluLevel &L : S.lev)
-        for (int32_t i = 0; i < L.rows; i++)
+        for (int32_t i = 0; i < L.rows; i++) {
+            const int32_t r = S.order[L.row0 + i], k0 = lower ? H.prs[r] : H.pdiag[r] + 1,
+                          n = (lower ? H.pdiag[r] : H.prs[r + 1]) - k0;
+            row[L.row0 + i] = ilu_level_row(r, H.prs.data(), H.pdiag.data(), H.perm.data(), lower);
+            rsrc[L.row0 + i] = H.pdiag[r];
             for (int st = 0; st < 8; st++)
-                ilu_level_stripe(L, i, st, S.order.data(), H.prs.data(), H.pcol.data(), H.pdiag.data(), H.perm.data(),
-                                 lower, row.data(), col.data(), src.data(), rsrc.data());
+                ilu_level_stripe(L, i, st, [&](int64_t at, int k) {
+                    col[at] = ilu_level_col(r, k0, n, k, H.pcol.data(), H.perm.data());
+                    src[at] = k < n ? k0 + k : -1;
+                });
+        }
 }
 
 }  // namespace pyhip

@@ -135,32 +135,27 @@ struct IluLevelSide {
     std::vector<int32_t> order;              // permuted rows by (level, decreasing steps)
     int64_t entries = 0;
 };
-// Written out, by a kernel (ilu_levels.h) or ilu_level_expand: problem rows (lower: | kIluLast
-// where it applies), problem columns, permuted-pattern index of each entry (-1: padding) and
-// of each row's pivot.
-// big_rows / big_ptr: the permuted rows by level (IluSlicedPlan).
-void ilu_level_host(const IluHostPlan &H, const std::vector<int32_t> &big_rows, const std::vector<int64_t> &big_ptr,
-                    bool lower, IluLevelSide &out);
+// rows / ptr: the permuted rows of the other sub-problems by level (IluSlicedPlan)
+void ilu_level_host(const IluHostPlan &H, std::vector<int32_t> rows, const std::vector<int64_t> &ptr, bool lower,
+                    IluLevelSide &out);
+// Written out, by kernels (ilu_levels.h) or for tests: problem rows (lower: | kIluLast where
+// it applies), problem columns, permuted-pattern index of each entry (-1: padding) and of each
+// row's pivot
 void ilu_level_expand(const IluHostPlan &H, const IluLevelSide &S, bool lower, std::vector<int32_t> &row,
                       std::vector<int32_t> &col, std::vector<int32_t> &src, std::vector<int32_t> &rsrc);
-// one stripe (entries st, st + 8, ...) of the level's row i
-PYHIP_HD inline void ilu_level_stripe(const IluLevel &L, int32_t i, int st, const int32_t *order, const int32_t *prs,
-                                      const int32_t *pcol, const int32_t *pdiag, const int32_t *perm, bool lower,
-                                      int32_t *row, int32_t *col, int32_t *src, int32_t *rsrc) {
-    const int32_t r = order[L.row0 + i], k0 = lower ? prs[r] : pdiag[r] + 1,
-                  n = (lower ? pdiag[r] : prs[r + 1]) - k0;
-    if (st == 0) {
-        const bool last = lower && prs[r + 1] - pdiag[r] == 1;
-        row[L.row0 + i] = last ? (perm[r] | kIluLast) : perm[r];
-        rsrc[L.row0 + i] = pdiag[r];
-    }
+// f(place, k) for the entries st, st + 8, ... of the level's row i, with its row's entries on
+// this side [k0, k0 + n) of the permuted pattern: k < n the row's k-th, else padding
+template <typename F>
+PYHIP_HD inline void ilu_level_stripe(const IluLevel &L, int32_t i, int st, F f) {
     int g = 0;
     while (i >= L.seg_row[g + 1]) g++;
-    for (int k = st; k < 8 * L.steps[g]; k += 8) {
-        const int64_t at = ilu_level_place(L, g, i, k);
-        col[at] = k < n ? perm[pcol[k0 + k]] : n ? perm[pcol[k0]] : perm[r];
-        src[at] = k < n ? k0 + k : -1;
-    }
+    for (int k = st; k < 8 * L.steps[g]; k += 8) f(ilu_level_place(L, g, i, k), k);
+}
+PYHIP_HD inline int32_t ilu_level_col(int32_t r, int32_t k0, int32_t n, int k, const int32_t *pcol, const int32_t *perm) {
+    return perm[k < n ? pcol[k0 + k] : n ? pcol[k0] : r];
+}
+PYHIP_HD inline int32_t ilu_level_row(int32_t r, const int32_t *prs, const int32_t *pdiag, const int32_t *perm, bool lower) {
+    return lower && prs[r + 1] - pdiag[r] == 1 ? (perm[r] | kIluLast) : perm[r];
 }
 
 }  // namespace pyhip

@@ -29,9 +29,11 @@ struct IluPlan {
     std::vector<int64_t> lo_ptr;  // factorisation level boundaries (host)
     void *lu = nullptr;           // [nnz] factor values (T)
     int lu_prec = -1;
-    void *tmp = nullptr;          // [n] (T) lower solve's result (with level-scheduled rows)
     // sub-problems solved in one workgroup each (ilu_sliced.h); the others level by
-    // level (ilu_levels.h)
+    // level (ilu_levels.h). Plan arrays in smem / lmem, factor values in sval / lval: one
+    // allocation each, since a plugin makes and frees a plan for every matrix
+    void *smem = nullptr, *lmem = nullptr, *sval = nullptr, *lval = nullptr;
+    void *tmp = nullptr;          // [n] (T) lower solve's result (with level-scheduled rows)
     struct Side {
         int32_t *nlev = nullptr, *chunk0 = nullptr, *order = nullptr;
         IluChunk *chunk = nullptr;
@@ -44,7 +46,8 @@ struct IluPlan {
     void *sdiag = nullptr;        // [chunks * 64] reciprocal pivot of each lane's row (upper side, T)
     struct Levels {
         std::vector<IluLevel> lev;
-        int32_t *row = nullptr, *col = nullptr, *src = nullptr, *rsrc = nullptr;
+        IluLevel *dlev = nullptr;
+        int32_t *order = nullptr, *row = nullptr, *col = nullptr;
         void *val = nullptr, *rdiag = nullptr;    // (T)
         int64_t entries = 0, rows = 0;
     } llo, lup;
@@ -87,11 +90,12 @@ struct KrylovWork {
     double *partial = nullptr;        // [nchunk][m+2]
     double *dots = nullptr;           // [m+2][nsub]
     // GMRES orthogonalisation (gmres_kernels.h): its chunks and their partial sums
+    void *gs_mem = nullptr;           // the arrays of the chunks
     int64_t *gs_begin = nullptr, *gs_end = nullptr;
     int32_t *gs_sub = nullptr, *gs_ptr = nullptr;
     int64_t gs_count = 0;
     int gs_max = 0;                   // chunks of the largest sub-problem
-    double *gs_part1 = nullptr, *gs_part2 = nullptr;   // [m+1][gs_count]
+    double *gs_part1 = nullptr, *gs_part2 = nullptr;   // [m+1][gs_count], one allocation
     GsChunks gs_chunks() const { return GsChunks{gs_begin, gs_end, gs_sub, gs_ptr, gs_count}; }
     // GMRES state per sub-problem
     double *H = nullptr;              // [nsub][m+1][m]

@@ -401,6 +401,41 @@ static int kalloc(T **p, size_t n, KrylovWork *W) {
     return dev_alloc(p, n, W->bytes);
 }
 
+// Several arrays in one device allocation: host arrays (put, in front) are copied at once
+// where they are small, others (room) only get their place.
+struct DevPack {
+    struct Part {
+        void **dst;
+        const void *src;
+        size_t bytes, at;
+    };
+    std::vector<Part> parts;
+    size_t bytes = 0, copied = 0;
+    void add(void **dst, const void *src, size_t n) {
+        parts.push_back({dst, src, n, bytes});
+        bytes += (n + 255) / 256 * 256;
+        if (src) copied = bytes;
+    }
+    template <typename T>
+    void put(T *&dst, const std::vector<T> &v) { add((void **)&dst, v.data(), v.size() * sizeof(T)); }
+    template <typename T>
+    void room(T *&dst, size_t n) { add((void **)&dst, nullptr, n * sizeof(T)); }
+    int make(void **mem, KrylovWork *W) {
+        int rc;
+        if ((rc = dev_alloc((unsigned char **)mem, bytes, W->bytes))) return rc;
+        std::vector<unsigned char> stage;
+        if (copied <= (1 << 20)) stage.resize(copied);
+        for (const Part &q : parts) {
+            *q.dst = (unsigned char *)*mem + q.at;
+            if (!q.src || !q.bytes) continue;
+            if (!stage.empty()) memcpy(stage.data() + q.at, q.src, q.bytes);
+            else PYHIP_CHECK_HIP(hipMemcpy(*q.dst, q.src, q.bytes, hipMemcpyHostToDevice));
+        }
+        if (!stage.empty()) PYHIP_CHECK_HIP(hipMemcpy(*mem, stage.data(), stage.size(), hipMemcpyHostToDevice));
+        return PYHIP_OK;
+    }
+};
+
 static int krylov_setup(pyhip_problem *p, int m) {
     PYHIP_REQUIRE(m >= 1 && m <= kMaxRestart, "restart must be in 1..1000");
     if (p->kw && p->kw->m >= m) return PYHIP_OK;
@@ -449,10 +484,12 @@ static int krylov_setup(pyhip_problem *p, int m) {
             }
             gptr[p->nsub] = (int32_t)gb.size();
             W->gs_count = (int64_t)gb.size();
-            KUP(W->gs_begin, gb);
-            KUP(W->gs_end, ge);
-            KUP(W->gs_sub, gsub);
-            KUP(W->gs_ptr, gptr);
+            DevPack pk;
+            pk.put(W->gs_begin, gb);
+            pk.put(W->gs_end, ge);
+            pk.put(W->gs_sub, gsub);
+            pk.put(W->gs_ptr, gptr);
+            if ((rc = pk.make(&W->gs_mem, W))) return rc;
         }
 #undef KUP
         const int64_t n = W->n, ns = W->nsub;
@@ -500,7 +537,6 @@ static int krylov_setup(pyhip_problem *p, int m) {
     dfree(W->g);
     dfree(W->y);
     dfree(W->gs_part1);
-    dfree(W->gs_part2);
     dfree(W->V);
     W->V = nullptr;
     W->vprec = -1;
@@ -510,9 +546,9 @@ static int krylov_setup(pyhip_problem *p, int m) {
         (rc = kalloc(&W->dots, (size_t)3 * (m + 2) * ns, W)) ||
         (rc = kalloc(&W->H, (size_t)ns * (m + 1) * m, W)) || (rc = kalloc(&W->cs, (size_t)ns * m, W)) ||
         (rc = kalloc(&W->sn, (size_t)ns * m, W)) || (rc = kalloc(&W->g, (size_t)ns * (m + 1), W)) ||
-        (rc = kalloc(&W->y, (size_t)ns * m, W)) || (rc = kalloc(&W->gs_part1, (size_t)(m + 1) * W->gs_count, W)) ||
-        (rc = kalloc(&W->gs_part2, (size_t)(m + 1) * W->gs_count, W)))
+        (rc = kalloc(&W->y, (size_t)ns * m, W)) || (rc = kalloc(&W->gs_part1, 2 * (size_t)(m + 1) * W->gs_count, W)))
         return rc;
+    W->gs_part2 = W->gs_part1 + (size_t)(m + 1) * W->gs_count;
     W->m = m;
     return PYHIP_OK;
 }
@@ -662,17 +698,8 @@ constexpr int kGmresCheck = 8;   // GMRES iterations between host reads of the a
 
 static void ilu_free(KrylovWork *W) {
     IluPlan &L = W->ilu;
-    void *ptrs[] = {L.perm, L.rs, L.col, L.src, L.diag, L.lo_rows, L.lu, L.tmp, L.ssubs, L.srow0,
-                    L.srows, L.sdiag};
+    void *ptrs[] = {L.perm, L.rs, L.col, L.src, L.diag, L.lo_rows, L.lu, L.smem, L.lmem, L.sval, L.lval};
     for (void *q : ptrs) dfree(q);
-    for (IluPlan::Side *S : {&L.slo, &L.sup}) {
-        void *sp[] = {S->nlev, S->chunk0, S->order, S->chunk, S->idx, S->val};
-        for (void *q : sp) dfree(q);
-    }
-    for (IluPlan::Levels *S : {&L.llo, &L.lup}) {
-        void *sp[] = {S->row, S->col, S->src, S->rsrc, S->val, S->rdiag};
-        for (void *q : sp) dfree(q);
-    }
     L = IluPlan();
 }
 
@@ -749,53 +776,61 @@ static int ilu_plan_build(pyhip_problem *p, KrylovWork *W) {
     LUP(L.src, H.psrc);
     LUP(L.diag, H.pdiag);
     LUP(L.lo_rows, H.lo_rows);
+#undef LUP
     if (L.nsliced) {
-        LUP(L.ssubs, Q.subs);
-        LUP(L.srow0, Q.row0);
-        LUP(L.srows, Q.rows);
-        auto side = [&](IluPlan::Side &D, const IluSlicedSide &S, bool lower) -> int {
-            LUP(D.nlev, S.nlev);
-            LUP(D.chunk0, S.chunk0);
-            LUP(D.order, S.order);
-            LUP(D.chunk, S.chunk);
-            D.chunks = (int64_t)S.chunk.size();
-            if ((rc = kalloc(&D.idx, (size_t)D.chunks * kIluChunkIdx, W))) return rc;
+        L.slo.chunks = (int64_t)Q.lo.chunk.size();
+        L.sup.chunks = (int64_t)Q.up.chunk.size();
+        DevPack pk;
+        pk.put(L.ssubs, Q.subs);
+        pk.put(L.srow0, Q.row0);
+        pk.put(L.srows, Q.rows);
+        auto put = [&](IluPlan::Side &D, const IluSlicedSide &S) {
+            pk.put(D.nlev, S.nlev);
+            pk.put(D.chunk0, S.chunk0);
+            pk.put(D.order, S.order);
+            pk.put(D.chunk, S.chunk);
+        };
+        put(L.slo, Q.lo);
+        put(L.sup, Q.up);
+        pk.room(L.slo.idx, (size_t)L.slo.chunks * kIluChunkIdx);
+        pk.room(L.sup.idx, (size_t)L.sup.chunks * kIluChunkIdx);
+        if ((rc = pk.make(&L.smem, W))) return rc;
+        auto index = [&](const IluPlan::Side &D, bool lower) {
             const int64_t lanes = D.chunks * kIluSliceLanes;
             hipLaunchKernelGGL(ilu_sliced_index_kernel, dim3(nblk(lanes)), dim3(256), 0, p->st, lanes, D.chunk, D.order,
                                L.rs, L.col, L.diag, L.srow0, L.srows, lower, (ilu_u32x4 *)D.idx);
-            KCHECK();
-            return PYHIP_OK;
         };
-        if ((rc = side(L.slo, Q.lo, true)) || (rc = side(L.sup, Q.up, false))) return rc;
+        index(L.slo, true);
+        index(L.sup, false);
+        KCHECK();
     }
     if (!Q.big_lo.empty()) {
-        int64_t once = 0;
-        auto levels = [&](IluPlan::Levels &D, const std::vector<int32_t> &rows, const std::vector<int64_t> &ptr,
-                          bool lower) -> int {
-            IluLevelSide S;
-            ilu_level_host(H, rows, ptr, lower, S);
-            D.entries = S.entries;
+        IluLevelSide lo, up;
+        ilu_level_host(H, std::move(Q.big_lo), Q.big_lo_ptr, true, lo);
+        ilu_level_host(H, std::move(Q.big_up), Q.big_up_ptr, false, up);
+        DevPack pk;
+        auto put = [&](IluPlan::Levels &D, const IluLevelSide &S) {
             D.rows = (int64_t)S.order.size();
-            if ((rc = kalloc(&D.row, D.rows, W)) || (rc = kalloc(&D.rsrc, D.rows, W)) ||
-                (rc = kalloc(&D.col, D.entries, W)) || (rc = kalloc(&D.src, D.entries, W)))
-                return rc;
-            int32_t *order = nullptr;   // read by the layout only
-            if ((rc = dev_alloc(&order, D.rows, once))) return rc;
-            hipError_t e = hipMemcpyAsync(order, S.order.data(), D.rows * sizeof(int32_t), hipMemcpyHostToDevice, p->st);
-            for (const IluLevel &V : S.lev)
-                hipLaunchKernelGGL(ilu_level_layout_kernel, dim3(nblk(8 * (int64_t)V.rows)), dim3(256), 0, p->st, V, order,
-                                   L.rs, L.col, L.diag, L.perm, lower, D.row, D.col, D.src, D.rsrc);
-            if (e == hipSuccess) e = hipGetLastError();
-            if (e == hipSuccess) e = hipStreamSynchronize(p->st);
-            dfree(order);
-            PYHIP_CHECK_HIP(e);
-            D.lev = std::move(S.lev);
-            return PYHIP_OK;
+            D.entries = S.entries;
+            pk.put(D.dlev, S.lev);
+            pk.put(D.order, S.order);
         };
-        if ((rc = levels(L.llo, Q.big_lo, Q.big_lo_ptr, true)) || (rc = levels(L.lup, Q.big_up, Q.big_up_ptr, false)))
-            return rc;
+        put(L.llo, lo);
+        put(L.lup, up);
+        for (IluPlan::Levels *D : {&L.llo, &L.lup}) {
+            pk.room(D->row, D->rows);
+            pk.room(D->col, D->entries);
+        }
+        if ((rc = pk.make(&L.lmem, W))) return rc;
+        auto index = [&](IluPlan::Levels &D, IluLevelSide &S, bool lower) {
+            hipLaunchKernelGGL(ilu_level_index_kernel, dim3(nblk(8 * D.rows)), dim3(256), 0, p->st, 8 * D.rows, D.dlev,
+                               (int)S.lev.size(), D.order, L.rs, L.col, L.diag, L.perm, lower, D.row, D.col);
+            D.lev = std::move(S.lev);
+        };
+        index(L.llo, lo, true);
+        index(L.lup, up, false);
+        KCHECK();
     }
-#undef LUP
     L.n = n;
     L.nnz = p->nnz;
     L.built = true;
@@ -812,15 +847,15 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
         L.lu = nullptr;
         L.lu_prec = -1;
         if ((rc = dev_alloc((T **)&L.lu, L.nnz, W->bytes))) return rc;
-        for (void **q : {&L.slo.val, &L.sup.val, &L.sdiag, &L.llo.val, &L.lup.val, &L.llo.rdiag, &L.lup.rdiag, &L.tmp}) {
-            dfree(*q);
-            *q = nullptr;
-        }
+        dfree(L.sval);
+        dfree(L.lval);
+        L.sval = L.lval = nullptr;
         if (L.nsliced) {
-            if ((rc = dev_alloc((T **)&L.slo.val, (size_t)L.slo.chunks * kIluChunkVal, W->bytes)) ||
-                (rc = dev_alloc((T **)&L.sup.val, (size_t)L.sup.chunks * kIluChunkVal, W->bytes)) ||
-                (rc = dev_alloc((T **)&L.sdiag, (size_t)L.sup.chunks * kIluSliceLanes, W->bytes)))
-                return rc;
+            DevPack pk;
+            pk.room((T *&)L.slo.val, (size_t)L.slo.chunks * kIluChunkVal);
+            pk.room((T *&)L.sup.val, (size_t)L.sup.chunks * kIluChunkVal);
+            pk.room((T *&)L.sdiag, (size_t)L.sup.chunks * kIluSliceLanes);
+            if ((rc = pk.make(&L.sval, W))) return rc;
             // The limit belongs to the function, not to this problem: always the largest one, so that
             // other problems' applies, older ones and those of other threads, stay within it.
             int cap = 0;
@@ -830,11 +865,13 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
                                                 (int)ilu_sliced_lds<T>(cap)));
         }
         if (L.llo.rows) {
-            for (IluPlan::Levels *S : {&L.llo, &L.lup})
-                if ((rc = dev_alloc((T **)&S->val, S->entries, W->bytes)) ||
-                    (rc = dev_alloc((T **)&S->rdiag, S->rows, W->bytes)))
-                    return rc;
-            if ((rc = dev_alloc((T **)&L.tmp, L.n, W->bytes))) return rc;
+            DevPack pk;
+            for (IluPlan::Levels *S : {&L.llo, &L.lup}) {
+                pk.room((T *&)S->val, S->entries);
+                pk.room((T *&)S->rdiag, S->rows);
+            }
+            pk.room((T *&)L.tmp, L.n);
+            if ((rc = pk.make(&L.lval, W))) return rc;
         }
         L.lu_prec = prec;
     }
@@ -857,15 +894,11 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
     };
     fill_side(L.slo, true, nullptr);
     fill_side(L.sup, false, (T *)L.sdiag);
-    auto fill = [&](int64_t m, const int32_t *src, void *val, int reciprocal) {
-        if (m)
-            hipLaunchKernelGGL((ilu_level_fill_kernel<T>), dim3(nblk(m)), dim3(256), 0, p->st, m, src, lu, (T *)val,
-                               reciprocal);
-    };
-    for (IluPlan::Levels *S : {&L.llo, &L.lup}) {
-        fill(S->entries, S->src, S->val, 0);
-        fill(S->rows, S->rsrc, S->rdiag, 1);
-    }
+    for (const IluPlan::Levels *S : {&L.llo, &L.lup})
+        if (S->rows)
+            hipLaunchKernelGGL((ilu_level_fill_kernel<T>), dim3(nblk(8 * S->rows)), dim3(256), 0, p->st, 8 * S->rows,
+                               S->dlev, (int)S->lev.size(), S->order, L.rs, L.diag, S == &L.llo, lu, (T *)S->val,
+                               (T *)S->rdiag);
     KCHECK();
     PYHIP_CHECK_HIP(hipMemcpyAsync(W->nactive_h, W->nactive_d, sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
     PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
@@ -881,8 +914,6 @@ static int ilu_factor(pyhip_problem *p, KrylovWork *W, const TV *vals, const int
 template <typename T>
 static int ilu_apply(pyhip_problem *p, KrylovWork *W, const T *v, T *z, const int32_t *act) {
     IluPlan &L = W->ilu;
-    const T *lu = (const T *)L.lu;
-    const int64_t n = L.n;
     if (L.nsliced) {
         auto dev = [](const IluPlan::Side &S, const T *rdiag) {
             return IluSlicedDev<T>{S.nlev, S.chunk0, S.idx, (const T *)S.val, rdiag};
@@ -2078,7 +2109,7 @@ void pyhip_krylov_free(pyhip_problem *p) {
     KrylovWork *W = p->kw;
     if (!W) return;
     void *ptrs[] = {W->chunk_sub, W->chunk_begin, W->chunk_end, W->sub_chunk_ptr, W->partial, W->dots,
-                    W->gs_begin, W->gs_end, W->gs_sub, W->gs_ptr, W->gs_part1, W->gs_part2, W->H, W->cs, W->sn, W->g, W->beta0, W->bnorm, W->kcols, W->active, W->nactive_d,
+                    W->gs_mem, W->gs_part1, W->H, W->cs, W->sn, W->g, W->beta0, W->bnorm, W->kcols, W->active, W->nactive_d,
                     W->y, W->V, W->r64, W->x64, W->d64, W->b64, W->r32, W->d32, W->w32, W->t32,
                     W->w64, W->t64, W->vals32, W->vals64, W->res64, W->maxres, W->sub_scalar,
                     W->jdiag64, W->jdiag32, W->dof_mask, W->need, W->cg_rz, W->cg_pq,

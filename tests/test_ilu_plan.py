@@ -414,3 +414,31 @@ def test_sliced_plan_of_many_small_problems_costs_about_as_much_as_their_row_ord
         L.pyhip_ilu_plan_free(h)
         assert sz[0] == count
     assert min(sliced) <= 6 * min(order)
+
+
+def test_level_plan_of_a_long_band_costs_less_than_its_row_order():
+    """The level lists of a matrix that no workgroup takes (120000 rows, half bandwidth 2: a
+    plugin factorises such a matrix anew every time): 0.04 of the row order, 0.7 when the
+    padded columns were written by the host."""
+    import time
+    n = 120000
+    A = sp.diags([np.ones(n - abs(k)) for k in range(-2, 3)], range(-2, 3), shape=(n, n)).tocsr()
+    A.sort_indices()
+    rs, col = A.indptr.astype(np.int32), A.indices.astype(np.int32)
+    so, g = np.array([0, n], np.int64), np.zeros(n, np.int8)
+    L, vp = _lib_ilu(), ctypes.c_void_p
+    f = L.pyhip_ilu_level_copy
+    f.argtypes = [vp, ctypes.c_int, _lib.c_i64p, ctypes.c_int, ctypes.c_int, _lib.c_i64p] + [vp] * 5
+    order, level = [], []
+    for _ in range(3):
+        t = time.perf_counter()
+        h = L.pyhip_ilu_plan_new(n, rs.ctypes.data_as(_lib.c_i32p), col.ctypes.data_as(_lib.c_i32p), 1,
+                                 so.ctypes.data_as(_lib.c_i64p), g.ctypes.data_as(ctypes.POINTER(ctypes.c_int8)), AUTO, 64)
+        order.append(time.perf_counter() - t)
+        sz = np.zeros(3, np.int64)
+        t = time.perf_counter()
+        assert f(h, 1, so.ctypes.data_as(_lib.c_i64p), 20000, 0, sz.ctypes.data_as(_lib.c_i64p), *[None] * 5) == 0
+        level.append(time.perf_counter() - t)
+        L.pyhip_ilu_plan_free(h)
+        assert sz[1] == n
+    assert min(level) <= 0.35 * min(order)
