@@ -71,6 +71,17 @@ constexpr int tri_min_elements(bool jac) {
     return jac ? (KIND == ELEM_TRI_P1 ? 0 : 32768) : 65536;
 }
 
+// Bricks that hex_element_kernel takes, n of a launch; the others a thread per row, in FP64 the
+// same bits. A wave's points are a chain of its own, so that few bricks take longer: FP64 matrices, row
+// and wave: 56 and 90 us for 1 brick, 94 and 93 for 8, 120 and 101 for 512; FP64 residuals 22 and
+// 17 us for 1 (its points in one round, as those of 2), 22 and 25 for 8, 25 and 30 for 512 to 2197,
+// 46 and 30 for 2744: the row kernel's workgroups hold 9 bricks, 2304 on the 256 CUs at once.
+// In FP32 one kernel serves every size (a sub-problem has the same bits alone and in a batch).
+template <typename T>
+constexpr bool hex_takes(int n, bool jac) {
+    return sizeof(T) == 4 || (jac ? n >= 8 : n <= 2 || n > 2304);
+}
+
 // TR: the form has a time derivative (a.transient); HV: the matrix output is the
 // Hessian-vector product sum_k dJ_ij/du_k y_k = int d2src (sum_k y_k psi_k) psi_j psi_i
 // (d2src: Bratu -lambda e^u, reaction-diffusion 6u, Poisson 0), symmetric in i, j and k,

@@ -28,7 +28,7 @@ static int launch_scalar(const ElemArgs<T> &a, hipStream_t s) {
         }
     }
     if constexpr (KIND == ELEM_HEX_Q2) {
-        if (!a.hvec && !a.deriv && a.flag < 2) {
+        if (!a.hvec && !a.deriv && a.flag < 2 && hex_takes<T>(a.e1 - a.e0, a.flag)) {
             const dim3 g((a.e1 - a.e0 + kHexPerBlock - 1) / kHexPerBlock), t(64 * kHexWaves);
             // most of a CU's LDS
             auto run = [&](auto *kernel, size_t lds) -> int {

@@ -55,3 +55,37 @@ def test_assembly_at_workgroup_edges(gpu, kind, kw, transient):
     tol = (27 + 16 * kw["N"]) * 2.0**-24
     assert float((v32.double() - v64).abs().max()) <= tol * scale
     assert np.max(np.abs(r32.cpu().numpy() - R)) <= tol * max(scale, np.max(np.abs(R)))
+
+
+@pytest.mark.parametrize("transient", [False, True])
+@pytest.mark.parametrize("cubes", [(1,), (1, 1), (1, 1, 1), (1,) * 7, (2,), (2, 1), (13,), (13, 5), (14,)])
+def test_brick_kernels_meet_at_their_rule(gpu, cubes, transient):
+    """1, 2, 3, 7, 8, 9, 2197, 2322 and 2744 bricks, on both sides of the sizes where the FP64
+    residual and the FP64 matrix change the kernel: the residual alone, the residual beside the
+    matrix and each cube's residual alone in a problem are the same bits."""
+    import torch
+    from pyoomph_amd import workloads as wl
+    from pyoomph_amd.problem import Problem
+    tw = ots.bdf2_weights(0.05, 0.08)
+
+    def assemble(parts, x, h1, h2):
+        P = Problem(parts)
+        P.set_current_dofs(x)
+        if transient:
+            P.set_time_state(tw, *(torch.tensor(h, dtype=torch.float64, device=P.device) for h in (h1, h2)))
+        res, vals = P.assemble_device("f64")
+        torch.cuda.synchronize()
+        return P, P.get_residuals(), res.cpu().numpy(), vals.cpu().numpy()
+
+    parts = [wl.reaction_diffusion_cube(N, seed=i) for i, N in enumerate(cubes)]
+    rng = np.random.default_rng(len(cubes))
+    v = [rng.uniform(-0.4, 0.4, sum((2 * N - 1) ** 3 for N in cubes)) for _ in range(3)]
+    P, only, res, vals = assemble(parts, *v)
+    assert np.array_equal(only, res) and np.isfinite(vals).all()
+    d = e = 0
+    for N, part in zip(cubes, parts):
+        n = (2 * N - 1) ** 3
+        _, o1, r1, v1 = assemble([part], *(x[d:d + n] for x in v))
+        assert np.array_equal(o1, only[d:d + n]) and np.array_equal(r1, res[d:d + n])
+        assert np.array_equal(v1, vals[e:e + v1.size])
+        d, e = d + n, e + v1.size
