@@ -211,8 +211,8 @@ static int sliced_side(const IluHostPlan &H, const std::vector<int32_t> &rows, c
             const int64_t R = e - a;
             const int32_t longest = len(S.order[a]);
             // lanes that still leave the level at most one slice per wave
-            int fill = 1;
-            while (fill < 16 && 2 * fill * R <= kIluSliceLanes * kIluSliceWaves && fill < longest) fill *= 2;
+            int fill = P.tiny[t] ? 4 : 1;
+            while (!P.tiny[t] && fill < 16 && 2 * fill * R <= kIluSliceLanes * kIluSliceWaves && fill < longest) fill *= 2;
             int k = 0;
             for (int64_t b = a; b < e; k++) {
                 int lanes = fill;
@@ -313,13 +313,22 @@ int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, i
             for (int64_t w = ptr[l]; w < ptr[l + 1]; w++) levels[u][row_sub[rows[w]]] = (int32_t)l + 1;
     }
     std::vector<int32_t> order;
+    std::vector<char> tiny(nsub, 0);
+    int64_t ntiny = 0;
     for (int s = 0; s < nsub; s++) {
         const int64_t m = sub_off[s + 1] - sub_off[s];
         const int64_t entries = (int64_t)H.prs[sub_off[s + 1]] - H.prs[sub_off[s]] - m;
-        if (m > 0 && m <= cap && levels[0][s] <= kIluMaxLevels && levels[1][s] <= kIluMaxLevels &&
-            entries <= kIluEntriesPerLevel * (levels[0][s] + levels[1][s]))
-            order.push_back(s);
+        if (m <= 0 || m > cap || levels[0][s] > kIluMaxLevels || levels[1][s] > kIluMaxLevels ||
+            entries > kIluEntriesPerLevel * (levels[0][s] + levels[1][s]))
+            continue;
+        order.push_back(s);
+        tiny[s] = m <= kIluTinyRows;
+        for (int64_t r = sub_off[s]; r < sub_off[s + 1] && tiny[s]; r++)
+            tiny[s] = H.pdiag[r] - H.prs[r] <= 4 * kIluChunk && H.prs[r + 1] - H.pdiag[r] - 1 <= 4 * kIluChunk;
+        ntiny += tiny[s];
     }
+    if (ntiny >= kIluTinyCount)
+        order.erase(std::remove_if(order.begin(), order.end(), [&](int32_t s) { return tiny[s] != 0; }), order.end());
     // longest first: the last workgroups to start are the shortest
     std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
         return sub_off[a + 1] - sub_off[a] > sub_off[b + 1] - sub_off[b];
@@ -331,6 +340,7 @@ int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, i
         out.subs.push_back(s);
         out.row0.push_back((int32_t)sub_off[s]);
         out.rows.push_back((int32_t)(sub_off[s + 1] - sub_off[s]));
+        out.tiny.push_back(tiny[s]);
         out.max_rows = std::max(out.max_rows, out.rows.back());
     }
     if (out.subs.empty()) {

@@ -75,6 +75,7 @@ struct IluSlicedPlan {
     std::vector<int32_t> big_lo, big_up;     // rows of the other sub-problems by level (as lo_rows / up_rows)
     std::vector<int64_t> big_lo_ptr, big_up_ptr;
     int max_rows = 0;                        // largest handled sub-problem
+    std::vector<char> tiny;                  // [handled] four lanes a row, see ilu_sliced_host
 };
 
 // Lane `lane` of a chunk: its permuted row (-1: none), the row's entries on this side
@@ -97,12 +98,21 @@ PYHIP_HD inline IluLane ilu_chunk_lane(const IluChunk &C, int lane, const int32_
 
 // The sliced plan of H (ilu_plan_host); cap < 65535. A sub-problem is handled if it has at
 // most cap rows and kIluMaxLevels levels on each side, and at most kIluEntriesPerLevel
-// triangle entries per level (both sides): one CU takes about 0.28 us per 1000 entries
+// triangle entries per level (both sides; but see tiny ones): one CU takes about 0.28 us per 1000 entries
 // (P2 Poisson 41^2, 67 k entries in 7 + 7 levels: 22 us; 64^2, 166 k in 7 + 7: 47 us;
 // Taylor-Hood 26^2, 223 k in 23 + 23: 58 us), a launch per level about 3 us (42, 42 and
 // 150 us). Decided per sub-problem, so that its solve is the same alone and in any batch.
+// Tiny sub-problems, of at most kIluTinyRows rows with at most 4 kIluChunk entries a side,
+// always take four lanes a row: a lane's two running sums are then two of the level kernels'
+// stripes, combined by the same tree, so that the level launches give the same bits and may serve
+// them. They do for kIluTinyCount of them or more, since a workgroup takes its own
+// chain of levels, 512 at a time on the 256 CUs, where a launch takes a level of all of them: Newton
+// solves of 2048 / 4096 with 49 rows 6.6 / 12.6 ms by workgroups, 6.5 / 8.1 by launches; with 121
+// rows 10.3 / 19.4 and 11.2 / 16.1; with 225 rows (P2) 21.8 / 41.6 and 30.5 / 38.2.
 // Returns 0 or -1 (err).
 constexpr int64_t kIluEntriesPerLevel = 10000;
+constexpr int kIluTinyRows = 256;
+constexpr int kIluTinyCount = 3072;
 int ilu_sliced_host(const IluHostPlan &H, const std::vector<int64_t> &sub_off, int cap, IluSlicedPlan &out,
                     std::string &err);
 // idx and, as indices in the permuted pattern (-1: none), val of a side

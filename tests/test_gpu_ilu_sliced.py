@@ -71,3 +71,17 @@ def test_large_problem_solves_again_after_a_small_one(gpu, precision):
     x = solve(large)
     solve(small)
     assert np.array_equal(x, solve(large))
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("N,space", [(2, "C1"), (4, "C2"), (8, "C1")])
+def test_tiny_problems_have_the_same_bits_in_workgroups_and_level_launches(gpu, N, space, precision):
+    """3072 tiny sub-problems share the level launches; a few of them take a workgroup each."""
+    from pyoomph_amd import workloads as wl
+    few = [wl.bratu(N, space, 0.5 + 0.7 * i) for i in range(4)]
+    # a larger one beside them keeps its workgroup
+    want = _solve(few, precision)
+    got = _solve(few * 768 + [wl.bratu(20, "C2", 1.0)], precision)
+    for i in (0, 1, 2, 3, 1536, 3071):
+        assert np.array_equal(got[i], want[i % 4])
+    assert np.array_equal(got[-1], _solve([wl.bratu(20, "C2", 1.0)], precision)[0])

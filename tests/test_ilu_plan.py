@@ -394,7 +394,7 @@ def test_sliced_plan_of_many_small_problems_costs_about_as_much_as_their_row_ord
     the padded arrays written by the host it took 28 times the row order here, now 0.5."""
     import time
     A, off, grp = _batch([oracle_problem("bratu", N=8, space="C1", lam=1.0)])
-    n, count = A.shape[0], 2048
+    n, count = A.shape[0], 2048   # fewer than take the level lists
     rs = np.concatenate([A.indptr[:-1] + i * A.nnz for i in range(count)] + [[A.nnz * count]]).astype(np.int32)
     col = np.concatenate([A.indices + i * n for i in range(count)]).astype(np.int32)
     so, g = np.arange(count + 1, dtype=np.int64) * n, np.tile(grp, count).astype(np.int8)
@@ -442,3 +442,23 @@ def test_level_plan_of_a_long_band_costs_less_than_its_row_order():
         L.pyhip_ilu_plan_free(h)
         assert sz[1] == n
     assert min(level) <= 0.35 * min(order)
+
+
+@pytest.mark.parametrize("kind,kw,tiny", [("bratu", dict(N=4, space="C1", lam=1.0), True),
+                                          ("poisson", dict(N=4), True), ("ns", dict(N=2), False)])
+def test_many_tiny_problems_take_the_level_lists(kind, kw, tiny):
+    """3072 sub-problems of at most 256 short rows share the level launches, 3071 take a
+    workgroup each, and so do rows of more than 24 entries a side; every slice of a tiny one
+    has four lanes a row (the sums of the level kernels)."""
+    A, off, grp = _batch([oracle_problem(kind, **kw)])
+    n = A.shape[0]
+    for count in (3071, 3072):
+        B = sp.csr_matrix((np.ones(A.nnz * count), np.tile(A.indices, count) + np.repeat(np.arange(count) * n, A.nnz),
+                           np.concatenate([A.indptr[:-1] + i * A.nnz for i in range(count)] + [[A.nnz * count]])),
+                          shape=(n * count, n * count))
+        S = _sliced((B, np.tile(grp, count), AUTO), np.arange(count + 1) * n, 20000, 0)
+        assert len(S["subs"]) == (0 if tiny and count == 3072 else count)
+        assert len(S["big"]) == n * (count - len(S["subs"]))
+        if tiny and len(S["subs"]):
+            rows = S["idx"][:, :, 6] != 0xffff
+            assert set((S["idx"][rows.any(1), 0, 7] >> 12) & 7) == {2}
