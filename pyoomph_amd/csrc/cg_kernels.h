@@ -17,6 +17,7 @@
 namespace pyhip {
 
 constexpr int kCgThreads = 256;
+constexpr int kGsFusedChunks = 640;   // the blocks of a longer sub-problem would read over 5 KB each
 
 // sum over the block's 256 threads: wave trees, then the waves in order; in thread 0
 __device__ __forceinline__ double cg_block_sum(double v, double *sh) {

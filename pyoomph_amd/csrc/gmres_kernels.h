@@ -8,11 +8,12 @@
 // sub-problem's rows, so that small systems still spread over many CUs and a sub-problem's
 // sums are the same alone and in any batch). The partials of a reduction are summed by every
 // block that needs the result (lane-strided over the sub-problem's chunks, then an xor tree)
-// instead of by a launch of its own, up to kGsFusedChunks chunks per sub-problem: reading
-// chunks x vectors x 8 bytes per block costs less than a launch there. Launches with nothing
-// but such sums, counters and single-thread loops took 25 us of an iteration.
-// Bound: reading V three times per iteration (once per pass; the second read of pass 2
-// comes from L2), in 16-byte loads; launch latency for small systems.
+// instead of by a launch of its own, up to kGsFusedPartials values a block; beyond, a launch of
+// gs_reduce adds them in the same order. Launches with nothing but such sums, counters and
+// single-thread loops took 25 us of an iteration.
+// Bound: reading V three times per iteration (once per pass and a second time in pass 2, from
+// L2 where the resident blocks' chunks of V fit it: 64 blocks an XCD, so up to some 30 vectors of
+// 256 rows), in 16-byte loads; launch latency for small systems.
 #pragma once
 #include "common.h"
 
@@ -20,7 +21,11 @@ namespace pyhip {
 
 constexpr int kGsThreads = 1024, kGsWaves = kGsThreads / 64;
 constexpr int kGsMaxRows = 1024;
-constexpr int kGsFusedChunks = 640;
+// Most partials (chunks x vectors) of a sub-problem that every block adds up for itself. 300
+// iterations of GMRES(100) / GMRES(30), summed by the blocks and by launches: 16129 rows (64
+// chunks) 10.9 / 9.2 and 11.6 / 10.9 ms; 64516 (127) 13.7 / 9.5 and 13.3 / 10.3; 129600 (254)
+// 20.2 / 11.1 and 18.7 / 11.7; 622521 (608) 79.9 / 32.9 and 70.2 / 30.8.
+constexpr int kGsFusedPartials = 8192;
 
 inline int gs_chunk_rows(int64_t rows) { return rows <= 32768 ? 256 : rows <= 131072 ? 512 : 1024; }
 
@@ -174,8 +179,8 @@ inline size_t gs_update_lds(int nvec, size_t esize) {
            (size_t)(nvec > kGsWaves ? nvec : kGsWaves) * sizeof(double);
 }
 
-// out[j][s] = sum over the chunks of s of part[j][chunk] (sub-problems of more than
-// kGsFusedChunks chunks), one wave per (j, s)
+// out[j][s] = sum over the chunks of s of part[j][chunk] (above kGsFusedPartials), one wave
+// per (j, s)
 __global__ __launch_bounds__(64) void gs_reduce_kernel(int nsub, GsChunks C, const int32_t *__restrict__ active,
                                                        const double *__restrict__ part, double *__restrict__ out) {
     const int j = blockIdx.x / nsub, s = blockIdx.x % nsub;

@@ -1290,7 +1290,6 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     // filtered launches; the device flags decide which rows are computed)
     int32_t *act_h = W->act_h;
     const GsChunks C = W->gs_chunks();
-    const bool reduced = W->gs_max > kGsFusedChunks;
     PYHIP_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gs_backsolve_kernel),
                                         hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)gs_backsolve_lds(kMaxRestart, kMaxRestart)));   // as any solve sets it
@@ -1326,6 +1325,7 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
                 TimeScope tsu(&p->timer, "vector", p->st);
                 const dim3 grid((unsigned)C.count), thr(kGsThreads);
                 const size_t lds = gs_update_lds(k + 1, sizeof(T));
+                const bool reduced = (int64_t)W->gs_max * (k + 1) > kGsFusedPartials;
                 auto reduce = [&](const double *part, double *out) {
                     if (reduced)
                         hipLaunchKernelGGL(gs_reduce_kernel, dim3((unsigned)((k + 1) * ns)), dim3(64), 0, p->st, ns, C,

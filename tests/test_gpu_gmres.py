@@ -54,3 +54,20 @@ def test_gmres_batch_with_different_chunk_lengths_equals_alone(gpu, opts):
         parts = [wl.bratu(9, "C1", 1.0), wl.bratu(30, "C2", 2.0)]
     for mp, x in zip(parts, solve(parts)):
         assert np.array_equal(x, solve([mp])[0])
+
+
+def test_sums_by_blocks_and_by_launches_have_the_same_bits(gpu):
+    """3481 rows (14 chunks: every block adds up the partials), alone and beside 297025 rows (291
+    chunks: launches add them from 29 vectors on), with more than 29 iterations."""
+    from pyoomph_amd import workloads as wl
+    from pyoomph_amd.problem import Problem
+
+    def solve(parts):
+        P = Problem(parts)
+        P.krylov, P.preconditioner, P.gmres_restart, P.gmres_max_iters = "gmres", "ilu0", 60, 20000
+        st = P.solve()
+        assert all(s["converged"] for s in st) and st[0]["linear_iters"] > 2 * 29
+        return P.sub_dofs(0, P.get_current_dofs())
+
+    small = wl.bratu(60, "C1", 1.5)
+    assert np.array_equal(solve([small]), solve([small, wl.bratu(546, "C1", 1.0)]))
