@@ -808,12 +808,12 @@ __global__ __launch_bounds__(kThThreads) void th_node_kernel(ElemArgs<T> a) {
     }
 }
 
-// Taylor-Hood Q2/Q1 steady Navier-Stokes (22 slots, 9 geometric nodes). Phase A: thread
-// t < 9 of an element computes integration point t (geometry, dx_shape, u, grad u, p);
-// phase B: thread = slot row.
+// Mass matrices (flag 2) and Hessian-vector products (HV) of the Taylor-Hood Q2/Q1 Navier-Stokes
+// form, each beside the residual (22 slots, 9 geometric nodes). Phase A: thread t < 9 of an element
+// computes integration point t (geometry, dx_shape, u, grad u, p); phase B: thread = slot row.
 // TR: time derivative of the velocities (a.transient): du/dt = tw0 u + sum_l H psi_l with
-// H = tw1 u(t-1) + tw2 u(t-2) per slot; momentum rows gain (rho du/dt) psi_i, the diagonal
-// velocity blocks tw0 rho psi_j psi_i; flag 2 writes the mass matrix rho psi_j psi_i there.
+// H = tw1 u(t-1) + tw2 u(t-2) per slot; momentum rows gain (rho du/dt) psi_i, and the mass
+// matrix is rho psi_j psi_i on the diagonal velocity blocks (none without TR).
 template <typename T, bool TR, bool HV = false>
 __global__ __launch_bounds__(256) void th_element_kernel(ElemArgs<T> a) {
     constexpr int NN = 9, DIM = 2, NQ = 9, NS = 22;
@@ -980,29 +980,9 @@ __global__ __launch_bounds__(256) void th_element_kernel(ElemArgs<T> a) {
                     } else {
                         continue;
                     }
-                } else if (a.flag == 2) {
+                } else {
                     if (kt < 2 && kt == ks) v = W * ((rho * P[ls]) * P[lt]);
                     else continue;
-                } else if (kt < 2 && ks < 2) {
-                    const T *dxs = sDx[le][q][ls];
-                    T visc = dxs[kt] * dxl[ks];
-                    T cv = P[ls] * du[kt][ks];
-                    if (kt == ks) {
-                        visc = (dxs[0] * dxl[0] + dxs[1] * dxl[1]) + visc;
-                        cv = cv + (u0 * dxs[0] + u1 * dxs[1]);
-                    }
-                    if (TR && kt == ks)
-                        v = W * ((mu * visc + (rho * cv) * P[lt]) + ((rho * T(a.tw0)) * P[ls]) * P[lt]);
-                    else
-                        v = W * (mu * visc + (rho * cv) * P[lt]);
-                } else if (kt < 2 && ks == 2) {
-                    const int pidx = kTHSlotP[ss];
-                    v = W * (-(C[pidx] * dxl[kt]));
-                } else if (kt == 2 && ks < 2) {
-                    const int pidx = kTHSlotP[slot];
-                    v = W * (sDx[le][q][ls][ks] * C[pidx]);
-                } else {
-                    continue;
                 }
                 Jacc[ss] = Jacc[ss] + v;
             }

@@ -87,7 +87,7 @@ struct KrylovWork {
     int64_t *chunk_begin = nullptr;   // [nchunk+1] (row ranges; chunk c = [begin[c], end[c]))
     int64_t *chunk_end = nullptr;
     int32_t *sub_chunk_ptr = nullptr; // [nsub+1]
-    double *partial = nullptr;        // [nchunk][m+2]
+    double *partial = nullptr;        // [nchunk] (largest entries)
     double *dots = nullptr;           // [m+2][nsub]
     // GMRES orthogonalisation (gmres_kernels.h): its chunks and their partial sums
     void *gs_mem = nullptr;           // the arrays of the chunks

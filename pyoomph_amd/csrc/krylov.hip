@@ -2,16 +2,17 @@
 //
 // Every vector spans all sub-problems of a problem (block-diagonal system). Every scalar
 // (dot products, norms, Hessenberg entries, Givens rotations, convergence state) is per
-// sub-problem. Reductions are two-level and deterministic: fixed 1024-row chunks that
-// never straddle a sub-problem, a fixed-tree block reduction per chunk, then a
-// sequential sum of a sub-problem's chunk partials in chunk order. A sub-problem's
-// arithmetic therefore depends only on its own data: it gives the same bits alone and in
-// any batch.
+// sub-problem. Reductions are two-level and deterministic, on chunks that never straddle a
+// sub-problem: GMRES and preconditioned CG in the order of gmres_kernels.h and cg_kernels.h
+// (256, 512 or 1024 rows by the sub-problem's rows, partials lane-strided, then an xor tree), the
+// work-list CG on fixed 1024-row chunks. A sub-problem's arithmetic therefore depends only on
+// its own data: it gives the same bits alone and in any batch.
 //
 // GMRES(m) with right preconditioning and classical Gram-Schmidt with one
-// re-orthogonalisation (CGS2); Hessenberg least squares by Givens rotations on the
-// device (one thread per sub-problem). The host reads one counter per iteration (the
-// number of sub-problems still iterating).
+// re-orthogonalisation (CGS2); Hessenberg least squares by Givens rotations on the device (in
+// the last orthogonalisation launch, by each sub-problem's first block). The host reads the
+// flags of the sub-problems every kGmresCheck iterations, in preconditioned CG every kPcgRead
+// to kPcgReadMax.
 //
 // Preconditioners: Jacobi, and ILU(0) on the structural pattern, level-scheduled (rows of
 // one level are independent). Its solves run in one workgroup per small sub-problem
@@ -35,41 +36,11 @@ namespace pyhip {
 // ------------------------------------------------------------------------------------
 // kernels
 
-// partial[c][j] = sum over chunk c of V_j . w, for the vectors j of block column
-// blockIdx.y (kDotVecs of them): wave q of the block takes j = q, q + 4, ...; its lanes
-// stride the chunk's rows, and the wave sums them with a fixed xor-shuffle tree.
-constexpr int kDotVecs = 16;
-template <typename T>
-__global__ __launch_bounds__(256) void multidot_kernel(int nvec, const T *__restrict__ V,
-                                                      int64_t ldv, const T *__restrict__ w,
-                                                      const int64_t *__restrict__ cb,
-                                                      const int64_t *__restrict__ ce,
-                                                      double *__restrict__ partial, int pstride,
-                                                      const int32_t *__restrict__ csub,
-                                                      const int32_t *__restrict__ act) {
-    const int64_t c = blockIdx.x;
-    // chunks of sub-problems that stopped (act[csub] == 0) are skipped: their partials are
-    // left as they are and nothing reads their sums
-    if (act && !act[csub[c]]) return;
-    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int64_t b0 = cb[c], b1 = ce[c];
-    for (int jj = q; jj < kDotVecs; jj += 4) {
-        const int j = blockIdx.y * kDotVecs + jj;
-        if (j >= nvec) break;
-        const T *v = V + (int64_t)j * ldv;
-        double acc = 0.0;
-#pragma unroll 4
-        for (int64_t i = b0 + lane; i < b1; i += 64) acc += double(v[i]) * double(w[i]);
-        for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if (lane == 0) partial[c * pstride + j] = acc;
-    }
-}
-
 // max |v| per chunk (non-finite -> +inf), DoubleVector::max (double_vector.cc:611-630)
 __global__ __launch_bounds__(256) void maxabs_kernel(const double *__restrict__ v,
                                                     const int64_t *__restrict__ cb,
                                                     const int64_t *__restrict__ ce,
-                                                    double *__restrict__ partial, int pstride) {
+                                                    double *__restrict__ partial) {
     __shared__ double red[256];
     const int64_t c = blockIdx.x;
     double m = 0.0;
@@ -84,27 +55,18 @@ __global__ __launch_bounds__(256) void maxabs_kernel(const double *__restrict__ 
         if (threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[c * pstride] = red[0];
+    if (threadIdx.x == 0) partial[c] = red[0];
 }
 
-// out[j][s] = sum (or max) of the chunk partials of sub-problem s, vector j: one 64-lane
-// block per (j, s); lane t takes chunks t, t+64, ... in order, then a fixed xor tree.
-__global__ __launch_bounds__(64) void reduce_partials_kernel(int nvec, int nsub,
-                                                            const int32_t *__restrict__ scp,
-                                                            const double *__restrict__ partial,
-                                                            int pstride, double *__restrict__ out,
-                                                            int is_max) {
-    const int j = blockIdx.x / nsub, s = blockIdx.x % nsub;
+// out[s] = max of the chunk partials of sub-problem s, one wave each
+__global__ __launch_bounds__(64) void reduce_max_kernel(const int32_t *__restrict__ scp,
+                                                        const double *__restrict__ partial,
+                                                        double *__restrict__ out) {
+    const int s = blockIdx.x;
     double acc = 0.0;
-    for (int c = scp[s] + threadIdx.x; c < scp[s + 1]; c += 64) {
-        const double v = partial[(int64_t)c * pstride + j];
-        acc = is_max ? fmax(acc, v) : acc + v;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const double o = __shfl_xor(acc, off, 64);
-        acc = is_max ? fmax(acc, o) : acc + o;
-    }
-    if (threadIdx.x == 0) out[j * nsub + s] = acc;
+    for (int c = scp[s] + threadIdx.x; c < scp[s + 1]; c += 64) acc = fmax(acc, partial[c]);
+    for (int off = 32; off > 0; off >>= 1) acc = fmax(acc, __shfl_xor(acc, off, 64));
+    if (threadIdx.x == 0) out[s] = acc;
 }
 
 // out = in * (1 / nrm[sub]) (0 where nrm == 0); only active sub-problems
@@ -513,7 +475,7 @@ static int krylov_setup(pyhip_problem *p, int m) {
             W->sub_nnz_h[s] = (int64_t)p->row_start_h[p->dof_off_h[s + 1]] - p->row_start_h[p->dof_off_h[s]];
         const size_t ngp = (size_t)3 * W->nchunk * kWlBlocksPerChunk;
         if ((rc = kalloc(&W->achunk, std::max<int64_t>(1, W->nchunk), W)) ||
-            (rc = kalloc(&W->gpart, ngp, W)) || (rc = kalloc(&W->cg_iters, ns, W)) ||
+            (rc = kalloc(&W->partial, W->nchunk, W)) || (rc = kalloc(&W->gpart, ngp, W)) || (rc = kalloc(&W->cg_iters, ns, W)) ||
             (rc = kalloc(&W->cg_iters2, ns, W)) ||
             (rc = kalloc(&W->cg_fail, ns, W)))
             return rc;
@@ -529,7 +491,6 @@ static int krylov_setup(pyhip_problem *p, int m) {
     }
     // restart-length dependent buffers
     int rc;
-    dfree(W->partial);
     dfree(W->dots);
     dfree(W->H);
     dfree(W->cs);
@@ -542,8 +503,7 @@ static int krylov_setup(pyhip_problem *p, int m) {
     W->vprec = -1;
     W->vcount = 0;
     const int64_t ns = W->nsub;
-    if ((rc = kalloc(&W->partial, (size_t)W->nchunk * (m + 2) + 1, W)) ||
-        (rc = kalloc(&W->dots, (size_t)3 * (m + 2) * ns, W)) ||
+    if ((rc = kalloc(&W->dots, (size_t)3 * (m + 2) * ns, W)) ||
         (rc = kalloc(&W->H, (size_t)ns * (m + 1) * m, W)) || (rc = kalloc(&W->cs, (size_t)ns * m, W)) ||
         (rc = kalloc(&W->sn, (size_t)ns * m, W)) || (rc = kalloc(&W->g, (size_t)ns * (m + 1), W)) ||
         (rc = kalloc(&W->y, (size_t)ns * m, W)) || (rc = kalloc(&W->gs_part1, 2 * (size_t)(m + 1) * W->gs_count, W)))
@@ -569,34 +529,31 @@ static int ensure_basis(KrylovWork *W, int64_t n, int nvec) {
     return PYHIP_OK;
 }
 
-// Per-sub-problem dot products of nvec vectors with w: out[j][sub].
+// Per-sub-problem dot products out[s] = (a, b) and, with c given, out[nsub + s] = (c, d), on the
+// chunks and in the order of the CG sums (cg_kernels.h). Overwrites gs_part1.
 template <typename T>
-// With act (device [nsub]) the chunks of sub-problems with act[s] == 0 are skipped and
-// their sums are not defined.
-static int batched_dots(pyhip_problem *p, KrylovWork *W, int nvec, const T *V, int64_t ldv,
-                        const T *w, double *out, const int32_t *act = nullptr) {
+static int batched_dots(pyhip_problem *p, KrylovWork *W, const T *a, const T *b, double *out, const T *c = nullptr,
+                        const T *d = nullptr) {
     TimeScope ts(&p->timer, "vector", p->st);
-    const int pstride = W->m + 2;
-    if (W->nchunk == 0) return PYHIP_OK;
-    hipLaunchKernelGGL((multidot_kernel<T>), dim3((unsigned)W->nchunk, (unsigned)((nvec + kDotVecs - 1) / kDotVecs)),
-                       dim3(256), 0, p->st, nvec,
-                       V, ldv, w, W->chunk_begin, W->chunk_end, W->partial, pstride, W->chunk_sub, act);
+    const GsChunks C = W->gs_chunks();
+    if (C.count == 0) return PYHIP_OK;
+    hipLaunchKernelGGL((cg_dots_kernel<T>), dim3((unsigned)C.count), dim3(kCgThreads), 0, p->st, a, b, c, d, C,
+                       (const int32_t *)nullptr, W->gs_part1);
     KCHECK();
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((unsigned)(nvec * W->nsub)), dim3(64), 0, p->st, nvec,
-                       W->nsub, W->sub_chunk_ptr, W->partial, pstride, out, 0);
+    hipLaunchKernelGGL(cg_sums_kernel, dim3((unsigned)((c ? 2 : 1) * W->nsub)), dim3(64), 0, p->st, W->nsub, C,
+                       (const int32_t *)nullptr, W->gs_part1, out);
     KCHECK();
     return PYHIP_OK;
 }
 
 int batched_maxabs(pyhip_problem *p, const double *v, double *out) {
     KrylovWork *W = p->kw;
-    const int pstride = W->m + 2;
     if (W->nchunk == 0) return PYHIP_OK;
     hipLaunchKernelGGL(maxabs_kernel, dim3((unsigned)W->nchunk), dim3(256), 0, p->st, v,
-                       W->chunk_begin, W->chunk_end, W->partial, pstride);
+                       W->chunk_begin, W->chunk_end, W->partial);
     KCHECK();
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((unsigned)W->nsub), dim3(64), 0, p->st, 1, W->nsub,
-                       W->sub_chunk_ptr, W->partial, pstride, out, 1);
+    hipLaunchKernelGGL(reduce_max_kernel, dim3((unsigned)W->nsub), dim3(64), 0, p->st, W->sub_chunk_ptr, W->partial,
+                       out);
     KCHECK();
     return PYHIP_OK;
 }
@@ -1280,7 +1237,7 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     T *t = std::is_same<T, float>::value ? (T *)W->t32 : (T *)W->t64;
     double *d1 = W->dots, *d2 = W->dots + (m + 2) * ns, *d3 = W->dots + 2 * (m + 2) * ns;
     // |b| per sub-problem
-    if ((rc = batched_dots<T>(p, W, 1, b, n, b, d3))) return rc;
+    if ((rc = batched_dots<T>(p, W, b, b, d3))) return rc;
     hipLaunchKernelGGL(sqrt_copy_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, d3, W->bnorm);
     KCHECK();
     // x0 = 0
@@ -1298,7 +1255,7 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     for (int cyc = 0; cyc < max_cycles; cyc++) {
         // r = b - A x  -> V_0 (unnormalised)
         if ((rc = spmv<TV, T, T>(p, vals, x, V, b))) return rc;
-        if ((rc = batched_dots<T>(p, W, 1, V, n, V, d3))) return rc;
+        if ((rc = batched_dots<T>(p, W, V, V, d3))) return rc;
         hipLaunchKernelGGL(gmres_start_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, d3,
                            W->bnorm, rtol, stag, cyc == 0 ? 1 : 0, need, W->g, W->active, W->kcols, W->beta0);
         KCHECK();
@@ -1366,7 +1323,7 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
     }
     // sub-problems still above tolerance (true residual of the returned x)
     if ((rc = spmv<TV, T, T>(p, vals, x, V, b))) return rc;
-    if ((rc = batched_dots<T>(p, W, 1, V, n, V, d3))) return rc;
+    if ((rc = batched_dots<T>(p, W, V, V, d3))) return rc;
     hipLaunchKernelGGL(gmres_start_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, m, d3, W->bnorm,
                        rtol * 1.01, 0.0, 1, need, W->g, W->active, W->kcols, W->beta0);
     KCHECK();
@@ -1381,38 +1338,6 @@ static int gmres(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *b, T 
 
 
 // ---- preconditioned conjugate gradients (symmetric positive definite systems) ----------
-
-template <typename T>
-__global__ __launch_bounds__(256) void dot2_kernel(const T *__restrict__ a, const T *__restrict__ b,
-                                                   const T *__restrict__ c, const T *__restrict__ d,
-                                                   const int64_t *__restrict__ cb,
-                                                   const int64_t *__restrict__ ce,
-                                                   double *__restrict__ partial, int pstride,
-                                                   const int32_t *__restrict__ csub,
-                                                   const int32_t *__restrict__ act) {
-    __shared__ double r0[256], r1[256];
-    const int64_t ch = blockIdx.x;
-    if (act && !act[csub[ch]]) return;   // a stopped sub-problem's chunk (whole block)
-    double s0 = 0.0, s1 = 0.0;
-    for (int64_t i = cb[ch] + threadIdx.x; i < ce[ch]; i += 256) {
-        s0 += double(a[i]) * double(b[i]);
-        s1 += double(c[i]) * double(d[i]);
-    }
-    r0[threadIdx.x] = s0;
-    r1[threadIdx.x] = s1;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            r0[threadIdx.x] += r0[threadIdx.x + s];
-            r1[threadIdx.x] += r1[threadIdx.x + s];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        partial[ch * pstride] = r0[0];
-        partial[ch * pstride + 1] = r1[0];
-    }
-}
 
 // preconditioned-CG iterations between host reads of the flags: at least kPcgRead, an eighth
 // of the iterations done so far up to kPcgReadMax (a read leaves the GPU idle for ~10 us; the
@@ -1434,21 +1359,6 @@ __global__ void cg_start_kernel(int nsub, const double *__restrict__ d2,
     rz[s] = d2[nsub + s];
     const int a = need[s] && d2[s] > 0.0 && isfinite(d2[s]);
     active[s] = a;
-}
-
-template <typename T>
-static int batched_dot2(pyhip_problem *p, KrylovWork *W, const T *a, const T *b, const T *c,
-                        const T *d, double *out, const int32_t *act = nullptr) {
-    TimeScope ts(&p->timer, "vector", p->st);
-    const int pstride = W->m + 2;
-    if (W->nchunk == 0) return PYHIP_OK;
-    hipLaunchKernelGGL((dot2_kernel<T>), dim3((unsigned)W->nchunk), dim3(256), 0, p->st, a, b, c, d,
-                       W->chunk_begin, W->chunk_end, W->partial, pstride, W->chunk_sub, act);
-    KCHECK();
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((unsigned)(2 * W->nsub)), dim3(64), 0, p->st, 2,
-                       W->nsub, W->sub_chunk_ptr, W->partial, pstride, out, 0);
-    KCHECK();
-    return PYHIP_OK;
 }
 
 // x = A^{-1} b per sub-problem with need[s]; CG in precision T on values TV, with any
@@ -1475,7 +1385,7 @@ static int cg_generic(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *
     PYHIP_CHECK_HIP(hipMemcpyAsync(act_h, need, ns * sizeof(int32_t), hipMemcpyDeviceToHost, p->st));
     PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
     if ((rc = precond_apply<T>(p, W, o.precond, r, z, need, act_h))) return rc;
-    if ((rc = batched_dot2<T>(p, W, r, r, r, z, d2))) return rc;
+    if ((rc = batched_dots<T>(p, W, r, r, d2, r, z))) return rc;
     hipLaunchKernelGGL(zero_i32_kernel, dim3(nblk(ns, 64)), dim3(64), 0, p->st, ns, W->cg_fail);
     // (r, z) alternates between two arrays (cg_kernels.h)
     double *rz[2] = {W->cg_rz, W->cg_beta};
@@ -1493,7 +1403,7 @@ static int cg_generic(pyhip_problem *p, KrylovWork *W, const TV *vals, const T *
         w0 = amg_fine_w<T>(W->amg);
         x0 = amg_fine_x<T>(W->amg);
     }
-    // The host reads the running count every kPcgRead iterations: in between, a converged
+    // The host reads the flags every kPcgRead to kPcgReadMax iterations: in between, a converged
     // sub-problem's flag is cleared on the device and every kernel skips its rows, so the
     // host keeps enqueueing instead of waiting. The spmv-family bytes of those launches
     // depend on which sub-problems were live: the launches add their per-launch part now
@@ -2006,7 +1916,7 @@ static int linear_solve(pyhip_problem *p, KrylovWork *W, const pyhip_linear_opts
     KCHECK();
     const int ns = W->nsub;
     double *d3 = W->dots + 2 * (W->m + 2) * ns;
-    if ((rc = batched_dots<double>(p, W, 1, r, n, r, W->dots))) return rc;
+    if ((rc = batched_dots<double>(p, W, r, r, W->dots))) return rc;
     std::vector<double> rn0(ns), rn(ns);
     PYHIP_CHECK_HIP(hipMemcpyAsync(rn0.data(), W->dots, ns * sizeof(double), hipMemcpyDeviceToHost, p->st));
     std::vector<int32_t> need_h(ns);
@@ -2029,7 +1939,7 @@ static int linear_solve(pyhip_problem *p, KrylovWork *W, const pyhip_linear_opts
         if (jac_prec == PYHIP_F64) rc = spmv<double, double, double>(p, W->vals64, d, W->r64, r);
         else rc = spmv<float, double, double>(p, W->vals32, d, W->r64, r);
         if (rc) return rc;
-        if ((rc = batched_dots<double>(p, W, 1, W->r64, n, W->r64, d3))) return rc;
+        if ((rc = batched_dots<double>(p, W, W->r64, W->r64, d3))) return rc;
         PYHIP_CHECK_HIP(hipMemcpyAsync(rn.data(), d3, ns * sizeof(double), hipMemcpyDeviceToHost, p->st));
         PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
         left = 0;
@@ -2403,7 +2313,7 @@ int pyhip_arclength_step(pyhip_problem *p, double *x, int param, const pyhip_new
     // per-sub-problem dot of two vectors, on the host
     auto sub_dot = [&](const double *a, const double *b, double *out) -> int {
         int r2;
-        if ((r2 = batched_dots<double>(p, W, 1, a, n, b, W->dots))) return r2;
+        if ((r2 = batched_dots<double>(p, W, a, b, W->dots))) return r2;
         PYHIP_CHECK_HIP(hipMemcpyAsync(out, W->dots, ns * sizeof(double), hipMemcpyDeviceToHost, p->st));
         PYHIP_CHECK_HIP(hipStreamSynchronize(p->st));
         return PYHIP_OK;
