@@ -57,6 +57,34 @@ def test_assembly_at_workgroup_edges(gpu, kind, kw, transient):
     assert np.max(np.abs(r32.cpu().numpy() - R)) <= tol * max(scale, np.max(np.abs(R)))
 
 
+@pytest.mark.parametrize("kind,kw", [("bratu", dict(N=N, space=sp, lam=float(N * N))) for sp, N in
+                                     (("C1", 181), ("C1", 182), ("C2", 127), ("C2", 128), ("C2", 182))] +
+                         [("poisson", dict(N=N)) for N in (127, 182, 203)])
+def test_fp32_sources_on_many_elements(gpu, kind, kw):
+    """The FP32 bar above is relative to the stiffness, beside which a source of order h^2 does not
+    count on a fine mesh. Here lambda = N^2 makes the Bratu terms as large as the stiffness, and
+    the residual without dofs is the source alone, held to the same bar relative to its own
+    largest entry."""
+    import torch
+    P, op = build(kind, kw)
+    tol = (27 + 16 * kw["N"]) * 2.0**-24
+
+    def assemble():
+        out = [P.assemble_device(p) for p in ("f32", "f64")]
+        torch.cuda.synchronize()
+        return out
+
+    rng = np.random.default_rng(kw["N"])
+    if kind == "bratu":
+        P.set_current_dofs(rng.uniform(-0.4, 0.4, P.ndof))
+        (r32, v32), (r64, v64) = assemble()
+        assert float((v32.double() - v64).abs().max()) <= tol * float(v64.abs().max())
+        assert float((r32 - r64).abs().max()) <= tol * max(float(v64.abs().max()), float(r64.abs().max()))
+    P.set_current_dofs(np.zeros(P.ndof))
+    (r32, _), (r64, _) = assemble()
+    assert float(r64.abs().max()) > 0 and float((r32 - r64).abs().max()) <= tol * float(r64.abs().max())
+
+
 @pytest.mark.parametrize("transient", [False, True])
 @pytest.mark.parametrize("cubes", [(1,), (1, 1), (1, 1, 1), (1,) * 7, (2,), (2, 1), (13,), (13, 5), (14,)])
 def test_brick_kernels_meet_at_their_rule(gpu, cubes, transient):

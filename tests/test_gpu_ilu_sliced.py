@@ -85,3 +85,23 @@ def test_tiny_problems_have_the_same_bits_in_workgroups_and_level_launches(gpu, 
     for i in (0, 1, 2, 3, 1536, 3071):
         assert np.array_equal(got[i], want[i % 4])
     assert np.array_equal(got[-1], _solve([wl.bratu(20, "C2", 1.0)], precision)[0])
+
+
+@pytest.mark.parametrize("n", [65, 96, 97, 130, 200, 256, 257, 300])
+def test_dense_matrices_are_factorised_exactly(gpu, n):
+    """ILU(0) of a full matrix is its LU in any order: rows of more than 64 lower and upper
+    entries, of exactly kIluRow = 256 entries (in LDS) and more (in memory), and slices that go
+    on over two and three chunks (more than 96 entries a side). One iteration then leaves the
+    rounding of an elimination, n 2^-52 times a growth of at most 2 on a diagonally dominant
+    matrix, far below the 1e-10 at which a solve with wrong factors would stop."""
+    from pyoomph_amd.plugins import HIPKrylovSerial
+    rng = np.random.default_rng(n)
+    A = rng.uniform(-1, 1, (n, n))
+    A[np.arange(n), np.arange(n)] = np.abs(A).sum(1) + 1.0
+    A = sp.csr_matrix(A)
+    b = rng.standard_normal(n)
+    x = b.copy()
+    S = HIPKrylovSerial(None)
+    S.solve_serial(1, n, A.nnz, 1, A.data, A.indices, A.indptr, None, n, 1)
+    S.solve_serial(2, n, A.nnz, 1, None, None, None, x, n, 1)
+    assert np.linalg.norm(A @ x - b) <= 8 * n * 2.0**-52 * np.linalg.norm(b)

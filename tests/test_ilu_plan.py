@@ -462,3 +462,37 @@ def test_many_tiny_problems_take_the_level_lists(kind, kw, tiny):
         if tiny and len(S["subs"]):
             rows = S["idx"][:, :, 6] != 0xffff
             assert set((S["idx"][rows.any(1), 0, 7] >> 12) & 7) == {2}
+
+
+@pytest.mark.parametrize("n,band", [(130, 129), (260, 259), (700, 120)])
+@pytest.mark.parametrize("order", [NATURAL, MULTICOLOR])
+def test_slices_over_several_chunks(order, n, band):
+    """Rows of more than 96 entries a side (16 lanes, 6 steps): their slices go on over two and
+    three chunks, every entry taken once, by the lane of its row, the same row in each chunk, with
+    the go-on mark on all but the last."""
+    offs = [k for k in range(-band, band + 1)]
+    A = sp.diags([np.ones(n - abs(k)) for k in offs], offs, shape=(n, n)).tocsr()
+    A.sort_indices()
+    off, grp = np.array([0, n]), np.zeros(n, np.int8)
+    P = _plan(A.indptr, A.indices, off, order=order)
+    for side in (0, 1):
+        S = _sliced((A, grp, order), off, 1000, side)
+        k0, k1 = (P["prs"][:-1], P["pdiag"]) if side == 0 else (P["pdiag"] + 1, P["prs"][1:])
+        taken, longest = [], 0
+        for w in range(16):
+            rows, length = None, 0
+            for ch in range(*S["chunk0"][w:w + 2]):
+                q = S["src"][ch].transpose(0, 2, 1).reshape(6, 64)
+                row, mark = S["idx"][ch, :, 6], int(S["idx"][ch, 0, 7])
+                assert rows is None or np.array_equal(rows, row)
+                r = np.broadcast_to(row.astype(int), q.shape)[q >= 0]
+                assert np.all((q[q >= 0] >= k0[r]) & (q[q >= 0] < k1[r]))
+                assert np.array_equal(S["idx"][ch, :, :6].T[q >= 0], P["pcol"][q[q >= 0]])
+                taken.append(q[q >= 0])
+                length += 1
+                longest = max(longest, length)
+                rows, length = (row, length) if mark >> 15 else (None, 0)
+            assert rows is None
+        assert np.array_equal(np.sort(np.concatenate(taken)),
+                              np.concatenate([np.arange(a, b) for a, b in zip(k0, k1)]))
+        assert longest == -(-int((k1 - k0).max()) // 96)
