@@ -204,9 +204,10 @@ __device__ __forceinline__ int32_t find_col(const int32_t *__restrict__ cols, in
 // (a source row has distinct columns, so no two lanes touch one sum in a step). A sum thus
 // receives its terms in increasing t whatever G, alone or in a batch. The loads and searches of
 // kProdAhead terms go together; one at a time, a term's two dependent loads and its search
-// were the time (192 P2 problems: A P 509 us, now 419, P^T Q 214, now 161; eight terms: 608 and
-// 153). Bound: the searches' LDS reads. Output rows longer than CAPR take the same sums
-// entry by entry (binary search in the source rows).
+// were the time (sweep of 192 problems, finest level: A P 960 us, now 815, P^T Q 377, now 275; mean
+// over the levels 499, now 426, and 213, now 161, with eight terms 608 and 153). Bound: the
+// searches' LDS reads. Output rows longer than CAPR take the same sums entry by entry (binary
+// search in the source rows).
 constexpr int kProdAhead = 4;
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -305,7 +306,7 @@ constexpr int kQCap = 64, kCCap = 128;
 // length (the lanes spread over a source row's entries: the element level's prolongator
 // rows hold 1-8 entries, an aggregation level's 10-40; a wave per output row from 24 on, where
 // half a wave takes a second round of loads and searches per term: P^T Q of 4 x 20^3 bricks
-// 590 us, now 284). Every G gives the same sums.
+// 617 us, now 285). Every G gives the same sums.
 template <int CAPR>
 static void launch_rowprod(double mean_src, hipStream_t st, int64_t nout, const int32_t *ors, const int32_t *ocol,
                            double *oval, const int32_t *trs, const int32_t *trow, const double *tval,

@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) void scalar_element_kernel(ElemArgs<T> a) {
 // coordinates and one point's geometry fit a thread's registers, so no value is read twice
 // from LDS: with a thread per (element, row) every matrix entry of every point took its
 // gradients, shape values and equation number from LDS, and the kernel waited 68 % of its
-// time (sweep of 192 problems: P2 part 557 us, now 257, P1 part 61, now 38). Same operations in the same order per
+// time (sweep of 192 problems: P2 part 585 us, now 264, P1 part 63, now 39). Same operations in the same order per
 // output. The matrices leave through LDS (odd stride per element: no bank conflicts), as
 // coalesced stores over the block's elements; entries of pinned rows and columns are
 // written too (nothing reads them). Bound: FP64 ALU without contraction, then the stores.
@@ -420,7 +420,7 @@ __global__ __launch_bounds__(kTriThreads) void tri_element_kernel(ElemArgs<T> a)
 // blocks and twice the waves gave the same for the matrix and more for the residual. Same
 // operations in the same order per output. Bound: FP64 ALU without contraction (9 operations
 // per entry and point) with the LDS reads beside it. Before and now: 13824 elements FP32 with
-// the matrix 316 and 90 us; 32000 FP64 858 and 580 us, residual only 234 (shared records of an
+// the matrix 320 and 85 us; 32000 FP64 858 and 585 us, residual only 234 (shared records of an
 // even number of doubles, whose lanes meet on few banks) and 151 us.
 constexpr int kHexPerWave = 7, kHexWaves = 4, kHexPerBlock = kHexPerWave * kHexWaves;
 template <typename T, int FORM, bool TR>
@@ -640,7 +640,7 @@ __global__ __launch_bounds__(64 * kHexWaves) void hex_element_kernel(ElemArgs<T>
 // in registers and walks the points and the nine column nodes; the four pressure rows follow.
 // A thread per slot row put the three kinds of rows side by side in a wave, which then ran
 // every kind's code for every entry, with an equation-number read and branch for each
-// (16384 elements: 176 us, now 45). Same operations in the same order per output; the entries of
+// (16384 elements: 181 us, now 44). Same operations in the same order per output; the entries of
 // pinned rows and columns are written too (nothing reads them). Bound: FP64 ALU without
 // contraction.
 constexpr int kThPer = 14, kThThreads = 128;   // elements and threads per workgroup (9 threads per element)

@@ -26,9 +26,9 @@ constexpr int kGatherBlock = 256;
 // kGatherBlock apart; the blocks after them (when res is given) own one residual row per
 // thread. An entry is a chain of dependent loads (contribution bounds, index, element value)
 // of which a thread keeps kGatherPer * kGatherAhead going at a time: with one entry per thread
-// the gather waited 93 % of its cycles (192 problems, 1.05 GB read and 0.33 GB written: 483 us,
-// now 430; visiting the entries in the order of the elements did not lower the bytes and took
-// 558). Each sum keeps its list's order.
+// the gather waited 93 % of its cycles (192 problems, 1.05 GB read and 0.33 GB written: 497 us,
+// now 468; visiting the entries in the order of the elements did not lower the bytes and took
+// 30 % more). Each sum keeps its list's order.
 constexpr int kGatherPer = 2, kGatherAhead = 3;
 template <typename TE, typename TV>
 __global__ __launch_bounds__(kGatherBlock) void gather_values_kernel(
